@@ -298,6 +298,26 @@ int vaa_paged_attention_prefill_split(const vaa_attn_params* p, const uint16_t* 
                                       size_t workspace_bytes, void* stream);
 
 /*
+ * Attention inside each sequence's own tokens, without a cache (encoder
+ * models; vllm_apple/v1/attention/backends/base_attn.py:223-306): token t of
+ * sequence s, the tokens [query_start_loc[s], query_start_loc[s + 1]), attends
+ * to the sequence's tokens up to itself (causal != 0) or to all of them.
+ * query_start_loc (num_seqs + 1 entries, on the device) does not decrease;
+ * query, key, value and output hold num_tokens rows, and key and value are
+ * read in place.  Tokens of no sequence are left unwritten.  p: scale,
+ * num_seqs, max_seq_len (the longest sequence, which sizes the tables),
+ * head_size, heads, dtype, q_/o_stride_* and k_/v_stride_token/head (the
+ * tensors' own); the paged fields are ignored.  workspace:
+ * vaa_attention_no_cache_workspace_size bytes, 4-byte aligned.  output must
+ * not overlap key or value.
+ */
+size_t vaa_attention_no_cache_workspace_size(int num_seqs, int num_tokens, int max_seq_len);
+int vaa_attention_no_cache(const vaa_attn_params* p, const uint16_t* query, const uint16_t* key,
+                           const uint16_t* value, const int32_t* query_start_loc,
+                           uint16_t* output, int num_tokens, int causal, void* workspace,
+                           size_t workspace_bytes, void* stream);
+
+/*
  * token_to_seq and positions for a flattened batch, computed on the device
  * from query_start_loc [num_seqs+1] and full seq_lens [num_seqs]:
  *   token_to_seq = repeat_interleave(arange(num_seqs), diff(query_start_loc))

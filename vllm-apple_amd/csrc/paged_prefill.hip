@@ -43,6 +43,8 @@
 // hd dims of a row written (the kPad instantiations).
 #include "common.h"
 
+#include <algorithm>
+
 namespace vaa {
 namespace {
 
@@ -1104,4 +1106,113 @@ extern "C" int vaa_paged_attention_prefill_split(const vaa_attn_params* p,
   return prefill_impl("vaa_paged_attention_prefill_split", p, query, key_cache, value_cache,
                       block_table, token_to_seq, positions, output, num_tokens, split_keys,
                       workspace, workspace_bytes, stream);
+}
+
+// ---------------------------------------------------------------------------
+// Attention inside each sequence's own tokens, no cache (encoder models).
+//
+// The prefill kernel reads K and V through block tables, so the caller's
+// tensors are described to it as a cache of overlapping blocks: block i holds
+// tokens i .. i + kNcBlock - 1 (block stride = token stride), and sequence s,
+// whose tokens start at query_start_loc[s], owns the blocks query_start_loc[s]
+// + kNcBlock j.  The kernel reads no row past a sequence's context, so nothing
+// outside the tensors is touched, and K and V are read in place: no staging
+// copy (9 us), and with one kernel for the per-token indices and the tables
+// instead of some twenty tensor ops and three host-to-device copies the call
+// takes two launches: 25 sequences of 12 to 512 tokens, 12 heads, D 64, the
+// backend's forward 237 -> 35 us a call, of which the prefill kernel is 28.
+namespace vaa {
+namespace {
+
+constexpr int kNcBlock = 16;      // tokens per block: one 16-key fetch group
+constexpr int kNcThreads = 256;
+constexpr int kNcSeqLds = 1024;   // sequence starts searched in LDS up to here
+
+__global__ void __launch_bounds__(kNcThreads)
+no_cache_index_kernel(const int32_t* qsl, int num_seqs, int num_tokens, int max_blocks, int causal,
+                      int32_t* tok_seq, int32_t* pos, int32_t* bt) {
+  __shared__ int32_t sl[kNcSeqLds + 1];
+  const bool lds = num_seqs <= kNcSeqLds;
+  if (lds) {
+    for (int i = threadIdx.x; i <= num_seqs; i += kNcThreads) sl[i] = qsl[i];
+    __syncthreads();
+  }
+  // Clamped to the tensors' rows, so that no table entry or position lets the
+  // prefill read past them whatever the starts hold.
+  auto start = [&](int s) { return min(max(lds ? sl[s] : qsl[s], 0), num_tokens); };
+  const int64_t i = static_cast<int64_t>(blockIdx.x) * kNcThreads + threadIdx.x;
+  if (i < num_tokens) {
+    const int t = static_cast<int>(i);
+    int s = -1, p = -1;
+    if (t >= start(0) && t < start(num_seqs)) {
+      // Largest s with start(s) <= t: skips empty sequences.
+      int lo = 0, hi = num_seqs - 1;
+      while (lo < hi) {
+        const int mid = (lo + hi + 1) >> 1;
+        if (start(mid) <= t) lo = mid; else hi = mid - 1;
+      }
+      if (t < start(lo + 1)) {
+        s = lo;
+        p = causal ? t - start(s) : start(s + 1) - start(s) - 1;
+      }
+    }
+    tok_seq[t] = s;
+    pos[t] = p;
+  }
+  if (i < static_cast<int64_t>(num_seqs) * max_blocks) {
+    const int s = static_cast<int>(i / max_blocks), j = static_cast<int>(i % max_blocks);
+    const int b = start(s) + kNcBlock * j;
+    bt[i] = b < start(s + 1) ? b : -1;
+  }
+}
+
+}  // namespace
+}  // namespace vaa
+
+extern "C" size_t vaa_attention_no_cache_workspace_size(int num_seqs, int num_tokens,
+                                                        int max_seq_len) {
+  if (num_seqs <= 0 || num_tokens <= 0 || max_seq_len <= 0) return 0;
+  const size_t mb = (static_cast<size_t>(max_seq_len) + kNcBlock - 1) / kNcBlock;
+  return (2 * static_cast<size_t>(num_tokens) + static_cast<size_t>(num_seqs) * mb) *
+         sizeof(int32_t);
+}
+
+extern "C" int vaa_attention_no_cache(const vaa_attn_params* p, const uint16_t* query,
+                                      const uint16_t* key, const uint16_t* value,
+                                      const int32_t* query_start_loc, uint16_t* output,
+                                      int num_tokens, int causal, void* workspace,
+                                      size_t workspace_bytes, void* stream) {
+  const char* what = "vaa_attention_no_cache";
+  if (!p) return fail(VAA_ERR_INVALID_ARG, "%s: null params", what);
+  if (num_tokens < 0 || p->num_seqs < 0 || p->max_seq_len < 0)
+    return fail(VAA_ERR_INVALID_ARG, "%s: num_tokens=%d num_seqs=%d max_seq_len=%d", what,
+                num_tokens, p->num_seqs, p->max_seq_len);
+  if (num_tokens == 0 || p->num_seqs == 0 || p->max_seq_len == 0) return VAA_OK;
+  if (!query_start_loc) return fail(VAA_ERR_INVALID_ARG, "%s: null pointer", what);
+  const size_t need =
+      vaa_attention_no_cache_workspace_size(p->num_seqs, num_tokens, p->max_seq_len);
+  if (!workspace || workspace_bytes < need || (reinterpret_cast<uintptr_t>(workspace) & 3u))
+    return fail(VAA_ERR_WORKSPACE, "%s: workspace of %zu bytes (4-byte aligned) needed, got %zu",
+                what, need, workspace ? workspace_bytes : static_cast<size_t>(0));
+  vaa_attn_params q = *p;
+  q.block_size = kNcBlock;
+  q.max_blocks_per_seq = (p->max_seq_len + kNcBlock - 1) / kNcBlock;
+  q.num_blocks = num_tokens;  // the first tokens of blocks: never past the tensors
+  q.k_stride_block = p->k_stride_token;
+  q.v_stride_block = p->v_stride_token;
+  int32_t* tok = static_cast<int32_t*>(workspace);
+  int32_t* pos = tok + num_tokens;
+  int32_t* bt = pos + num_tokens;
+  const int64_t n = std::max<int64_t>(
+      num_tokens, static_cast<int64_t>(p->num_seqs) * q.max_blocks_per_seq);
+  if ((n + kNcThreads - 1) / kNcThreads > INT32_MAX)
+    return fail(VAA_ERR_UNSUPPORTED, "%s: num_seqs=%d max_seq_len=%d", what, p->num_seqs,
+                p->max_seq_len);
+  hipLaunchKernelGGL(no_cache_index_kernel, dim3((n + kNcThreads - 1) / kNcThreads),
+                     dim3(kNcThreads), 0, static_cast<hipStream_t>(stream), query_start_loc,
+                     p->num_seqs, num_tokens, q.max_blocks_per_seq, causal, tok, pos, bt);
+  const int st = check_launch("no_cache_index_kernel");
+  if (st) return st;
+  return prefill_impl(what, &q, query, key, value, bt, tok, pos, output, num_tokens, 0, nullptr, 0,
+                      stream);
 }

@@ -244,6 +244,23 @@ def _overlap_enabled() -> bool:
     return os.environ.get(OVERLAP_ENV, "1") != "0"
 
 
+def _rows_ok(t: torch.Tensor) -> bool:
+    """16-byte aligned rows with a contiguous last dim: what the attention
+    kernels read directly."""
+    return (t.dim() == 3 and t.stride(2) == 1 and t.stride(1) % 8 == 0 and t.stride(0) % 8 == 0
+            and t.data_ptr() % 16 == 0)
+
+
+def _overlaps(a: torch.Tensor, b: torch.Tensor) -> bool:
+    """Whether the address ranges that two tensors span meet."""
+    def span(t):
+        n = sum((d - 1) * s for d, s in zip(t.shape, t.stride())) + 1
+        return t.data_ptr(), t.data_ptr() + n * t.element_size()
+
+    (a0, a1), (b0, b1) = span(a), span(b)
+    return a0 < b1 and b0 < a1
+
+
 class HipAttentionImpl(AttentionImpl):
     def __init__(self, num_heads: int, head_size: int, scale: float, num_kv_heads: int,
                  alibi_slopes: Optional[list], sliding_window: Optional[int],
@@ -414,14 +431,34 @@ class HipAttentionImpl(AttentionImpl):
         """Attention inside each sequence's own tokens (encoder / no KV cache),
         the semantics of _compute_attention_sdpa (base_attn.py:223-306).
 
-        The tokens are staged into a scratch paged cache, one block-aligned
-        range per sequence, and run through the prefill kernel; positions are
-        the in-sequence index (causal) or the last index (bidirectional).
+        Rows that the kernels can read directly, with the sequence starts at
+        hand on the device, run in place (kernels.attention_no_cache).
+        Otherwise the tokens are staged into a scratch paged cache, one
+        block-aligned range per sequence, and run through the prefill kernel;
+        positions are the in-sequence index (causal) or the last index
+        (bidirectional).
         """
         qsl = attn_metadata.query_start_loc_cpu
         num_seqs = len(qsl) - 1
         T = min(query.shape[0], qsl[-1] if num_seqs > 0 else 0)
         if T <= 0:
+            return output
+        lens_host = [b - a for a, b in zip(qsl[:-1], qsl[1:])]
+        dqsl = attn_metadata.query_start_loc
+        if (qsl[0] == 0 and min(lens_host) >= 0 and T == qsl[-1]
+                and isinstance(dqsl, torch.Tensor) and dqsl.dtype == torch.int32
+                and dqsl.device == query.device and dqsl.is_contiguous()
+                and dqsl.numel() == num_seqs + 1
+                and min(key.shape[0], value.shape[0], output.shape[0]) >= T
+                and key.shape == value.shape and key.stride() == value.stride()
+                and key.shape[2] == self.head_size == query.shape[2]
+                and query.shape[1] % key.shape[1] == 0
+                and query.shape[1:] == output.shape[1:]
+                and all(_rows_ok(t) for t in (query, key, value, output))
+                and not _overlaps(output, key) and not _overlaps(output, value)):
+            kernels.attention_no_cache(query[:T], key[:T], value[:T], dqsl, output[:T],
+                                       scale=self.scale, max_seq_len=max(lens_host),
+                                       causal=causal)
             return output
         bs = 16
         dev = query.device

@@ -623,6 +623,48 @@ def paged_prefill(query: torch.Tensor, key_cache: torch.Tensor, value_cache: tor
     return output
 
 
+def attention_no_cache(query: torch.Tensor, key: torch.Tensor, value: torch.Tensor,
+                       query_start_loc: torch.Tensor, output: torch.Tensor, *, scale: float,
+                       max_seq_len: int, causal: bool) -> torch.Tensor:
+    """Attention inside each sequence's own tokens, K and V read in place
+    (vaa_attention_no_cache), on the current stream.
+
+    query/output [T, H, D], key/value [T, KV, D], all fp16 or all bf16, with a
+    contiguous last dim and 16-byte aligned rows; query_start_loc int32
+    [num_seqs + 1] on the device; max_seq_len bounds the sequences' lengths.
+    output must not overlap key or value.
+    """
+    _require_gpu(query, key, value, query_start_loc, output)
+    dt = _attn_dtype(query=query, key=key, value=value, output=output)
+    if query_start_loc.dtype != torch.int32 or not query_start_loc.is_contiguous() \
+            or query_start_loc.numel() < 1:
+        raise ValueError("query_start_loc must be a contiguous int32 [num_seqs + 1] tensor")
+    for t, n in ((query, "query"), (key, "key"), (value, "value"), (output, "output")):
+        if t.dim() != 3 or t.stride(2) != 1:
+            raise ValueError(f"{n} must be [tokens, heads, head_size] with contiguous last dim")
+    T, H, D = query.shape
+    KV = key.shape[1]
+    if key.shape != value.shape or key.shape[0] < T or key.shape[2] != D \
+            or output.shape != query.shape or KV == 0 or H % KV:
+        raise ValueError(f"shapes differ: query {tuple(query.shape)}, key {tuple(key.shape)}, "
+                         f"value {tuple(value.shape)}, output {tuple(output.shape)}")
+    p = _lib.VaaAttnParams()
+    p.dtype = ATTN_DTYPES[dt]
+    p.scale = float(scale)
+    p.num_seqs, p.max_seq_len = query_start_loc.numel() - 1, int(max_seq_len)
+    p.head_size, p.num_kv_heads, p.num_query_heads, p.queries_per_kv = D, KV, H, H // KV
+    p.k_stride_token, p.k_stride_head = key.stride(0), key.stride(1)
+    p.v_stride_token, p.v_stride_head = value.stride(0), value.stride(1)
+    p.q_stride_token, p.q_stride_head = query.stride(0), query.stride(1)
+    p.o_stride_token, p.o_stride_head = output.stride(0), output.stride(1)
+    nbytes = _lib.load().vaa_attention_no_cache_workspace_size(p.num_seqs, T, p.max_seq_len)
+    ws = torch.empty(nbytes, dtype=torch.uint8, device=query.device)
+    _lib.call("vaa_attention_no_cache", ctypes.byref(p), query.data_ptr(), key.data_ptr(),
+              value.data_ptr(), query_start_loc.data_ptr(), output.data_ptr(), T, int(causal),
+              ws.data_ptr(), ws.numel(), _lib.stream_handle())
+    return output
+
+
 def build_token_index(query_start_loc: torch.Tensor, seq_lens: torch.Tensor, num_tokens: int,
                       stream=None) -> tuple[torch.Tensor, torch.Tensor]:
     """(token_to_seq, positions) int32 [num_tokens] computed on the device."""
