@@ -166,3 +166,47 @@ def test_topk_wave_path_ragged_tail_strided(gpu):
     ref_idx, ref_vals = otk.topk(_bits(big[:, :V].contiguous()), k)
     assert np.array_equal(idx.cpu().numpy(), ref_idx)
     assert np.array_equal(_bits(vals), ref_vals)
+
+
+# The row kernel's edges: one register slice (8192 columns) and one column
+# more, slice remainders, its largest row (163833), and a row past it.
+@pytest.mark.parametrize("V", [8192, 8193, 16383, 65529, 131065, 163833, 163834])
+@pytest.mark.parametrize("shift,stride_extra", [(0, 0), (1, 0), (7, 3), (4, 8)])
+def test_topk_row_kernel_edges(gpu, V, shift, stride_extra):
+    """Rows that start at any 2-byte address (their ragged ends are read one by
+    one), with the maxima and ties in the ends, a flat row, a row masked to
+    -inf but for fewer than k columns, and a row of the lowest key (-NaN bits)
+    but for a few."""
+    from vllm_apple_amd import kernels
+
+    T, k = 6, 50
+    g = torch.Generator().manual_seed(V + shift)
+    x = (torch.randn(T, V + stride_extra, generator=g) * 3).half()
+    x[0, :3] = 30.0
+    x[0, V - 3:V] = 30.0
+    x[1] = 0.25
+    x[2] = -float("inf")
+    x[2, V - 5:V] = torch.arange(5).half()
+    x[3].view(torch.int16).fill_(-1)     # 0xffff: the lowest key
+    x[3, 4000:4020] = 1.0
+    x[4] = torch.randint(-1, 2, (V + stride_extra,), generator=g).half()
+    buf = torch.zeros(x.numel() + 8, dtype=torch.float16, device="cuda")
+    buf[shift:shift + x.numel()] = x.reshape(-1).cuda()
+    logits = buf[shift:shift + x.numel()].view(T, V + stride_extra)[:, :V]
+    for kk in (1, k, 256):
+        idx, vals = kernels.topk_logits(logits, kk)
+        torch.cuda.synchronize()
+        ref_idx, ref_vals = otk.topk(_bits(x[:, :V].contiguous()), kk)
+        assert np.array_equal(idx.cpu().numpy(), ref_idx), kk
+        assert np.array_equal(_bits(vals), ref_vals), kk
+
+
+def test_topk_row_kernel_batch_limit(gpu):
+    """One slice and more than 2048 rows take the chunk path, 2048 the row
+    kernel: the same results."""
+    from vllm_apple_amd import kernels
+
+    g = torch.Generator().manual_seed(2)
+    x = (torch.randn(2049, 8200, generator=g) * 3).half().cuda()
+    a, b = kernels.topk_logits(x, 20), kernels.topk_logits(x[:2048], 20)
+    assert torch.equal(a[0][:2048], b[0]) and torch.equal(a[1][:2048], b[1])

@@ -6,8 +6,11 @@
 // bytes per token.  There, one threadgroup per row keeps insertion-sorted
 // per-thread lists and merges them in threadgroup memory.
 //
-// Here a row is cut into S chunks of at most kChunkMax columns, one workgroup
-// per chunk, so a 32-row decode batch still fills the chip.  A workgroup loads
+// Rows of 8192 to 163833 columns (the vocabularies served in practice) are
+// selected whole by one 16-wave workgroup each, in its registers
+// (topk_row_kernel).  Other rows, and large batches of the shortest of these,
+// are cut into S chunks of at most kChunkMax columns, one workgroup per chunk,
+// so a small batch still fills the chip.  A workgroup loads
 // its whole chunk into registers with every load in flight at once (one HBM
 // round trip) and selects on order-preserving 16-bit keys: a lower bound L
 // from k thread-group maxima (the top k are all >= L; on logits only ~1-5% of
@@ -403,14 +406,15 @@ __global__ void __launch_bounds__(kTkThreads) topk_chunk_kernel(TopkArgs a) {
 // exactly k items (ties taken in item order, which is column order).
 constexpr int kTkWaves = kTkThreads / kWave;  // waves per workgroup
 typedef unsigned short u16x2 __attribute__((ext_vector_type(2)));
+typedef short i16x2 __attribute__((ext_vector_type(2)));
 constexpr int kWaveChunk = 8 * 8 * kWave;     // 4096 columns per wave
 constexpr int kWaveK = kWave;                 // the bound takes the k-th of 64 lane maxima
 constexpr int kWaveCand = 512;                // list capacity per wave
 // The wave kernel once there are at least this many chunks: below, a wave per
-// chunk leaves the SIMDs too few waves to hide its serial phases (vocab
-// 128256 in 32 chunks, k = 50, wave against workgroup kernel: 32 rows 21.1
-// against 17.7 us; 64 rows 22.5 / 24.6; 128 rows 26.9 / 35.5; 256 rows 38.3 /
-// 59.4; 512 rows 57.3 / 106.2).
+// chunk leaves the SIMDs too few waves to hide its serial phases (32 chunks a
+// row, k = 50, wave against workgroup kernel: 32 rows 21.1 against 17.7 us; 64
+// rows 22.5 / 24.6; 128 rows 26.9 / 35.5; 256 rows 38.3 / 59.4; 512 rows 57.3 /
+// 106.2).
 constexpr int kWaveMinWork = 2048;
 
 __device__ __forceinline__ int wave_sum_i(int v) {
@@ -668,6 +672,248 @@ __global__ void __launch_bounds__(kTkThreads) topk_chunk_wave_kernel(TopkArgs a)
   }
 }
 
+// One workgroup of 16 waves per row, the whole row in its registers (2 bytes a
+// column: 128256 columns are 251 KB of the CU's 512 KB of VGPRs), so that a
+// call is one launch with no survivors in memory and no merge (k = 50, chunk
+// and merge kernels -> this one: 128256 columns, 32 rows 18.6 -> 10.6 us, 256
+// rows 37.8 -> 17.8, 1024 rows 97.8 -> 69.8; 32000 columns, 32 rows 14.8 ->
+// 7.3, 1024 rows 39.3 -> 21.4).  Bound by the row's load at one CU's rate and
+// then by the latency of a few workgroup-wide phases; from 1024 rows of 128256
+// columns on it streams at 3.8 to 4.2 TB/s, one row's load not overlapping
+// another's selection on a CU:
+//   load     chunk j * 1024 + tid of 16 aligned bytes, every load in flight at
+//            once through a buffer resource that returns zeros past the last
+//            whole chunk; the row's ragged ends (a row may start at any
+//            2-byte address) are read by their two threads one by one;
+//   bound    L = the k-th largest of the 1024 thread maxima (exact, four
+//            rounds of four bits: wave w counts the maxima that reach the
+//            w-th of 16 thresholds).  k distinct items are >= L, so the top k
+//            are, and few others (those that share a thread with another);
+//   list     the real items >= L go to an LDS list in any order (their words
+//            hold the column);
+//   rank     1024 / n lanes share one listed word's comparisons with the n
+//            listed words; its rank is its output position when < k.
+// When more than kRowCand items reach L (flat or heavily tied rows, masked
+// rows of -inf), the k-th key is searched bit by bit over all items and
+// exactly k items are listed, ties taken in column order.
+constexpr int kRowThreads = 1024;
+constexpr int kRowWaves = kRowThreads / kWave;
+constexpr int kRowSlice = kRowThreads * 8;  // columns per register slice
+constexpr int kRowMaxNj = 20;
+constexpr int kRowCand = 1024;
+
+struct RowSmem {
+  uint16_t mx[kRowThreads];  // thread maxima
+  int cnt[2][kRowWaves];
+  int n_cand;
+  uint64_t cand[kRowCand];
+};
+
+// Workgroup sum of one int per thread (buf: one of two alternating arrays, so
+// that one barrier per sum is enough).
+__device__ __forceinline__ int row_sum(int v, int* buf) {
+  v = wave_sum_i(v);
+  if (threadIdx.x % kWave == 0) buf[threadIdx.x / kWave] = v;
+  __syncthreads();
+  int s = 0;
+#pragma unroll
+  for (int i = 0; i < kRowWaves; ++i) s += buf[i];
+  return s;
+}
+
+template <int NJ>
+__global__ void __launch_bounds__(kRowThreads) __attribute__((amdgpu_waves_per_eu(NJ <= 4 ? 8 : 4)))
+topk_row_kernel(TopkArgs a) {
+  __shared__ RowSmem sm;
+  const int tid = threadIdx.x, lane = tid % kWave;
+  const int wv = __builtin_amdgcn_readfirstlane(tid / kWave);
+  const int V = a.V, k = a.k;
+  for (int row = blockIdx.x; row < a.T; row += gridDim.x) {
+    const uint16_t* x = a.logits + row * a.row_st;
+    // Chunk c holds columns 8c - off .. 8c - off + 7: whole for lo <= c < hi.
+    const int off = static_cast<int>((reinterpret_cast<uintptr_t>(x) & 15u) >> 1);
+    const int lo = off > 0 ? 1 : 0, hi = max(lo, (V + off) / 8);
+    const int n_chunks = (V + off + 7) / 8;
+    const auto rsrc = __builtin_amdgcn_make_buffer_rsrc(
+        const_cast<uint16_t*>(x - off + 8 * lo), 0, 16 * (hi - lo), 0x00020000);
+    u32x4 kp[NJ];
+#pragma unroll
+    for (int j = 0; j < NJ; ++j) {
+      // Past the last whole chunk (and before the first: the offset wraps)
+      // the load returns zeros.
+      kp[j] = __builtin_bit_cast(
+          u32x4, __builtin_amdgcn_raw_buffer_load_b128(
+                     rsrc, 16 * (j * kRowThreads + tid - lo), 0, 0));
+    }
+    if (tid == 0) sm.n_cand = 0;
+    // Keys: v ^ (sign ? 0xffff : 0x8000) per half; chunks that are not whole
+    // are 0, the padding's key.
+#pragma unroll
+    for (int j = 0; j < NJ; ++j) {
+      const int c = j * kRowThreads + tid;
+      const bool whole = c >= lo && c < hi;
+#pragma unroll
+      for (int q = 0; q < 4; ++q) {
+        const uint32_t v = kp[j][q];
+        const i16x2 s = __builtin_bit_cast(i16x2, v) >> static_cast<short>(15);
+        const uint32_t key = v ^ (__builtin_bit_cast(uint32_t, s) | 0x80008000u);
+        kp[j][q] = whole ? key : 0u;
+      }
+    }
+    auto fill = [&](int c) {
+#pragma unroll
+      for (int j = 0; j < NJ; ++j) {
+        if (c != j * kRowThreads + tid) continue;
+#pragma unroll
+        for (int e = 0; e < 8; ++e) {
+          const int col = 8 * c - off + e;
+          if (col >= 0 && col < V) kp[j][e / 2] |= sort_key(x[col]) << (16 * (e & 1));
+        }
+      }
+    };
+    if (lo > 0) fill(0);
+    if (hi < n_chunks && (hi > 0 || lo == 0)) fill(hi);
+    auto key_of = [&](int j, int e) { return (kp[j][e / 2] >> (16 * (e & 1))) & 0xffffu; };
+    // Makes the keys opaque to the compiler at a phase boundary: each phase
+    // unpacks them again instead of keeping the previous one's values alive.
+    auto reload_row = [&] {
+#pragma unroll
+      for (int j = 0; j < NJ; ++j) asm volatile("" : "+v"(kp[j]));
+    };
+    auto slice_max = [&](int j) {
+      u16x2 m = {0, 0};
+#pragma unroll
+      for (int q = 0; q < 4; ++q) {
+        const uint32_t v = kp[j][q];
+        m = __builtin_elementwise_max(m, __builtin_bit_cast(u16x2, v));
+      }
+      return m;
+    };
+    // Bound.
+    u16x2 mm = slice_max(0);
+#pragma unroll
+    for (int j = 1; j < NJ; ++j) mm = __builtin_elementwise_max(mm, slice_max(j));
+    sm.mx[tid] = max(mm[0], mm[1]);
+    __syncthreads();
+    uint32_t mv[16];
+#pragma unroll
+    for (int i = 0; i < 16; ++i) mv[i] = sm.mx[i * kWave + lane];
+    uint32_t L = 0;
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      const uint32_t t = L | (static_cast<uint32_t>(wv) << (12 - 4 * r));
+      int c = 0;
+#pragma unroll
+      for (int i = 0; i < 16; ++i) c += __popcll(__ballot(mv[i] >= t));
+      if (lane == 0) sm.cnt[r & 1][wv] = c;
+      __syncthreads();
+      // At least k maxima reach the first threshold (L itself).
+      const uint64_t ok = __ballot(lane < kRowWaves && sm.cnt[r & 1][lane % kRowWaves] >= k);
+      L |= static_cast<uint32_t>(63 - __builtin_clzll(ok | 1)) << (12 - 4 * r);
+    }
+    // List (with L > 0 no padding reaches it).
+    reload_row();
+    if (L > 0) {
+#pragma unroll
+      for (int j = 0; j < NJ; ++j) {
+        const u16x2 m = slice_max(j);
+        if (max(m[0], m[1]) >= L) {
+          const int col0 = 8 * (j * kRowThreads + tid) - off;
+#pragma unroll
+          for (int e = 0; e < 8; ++e) {
+            if (key_of(j, e) >= L) {
+              const int pos = atomicAdd(&sm.n_cand, 1);
+              if (pos < kRowCand) sm.cand[pos] = pack(key_of(j, e), col0 + e);
+            }
+          }
+        }
+      }
+    }
+    __syncthreads();
+    int n = sm.n_cand;
+    if (n > kRowCand || L == 0) {
+      // The k-th key K over all real items, bit by bit, then exactly k items:
+      // those above K and the first k - above of its ties in item order, which
+      // is column order.
+      uint32_t K = 0;
+      int round = 0;
+      auto count_ge = [&](uint32_t t) {  // t > 0: counts no padding
+        reload_row();
+        int c = 0;
+#pragma unroll
+        for (int j = 0; j < NJ; ++j)
+#pragma unroll
+          for (int e = 0; e < 8; ++e) c += key_of(j, e) >= t ? 1 : 0;
+        return row_sum(c, sm.cnt[round++ & 1]);
+      };
+#pragma unroll 1
+      for (int b = 15; b >= 0; --b) {
+        const uint32_t t = K | (1u << b);
+        if (count_ge(t) >= k) K = t;
+      }
+      const int above = count_ge(K + 1);
+      const int need_eq = k - above;
+      int gt_run = 0, eq_run = 0;
+      reload_row();
+#pragma unroll
+      for (int j = 0; j < NJ; ++j) {
+        if (gt_run == above && eq_run >= need_eq) break;  // block-uniform
+        int col0 = 8 * (j * kRowThreads + tid) - off;
+        asm volatile("" : "+v"(col0));  // not computed ahead for every slice
+        auto real = [&](int e) { return col0 + e >= 0 && col0 + e < V; };
+        int ngt = 0, neq = 0;
+#pragma unroll
+        for (int e = 0; e < 8; ++e) {
+          ngt += key_of(j, e) > K && real(e) ? 1 : 0;
+          neq += key_of(j, e) == K && real(e) ? 1 : 0;
+        }
+        // Exclusive scan of both counts (each below 65536) over the workgroup.
+        int wtot;
+        const int pre = wave_excl_scan(ngt | (neq << 16), lane, wtot);
+        int* buf = sm.cnt[round++ & 1];
+        if (lane == 0) buf[wv] = wtot;
+        __syncthreads();
+        int woff = 0, tot = 0;
+#pragma unroll
+        for (int i = 0; i < kRowWaves; ++i) {
+          if (i < wv) woff += buf[i];
+          tot += buf[i];
+        }
+        int g = gt_run + ((woff + pre) & 0xffff), q = eq_run + ((woff + pre) >> 16);
+#pragma unroll
+        for (int e = 0; e < 8; ++e) {
+          const uint32_t key = key_of(j, e);
+          if (!real(e)) continue;
+          if (key > K) {
+            sm.cand[g + min(q, need_eq)] = pack(key, col0 + e);
+            ++g;
+          } else if (key == K) {
+            if (q < need_eq) sm.cand[g + q] = pack(key, col0 + e);
+            ++q;
+          }
+        }
+        gt_run += tot & 0xffff;
+        eq_run += tot >> 16;
+      }
+      n = k;
+      __syncthreads();
+    }
+    // Rank: 2^ps lanes per word, 2^ps n <= 1024.
+    int ps = 0;
+    while (ps < 6 && (n << (ps + 1)) <= kRowThreads) ++ps;
+    const int i = tid >> ps, part = tid & ((1 << ps) - 1);
+    const uint64_t w = i < n ? sm.cand[i] : 0;
+    int r = 0;
+    if (i < n) {
+#pragma unroll 4
+      for (int t = part; t < n; t += 1 << ps) r += sm.cand[t] > w ? 1 : 0;
+    }
+    for (int o = 1; o < (1 << ps); o <<= 1) r += __shfl_xor(r, o, kWave);
+    if (i < n && part == 0 && r < k) write_final(a, row, r, w);
+    __syncthreads();  // the list and counters are free for the next row
+  }
+}
+
 // One workgroup per row: k of the S sorted survivor lists.
 __global__ void __launch_bounds__(kTkThreads) topk_merge_kernel(TopkArgs a) {
   __shared__ SelSmem sm;
@@ -727,6 +973,33 @@ bool plan_chunks(int T, int V, int k, int* S_out, int* C_out) {
   *S_out = S;
   *C_out = C;
   return true;
+}
+
+// The row kernel where a row fits its registers and fills its threads.  Below
+// two slices a batch of thousands of rows leaves it more barriers than columns
+// (8192 columns, chunk path against this: 2048 rows 34.5 against 31.2 us, 4096
+// rows 55.1 against 59.0; 16000 columns, 4096 rows 74.6 against 62.2).
+constexpr int kRowSmallMaxT = 2048;
+bool row_kernel_ok(int T, int V) {
+  return V >= kRowSlice && V + 7 <= kRowMaxNj * kRowSlice &&
+         (V >= 3 * kRowSlice / 2 || T <= kRowSmallMaxT);
+}
+
+int launch_row(const TopkArgs& a, hipStream_t s) {
+  const dim3 grid(a.T < (1 << 20) ? a.T : (1 << 20)), block(kRowThreads);
+  const int nj = (a.V + 7 + kRowSlice - 1) / kRowSlice;
+#define VAA_TOPK_ROW(NJ)                                              \
+  if (nj <= NJ) {                                                     \
+    hipLaunchKernelGGL(topk_row_kernel<NJ>, grid, block, 0, s, a);    \
+    return check_launch("topk_row_kernel");                           \
+  }
+  VAA_TOPK_ROW(4)
+  VAA_TOPK_ROW(8)
+  VAA_TOPK_ROW(12)
+  VAA_TOPK_ROW(16)
+  VAA_TOPK_ROW(kRowMaxNj)
+#undef VAA_TOPK_ROW
+  return fail(VAA_ERR_UNSUPPORTED, "topk_row_kernel: vocab_size=%d", a.V);
 }
 
 int check_topk(int num_tokens, int vocab_size, int k, const char* what) {
@@ -792,6 +1065,9 @@ extern "C" int vaa_topk_logits(const uint16_t* logits, int num_tokens, int vocab
   const hipStream_t s = static_cast<hipStream_t>(stream);
   const int64_t n_work = static_cast<int64_t>(num_tokens) * a.S;
   const int grid1 = static_cast<int>(n_work < (1 << 20) ? n_work : (1 << 20));
+  // The row kernel leaves the workspace, which the call takes either way (its
+  // size depends only on the arguments), unused.
+  if (row_kernel_ok(num_tokens, vocab_size)) return launch_row(a, s);
   if (a.vec && a.k <= kWaveK && a.C <= kWaveChunk && n_work >= kWaveMinWork) {
     const int64_t wgs = (n_work + kTkWaves - 1) / kTkWaves;
     hipLaunchKernelGGL(topk_chunk_wave_kernel, dim3(static_cast<int>(wgs < (1 << 20) ? wgs : (1 << 20))),
