@@ -430,6 +430,37 @@ int vaa_gate_up_silu(const uint16_t* x, int64_t x_stride, const uint16_t* w_gate
                      int64_t output_stride, int num_tokens, int hidden_size,
                      int intermediate_size, int dtype, void* stream);
 
+/*
+ * vaa_gate_up_silu with a workspace, which lets few tokens over a small
+ * intermediate size split the contraction over enough workgroups to fill the
+ * GPU: fp32 partial sums go to the workspace and a second kernel adds them and
+ * applies the epilogue.  vaa_gate_up_silu_workspace_size gives the bytes (0:
+ * none needed, workspace may be null); 16-byte aligned, not shared by calls
+ * that can run concurrently.  No counterpart in the reference.
+ */
+size_t vaa_gate_up_silu_workspace_size(int num_tokens, int hidden_size, int intermediate_size);
+int vaa_gate_up_silu_split(const uint16_t* x, int64_t x_stride, const uint16_t* w_gate,
+                           const uint16_t* w_up, int64_t w_stride, uint16_t* output,
+                           int64_t output_stride, int num_tokens, int hidden_size,
+                           int intermediate_size, int dtype, void* workspace,
+                           size_t workspace_bytes, void* stream);
+
+/*
+ * Plain product of few tokens with a weight matrix, the down projection of a
+ * decode batch's MLP (vllm_apple/engine/ops/mlp.py:332-384):
+ *   output[t, n] = round16(sum_k x[t, k] w[n, k]),  fp32 accumulation,
+ * for num_tokens <= 128, in_features a multiple of 64 and out_features of 128
+ * (VAA_ERR_UNSUPPORTED otherwise); strides in elements, multiples of 8, 16-byte
+ * aligned tensors.  The contraction is split over workgroups; workspace:
+ * vaa_linear_small_workspace_size bytes (0: shape not supported), 16-byte
+ * aligned, not shared by calls that can run concurrently.
+ */
+size_t vaa_linear_small_workspace_size(int num_tokens, int in_features, int out_features);
+int vaa_linear_small(const uint16_t* x, int64_t x_stride, const uint16_t* w, int64_t w_stride,
+                     uint16_t* output, int64_t output_stride, int num_tokens, int in_features,
+                     int out_features, int dtype, void* workspace, size_t workspace_bytes,
+                     void* stream);
+
 /* ------------------------------------------------------------------------
  * Fused QKV epilogue
  * ---------------------------------------------------------------------- */

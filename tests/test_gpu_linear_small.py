@@ -1,0 +1,71 @@
+"""The few-token product (vaa_linear_small) and the split gate/up product
+(vaa_gate_up_silu_split) against fp64 products of the same 16-bit values:
+token counts at the edges of the 32-token blocks, one to many splits with short
+last splits, row strides that are and are not multiples of 4 KB (which walk
+their steps from different starts), strided rows."""
+import pytest
+import torch
+
+from helpers import assert_close, assert_close_bf16, host
+
+import oracle.layer_ops as olo
+
+pytestmark = pytest.mark.gpu
+
+
+def _check(out, ref, dtype, what):
+    if dtype == torch.float16:
+        assert_close(host(out), ref, what=what)
+    else:
+        assert_close_bf16(out.cpu().double().numpy(), ref, what=what)
+
+
+@pytest.mark.parametrize("T", [1, 31, 32, 33, 64, 65, 96, 97, 127, 128])
+@pytest.mark.parametrize("K,N", [(64, 128), (1024, 256), (2048 + 64, 384), (8192, 128)])
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+def test_linear_small(gpu, T, K, N, dtype):
+    from vllm_apple_amd import kernels
+
+    g = torch.Generator().manual_seed(T + K + N)
+    x = torch.randn(T, K, generator=g).to(dtype)
+    w = (torch.randn(N, K, generator=g) / K ** 0.5).to(dtype)
+    buf = torch.full((T + 1, N + 8), 7.0, dtype=dtype, device="cuda")
+    out = buf[:T, :N]
+    kernels.linear_small(x.cuda(), w.cuda(), out)
+    torch.cuda.synchronize()
+    _check(out, (x.double() @ w.double().T).numpy(), dtype, f"linear {T}x{K}x{N}")
+    assert bool((buf[T:] == 7.0).all()) and bool((buf[:, N:] == 7.0).all()), "padding written"
+
+
+@pytest.mark.parametrize("T", [1, 24, 33, 64, 100, 128])
+@pytest.mark.parametrize("H,I", [(2048, 256), (1088, 128), (4096, 1024)])
+def test_gate_up_silu_split(gpu, T, H, I):
+    from vllm_apple_amd import _lib, kernels
+
+    assert _lib.load().vaa_gate_up_silu_workspace_size(T, H, I) > 0
+    g = torch.Generator().manual_seed(T + H)
+    x = torch.randn(T, H, generator=g).half()
+    w = (torch.randn(2 * I, H, generator=g) / H ** 0.5).half()
+    out = kernels.gate_up_silu(x.cuda(), w.cuda())
+    torch.cuda.synchronize()
+    assert_close(host(out), olo.gate_up_silu(host(x), host(w)), what=f"gate_up {T}x{H}x{I}")
+
+
+def test_linear_small_strided_rows_and_refusals(gpu):
+    from vllm_apple_amd import kernels
+
+    g = torch.Generator().manual_seed(4)
+    xb = torch.randn(40, 576, generator=g).half()
+    wb = (torch.randn(256, 640, generator=g) / 23).half()
+    x, w = xb.cuda()[:, 64:576], wb.cuda()[:, 64:576]
+    out = torch.empty(40, 256, dtype=torch.float16, device="cuda")
+    kernels.linear_small(x, w, out)
+    torch.cuda.synchronize()
+    assert_close(host(out), (xb[:, 64:].double() @ wb[:, 64:576].double().T).numpy(), what="strided")
+    z = torch.zeros(129, 512, dtype=torch.float16, device="cuda")
+    assert not kernels.linear_small_ok(z, w, torch.empty(129, 256, dtype=z.dtype, device="cuda"))
+    assert not kernels.linear_small_ok(xb.cuda()[:, 1:513], w, out)      # unaligned rows
+    assert not kernels.linear_small_ok(x, w[:200], out[:, :200])         # 200 columns
+    assert not kernels.linear_small_ok(x.bfloat16(), w, out)             # two types
+    with pytest.raises(ValueError):
+        kernels.linear_small(x, w[:200], out[:, :200])

@@ -45,6 +45,8 @@
 // weight tile run at the same time on one XCD and read it through its L2.
 #include "common.h"
 
+#include <algorithm>
+
 namespace vaa {
 namespace {
 
@@ -108,6 +110,11 @@ struct GluArgs {
   char* out;
   int64_t xs, ws, os;  // row strides, bytes
   int num_tokens, ksteps, t_tiles, tiles;
+  // Few-token kernel: k-steps per split, byte step of wg and wu between column
+  // tiles, and the split's fp32 partials (null: one split, SwiGLU epilogue).
+  int k_per;
+  int64_t w_tile;
+  float* part;
 };
 
 // s_waitcnt vmcnt(8) lgkmcnt(0), at the top of step k: every vector memory
@@ -292,7 +299,13 @@ gate_up_silu_kernel(GluArgs a) {
 // Few tokens (decode-sized batches, T <= 128): the weights are the stream
 // (671 MB at hidden 5120 x 2 x intermediate 32768) and the product is small,
 // so the 256-token tile above spends most of its MFMAs on padding and runs
-// one workgroup per CU.  Here a workgroup owns 64 output columns (64 gate and
+// one workgroup per CU.  The same kernel streams the gate and up rows of the
+// SwiGLU product or 128 rows of a plain one (the down projection), and where
+// the column tiles alone leave CUs idle it splits the contraction: fp32
+// partials to a workspace, summed by split_sum_kernel (24 tokens, down
+// projection 32768 x 5120: 53 us, 6.3 TB/s, against 160 us for the library's
+// GEMM; 14336 x 4096 24 against 32; 8192 x 2048 11.4 against 14; gate/up 2048 x
+// 8192 21.7 unsplit -> 17.4).  Here a workgroup owns 64 output columns (64 gate and
 // the 64 up rows of the same columns) and all tokens (TB blocks of 32): its
 // weight tile is 16 KB per 64-element k-step, so two workgroups share a CU
 // and 512 of them cover intermediate 32768.  Tiles move with the same direct
@@ -309,12 +322,13 @@ gate_up_silu_kernel(GluArgs a) {
 constexpr int kSCols = 64;                    // output columns per workgroup
 constexpr int kSWTile = 2 * kSCols * kGRowB;  // weight tile per k-step: 128 rows, 16 KB
 constexpr int kSWStages = 3;
+constexpr int kRotStep = 5;  // k-steps between neighbouring tiles' starts
 
 // s_waitcnt vmcnt(4) lgkmcnt(0): all of this wave's loads but the newest 4
 // (its weight loads of the next step) have landed.
 __device__ __forceinline__ void glu_small_wait() { __builtin_amdgcn_s_waitcnt(0x0074); }
 
-template <typename T, int TB>
+template <typename T, int TB, bool kPart>
 __global__ void __launch_bounds__(kGThreads) gate_up_silu_small_kernel(GluArgs a) {
   extern __shared__ __align__(16) char smem[];  // W stages, then x stages
   constexpr int kXTile = TB * 32 * kGRowB;
@@ -330,7 +344,7 @@ __global__ void __launch_bounds__(kGThreads) gate_up_silu_small_kernel(GluArgs a
   // Loads: weight rows 0-63 are the gate rows i0.., 64-127 the up rows;
   // wave w loads rows 32w .. 32w + 31 (four 1 KB loads of 8 rows) and the
   // activation loads w, w + 4, ... of the TB * 4 in a tile.
-  const char* wbase = (wave < 2 ? a.wg : a.wu) + static_cast<int64_t>(i0) * a.ws;
+  const char* wbase = (wave < 2 ? a.wg : a.wu) + blockIdx.x * a.w_tile;
   const i32x4v wrs = buffer_rsrc(wbase, static_cast<int>(kSCols * a.ws));
   const i32x4v xrs = buffer_rsrc(a.x, static_cast<int>(a.num_tokens * a.xs));
   const int rw = 32 * (wave & 1) + (lane >> 3);  // weight row of load 0 within its matrix
@@ -359,14 +373,29 @@ __global__ void __launch_bounds__(kGThreads) gate_up_silu_small_kernel(GluArgs a
 #pragma unroll
     for (int r = 0; r < 16; ++r) g[b][r] = u[b][r] = 0.f;
 
-  const int n = a.ksteps;
+  // Steps k0 .. k0 + n - 1 of this split.
+  const int k0 = kPart ? static_cast<int>(blockIdx.y) * a.k_per : 0;
+  const int n = kPart ? min(a.ksteps - k0, a.k_per) : a.ksteps;
+  // Row strides that are a multiple of 4 KB put the pieces that every
+  // workgroup wants at one step on a few memory channels, so the tiles then
+  // walk their steps from different starts (stride 64 KB, K 32768 x 5120, 24
+  // tokens: 66.6 -> 53.2 us; stride 8 KB, gate/up 4096 x 14336: 47.8 -> 40.8).
+  // Other strides spread by themselves, and one common order keeps the
+  // activations in the L1 and L2 (stride 10 KB, gate/up 5120 x 32768: 100.8
+  // against 103.1 us).
+  const int rot = a.ws % 4096 == 0 ? static_cast<int>((blockIdx.x * kRotStep) % n) : 0;
+  auto kstep = [&](int ks) {
+    int s = min(ks, n - 1) + rot;
+    if (s >= n) s -= n;
+    return (k0 + s) * kGRowB;
+  };
   auto load_w = [&](int ks, uint32_t dst) {
-    const int kb = min(ks, n - 1) * kGRowB;
+    const int kb = kstep(ks);
 #pragma unroll
     for (int q = 0; q < 4; ++q) dma16_stream(wrs, woff, kb + q * wstep, dst + wdst + 1024 * q);
   };
   auto load_x = [&](int ks, uint32_t dst) {
-    const int kb = min(ks, n - 1) * kGRowB;
+    const int kb = kstep(ks);
 #pragma unroll
     for (int j = 0; j < TB; ++j) dma16(xrs, xoff[j], kb, dst + 1024 * (wave + 4 * j));
   };
@@ -398,7 +427,24 @@ __global__ void __launch_bounds__(kGThreads) gate_up_silu_small_kernel(GluArgs a
   // Every load has landed and every wave is done with the tiles before the
   // LDS is reused for the k-half sums.
   __builtin_amdgcn_s_waitcnt(0x0070);
-  if constexpr (kTokSplit) {
+  // This lane's four values of matrix m (0: first, 1: second), token block b
+  // and column run r4 in the split's partials, laid out as the lanes hold them.
+  auto part_at = [&](int m, int b, int r4) {
+    const int64_t tile = static_cast<int64_t>(blockIdx.y) * gridDim.x + blockIdx.x;
+    return reinterpret_cast<f32x4*>(a.part) +
+           ((((tile * 2 + m) * 2 + c) * TB + b) * 4 + r4) * kWave + lane;
+  };
+  if constexpr (kTokSplit && kPart) {
+#pragma unroll
+    for (int b = 0; b < NB; ++b)
+#pragma unroll
+      for (int r4 = 0; r4 < 4; ++r4) {
+        *part_at(0, b0 + b, r4) =
+            f32x4{g[b][4 * r4], g[b][4 * r4 + 1], g[b][4 * r4 + 2], g[b][4 * r4 + 3]};
+        *part_at(1, b0 + b, r4) =
+            f32x4{u[b][4 * r4], u[b][4 * r4 + 1], u[b][4 * r4 + 2], u[b][4 * r4 + 3]};
+      }
+  } else if constexpr (kTokSplit) {
     // Lane holds token 32(b0 + b) + l32 and, of column half c, columns
     // 8 (r / 4) + 4 hb + r % 4.
 #pragma unroll
@@ -438,6 +484,18 @@ __global__ void __launch_bounds__(kGThreads) gate_up_silu_small_kernel(GluArgs a
       const int tok = 32 * b + l32;
 #pragma unroll
       for (int r4 = 0; r4 < 4; ++r4) {
+        if constexpr (kPart) {
+          f32x4 pg, pu;
+#pragma unroll
+          for (int e = 0; e < 4; ++e) {
+            const int r = 4 * r4 + e;
+            pg[e] = g[b][r] + part[(32 * b + r) * kWave];
+            pu[e] = u[b][r] + part[(32 * b + 16 + r) * kWave];
+          }
+          *part_at(0, b, r4) = pg;
+          *part_at(1, b, r4) = pu;
+          continue;
+        }
         T v[4];
 #pragma unroll
         for (int e = 0; e < 4; ++e) {
@@ -454,22 +512,85 @@ __global__ void __launch_bounds__(kGThreads) gate_up_silu_small_kernel(GluArgs a
   }
 }
 
-template <typename T, int TB>
-int launch_small(const GluArgs& a, int inter, hipStream_t stream) {
-  const size_t lds = static_cast<size_t>(kSWStages) * kSWTile + 2 * TB * 32 * kGRowB;
-  hipLaunchKernelGGL((gate_up_silu_small_kernel<T, TB>), dim3(inter / kSCols), dim3(kGThreads),
-                     lds, stream, a);
-  return check_launch("gate_up_silu_small_kernel");
+// Sums the splits' partials in a fixed order and rounds.  kSilu: the first and
+// second matrix are the gate and up rows of the same 64 columns; else they are
+// 128 columns of one product.  A thread owns four consecutive columns of one
+// token, in the partials' own order, so a wave's reads are whole cache lines
+// and the splits' loads are independent.
+template <typename T, bool kSilu, int TB>
+__global__ void __launch_bounds__(256) split_sum_kernel(GluArgs a, int splits) {
+  constexpr int kPerM = 2 * TB * 4 * kWave;  // f32x4 of one matrix of a tile
+  const int tile = blockIdx.x, in = blockIdx.y * 256 + threadIdx.x;
+  const int m = kSilu ? 0 : in / kPerM;
+  const int lane = in % kWave, r4 = (in / kWave) % 4;
+  const int b = (in / (4 * kWave)) % TB, c = (in / (4 * kWave * TB)) % 2;
+  const int tok = 32 * b + (lane & 31);
+  if (tok >= a.num_tokens) return;
+  const f32x4* p = reinterpret_cast<const f32x4*>(a.part) +
+                   static_cast<int64_t>(tile) * 2 * kPerM + in;
+  const int64_t step = static_cast<int64_t>(a.tiles) * 2 * kPerM;
+  f32x4 s = {0.f, 0.f, 0.f, 0.f}, s2 = s;
+#pragma unroll 8
+  for (int z = 0; z < splits; ++z) {
+    s += p[z * step];
+    if constexpr (kSilu) s2 += p[z * step + kPerM];
+  }
+  T v[4];
+#pragma unroll
+  for (int e = 0; e < 4; ++e) v[e] = Elem<T>::from_f(kSilu ? silu_mul1(s[e], s2[e]) : s[e]);
+  const int64_t col = static_cast<int64_t>(tile) * (kSilu ? kSCols : 2 * kSCols) + kSCols * m +
+                      32 * c + 8 * r4 + 4 * (lane >> 5);
+  *reinterpret_cast<u32x2*>(a.out + tok * a.os + 2 * col) = __builtin_bit_cast(u32x2, v);
 }
 
-template <typename T>
-int launch_gate_up_silu_small(const GluArgs& a, int inter, hipStream_t stream) {
-  switch ((a.num_tokens + 31) / 32) {
-    case 1: return launch_small<T, 1>(a, inter, stream);
-    case 2: return launch_small<T, 2>(a, inter, stream);
-    case 3: return launch_small<T, 3>(a, inter, stream);
-    default: return launch_small<T, 4>(a, inter, stream);
+// The few-token product over `splits` ranges of a.k_per k-steps.  kSilu: gate
+// and up rows with the SwiGLU epilogue (in the product kernel itself without
+// partials); else one plain product.
+template <typename T, bool kSilu, int TB>
+int launch_small_tb(const GluArgs& a, int splits, hipStream_t stream) {
+  const size_t lds = static_cast<size_t>(kSWStages) * kSWTile + 2 * TB * 32 * kGRowB;
+  if (!a.part) {
+    hipLaunchKernelGGL((gate_up_silu_small_kernel<T, TB, false>), dim3(a.tiles), dim3(kGThreads),
+                       lds, stream, a);
+    return check_launch("gate_up_silu_small_kernel");
   }
+  hipLaunchKernelGGL((gate_up_silu_small_kernel<T, TB, true>), dim3(a.tiles, splits),
+                     dim3(kGThreads), lds, stream, a);
+  const int st = check_launch("gate_up_silu_small_kernel");
+  if (st) return st;
+  hipLaunchKernelGGL((split_sum_kernel<T, kSilu, TB>), dim3(a.tiles, (kSilu ? 2 : 4) * TB),
+                     dim3(256), 0, stream, a, splits);
+  return check_launch("split_sum_kernel");
+}
+
+template <typename T, bool kSilu>
+int launch_small(const GluArgs& a, int splits, hipStream_t stream) {
+  switch ((a.num_tokens + 31) / 32) {
+    case 1: return launch_small_tb<T, kSilu, 1>(a, splits, stream);
+    case 2: return launch_small_tb<T, kSilu, 2>(a, splits, stream);
+    case 3: return launch_small_tb<T, kSilu, 3>(a, splits, stream);
+    default: return launch_small_tb<T, kSilu, 4>(a, splits, stream);
+  }
+}
+
+// Splits of the contraction for `tiles` column tiles of `ksteps` k-steps: up to
+// one workgroup per CU (256 CUs), each with at least kSplitMinSteps steps; its
+// three-stage ring keeps a CU's share of HBM busy, and more splits cost more
+// partials than they gain (linear, two workgroups per CU against one: 32768 x
+// 5120, 24 tokens 56.2 against 53.2 us, 14336 x 4096, 128 tokens 42.5 against
+// 35.7; at least 4 steps against 8: 8192 x 2048, 24 tokens 16.4 against 11.4).
+constexpr int kSplitGroups = 256;
+constexpr int kSplitMinSteps = 8;
+
+int split_plan(int tiles, int ksteps, int* k_per) {
+  const int s = std::max(1, std::min(kSplitGroups / std::max(1, tiles), ksteps / kSplitMinSteps));
+  *k_per = (ksteps + s - 1) / s;
+  return (ksteps + *k_per - 1) / *k_per;
+}
+
+size_t split_bytes(int tiles, int splits, int num_tokens) {
+  return static_cast<size_t>(splits) * tiles * 2 * kSCols * ((num_tokens + 31) / 32 * 32) *
+         sizeof(float);
 }
 
 template <typename T>
@@ -489,11 +610,15 @@ int launch_gate_up_silu(const GluArgs& a0, hipStream_t stream) {
 
 using namespace vaa;
 
-extern "C" int vaa_gate_up_silu(const uint16_t* x, int64_t x_stride, const uint16_t* w_gate,
-                                const uint16_t* w_up, int64_t w_stride, uint16_t* output,
-                                int64_t output_stride, int num_tokens, int hidden_size,
-                                int intermediate_size, int dtype, void* stream) {
-  const char* what = "vaa_gate_up_silu";
+namespace vaa {
+namespace {
+
+// The body of vaa_gate_up_silu, with the split's workspace (null: none).
+int gate_up_silu_impl(const char* what, const uint16_t* x, int64_t x_stride,
+                      const uint16_t* w_gate, const uint16_t* w_up, int64_t w_stride,
+                      uint16_t* output, int64_t output_stride, int num_tokens, int hidden_size,
+                      int intermediate_size, int dtype, void* workspace, size_t workspace_bytes,
+                      void* stream) {
   if (!valid_dtype(dtype)) return fail(VAA_ERR_UNSUPPORTED, "%s: dtype=%d", what, dtype);
   if (num_tokens < 0 || hidden_size <= 0 || intermediate_size <= 0)
     return fail(VAA_ERR_INVALID_ARG, "%s: num_tokens=%d hidden_size=%d intermediate_size=%d",
@@ -530,9 +655,120 @@ extern "C" int vaa_gate_up_silu(const uint16_t* x, int64_t x_stride, const uint1
       static_cast<int64_t>(kGI) * a.ws >= (int64_t(1) << 31))
     return fail(VAA_ERR_UNSUPPORTED, "%s: problem too large", what);
   a.tiles = static_cast<int>(tiles);
+  a.k_per = a.ksteps;
+  a.w_tile = kSCols * a.ws;
+  a.part = nullptr;
   hipStream_t s = static_cast<hipStream_t>(stream);
-  if (num_tokens <= kSmallTokens)
-    return dtype == VAA_DTYPE_F16 ? launch_gate_up_silu_small<f16>(a, intermediate_size, s)
-                                  : launch_gate_up_silu_small<bf16>(a, intermediate_size, s);
+  if (num_tokens <= kSmallTokens) {
+    a.tiles = intermediate_size / kSCols;
+    int splits = 1;
+    if (workspace) {
+      splits = split_plan(a.tiles, a.ksteps, &a.k_per);
+      if (splits > 1) {
+        const size_t need = split_bytes(a.tiles, splits, num_tokens);
+        if (workspace_bytes < need || !aligned16(workspace))
+          return fail(VAA_ERR_WORKSPACE,
+                      "%s: workspace of %zu bytes (16-byte aligned) needed, got %zu", what, need,
+                      workspace_bytes);
+        a.part = static_cast<float*>(workspace);
+      }
+    }
+    return dtype == VAA_DTYPE_F16 ? launch_small<f16, true>(a, splits, s)
+                                  : launch_small<bf16, true>(a, splits, s);
+  }
   return dtype == VAA_DTYPE_F16 ? launch_gate_up_silu<f16>(a, s) : launch_gate_up_silu<bf16>(a, s);
+}
+
+}  // namespace
+}  // namespace vaa
+
+extern "C" int vaa_gate_up_silu(const uint16_t* x, int64_t x_stride, const uint16_t* w_gate,
+                                const uint16_t* w_up, int64_t w_stride, uint16_t* output,
+                                int64_t output_stride, int num_tokens, int hidden_size,
+                                int intermediate_size, int dtype, void* stream) {
+  return gate_up_silu_impl("vaa_gate_up_silu", x, x_stride, w_gate, w_up, w_stride, output,
+                           output_stride, num_tokens, hidden_size, intermediate_size, dtype,
+                           nullptr, 0, stream);
+}
+
+extern "C" size_t vaa_gate_up_silu_workspace_size(int num_tokens, int hidden_size,
+                                                  int intermediate_size) {
+  if (num_tokens <= 0 || num_tokens > kSmallTokens || hidden_size <= 0 || hidden_size % kGK ||
+      intermediate_size <= 0 || intermediate_size % kGI)
+    return 0;
+  int k_per = 0;
+  const int tiles = intermediate_size / kSCols;
+  const int splits = split_plan(tiles, hidden_size / kGK, &k_per);
+  return splits > 1 ? split_bytes(tiles, splits, num_tokens) : 0;
+}
+
+extern "C" int vaa_gate_up_silu_split(const uint16_t* x, int64_t x_stride, const uint16_t* w_gate,
+                                      const uint16_t* w_up, int64_t w_stride, uint16_t* output,
+                                      int64_t output_stride, int num_tokens, int hidden_size,
+                                      int intermediate_size, int dtype, void* workspace,
+                                      size_t workspace_bytes, void* stream) {
+  const char* what = "vaa_gate_up_silu_split";
+  if (!workspace && vaa_gate_up_silu_workspace_size(num_tokens, hidden_size, intermediate_size))
+    return fail(VAA_ERR_WORKSPACE, "%s: null workspace", what);
+  return gate_up_silu_impl(what, x, x_stride, w_gate, w_up, w_stride, output, output_stride,
+                           num_tokens, hidden_size, intermediate_size, dtype, workspace,
+                           workspace_bytes, stream);
+}
+
+extern "C" size_t vaa_linear_small_workspace_size(int num_tokens, int in_features,
+                                                  int out_features) {
+  if (num_tokens <= 0 || num_tokens > kSmallTokens || in_features <= 0 || in_features % kGK ||
+      out_features <= 0 || out_features % (2 * kSCols))
+    return 0;
+  int k_per = 0;
+  const int tiles = out_features / (2 * kSCols);
+  return split_bytes(tiles, split_plan(tiles, in_features / kGK, &k_per), num_tokens);
+}
+
+extern "C" int vaa_linear_small(const uint16_t* x, int64_t x_stride, const uint16_t* w,
+                                int64_t w_stride, uint16_t* output, int64_t output_stride,
+                                int num_tokens, int in_features, int out_features, int dtype,
+                                void* workspace, size_t workspace_bytes, void* stream) {
+  const char* what = "vaa_linear_small";
+  if (!valid_dtype(dtype)) return fail(VAA_ERR_UNSUPPORTED, "%s: dtype=%d", what, dtype);
+  if (num_tokens < 0 || in_features <= 0 || out_features <= 0)
+    return fail(VAA_ERR_INVALID_ARG, "%s: num_tokens=%d in_features=%d out_features=%d", what,
+                num_tokens, in_features, out_features);
+  if (num_tokens > kSmallTokens || in_features % kGK || out_features % (2 * kSCols))
+    return fail(VAA_ERR_UNSUPPORTED,
+                "%s: num_tokens=%d (at most %d), in_features=%d (a multiple of %d), "
+                "out_features=%d (a multiple of %d)",
+                what, num_tokens, kSmallTokens, in_features, kGK, out_features, 2 * kSCols);
+  if (num_tokens == 0) return VAA_OK;
+  if (!x || !w || !output) return fail(VAA_ERR_INVALID_ARG, "%s: null pointer", what);
+  if (x_stride < in_features || w_stride < in_features || output_stride < out_features ||
+      x_stride % 8 || w_stride % 8 || output_stride % 8)
+    return fail(VAA_ERR_INVALID_ARG, "%s: strides x=%lld w=%lld out=%lld", what,
+                (long long)x_stride, (long long)w_stride, (long long)output_stride);
+  if (!aligned16(x) || !aligned16(w) || !aligned16(output))
+    return fail(VAA_ERR_INVALID_ARG, "%s: x, weights and output must be 16-byte aligned", what);
+  GluArgs a;
+  a.x = reinterpret_cast<const char*>(x);
+  a.wg = reinterpret_cast<const char*>(w);
+  a.xs = 2 * x_stride;
+  a.ws = 2 * w_stride;
+  a.os = 2 * output_stride;
+  a.wu = a.wg + kSCols * a.ws;
+  a.w_tile = 2 * kSCols * a.ws;
+  a.out = reinterpret_cast<char*>(output);
+  a.num_tokens = num_tokens;
+  a.ksteps = in_features / kGK;
+  a.t_tiles = 1;
+  a.tiles = out_features / (2 * kSCols);
+  if (num_tokens * a.xs >= (int64_t(1) << 31) || kSCols * a.ws >= (int64_t(1) << 31))
+    return fail(VAA_ERR_UNSUPPORTED, "%s: problem too large", what);
+  const int splits = split_plan(a.tiles, a.ksteps, &a.k_per);
+  const size_t need = split_bytes(a.tiles, splits, num_tokens);
+  if (!workspace || workspace_bytes < need || !aligned16(workspace))
+    return fail(VAA_ERR_WORKSPACE, "%s: workspace of %zu bytes (16-byte aligned) needed, got %zu",
+                what, need, workspace ? workspace_bytes : static_cast<size_t>(0));
+  a.part = static_cast<float*>(workspace);
+  hipStream_t s = static_cast<hipStream_t>(stream);
+  return dtype == VAA_DTYPE_F16 ? launch_small<f16, false>(a, splits, s)
+                                : launch_small<bf16, false>(a, splits, s);
 }

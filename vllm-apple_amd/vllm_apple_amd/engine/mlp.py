@@ -4,9 +4,10 @@ encode (mlp.py:170-245 with _encode_gated_mlp, :247-384) computes
 down_proj(silu(gate_proj(x)) * up_proj(x)).  The reference runs the gate and
 up GEMMs into two [T, I] intermediates and a silu_mul pass over them; here
 the first half is one MFMA kernel with the SwiGLU epilogue
-(kernels.gate_up_silu), so only the activated [T, I] intermediate exists, and
-the down projection is a plain library GEMM (torch.matmul on the step's
-stream).  Weights keep the reference's layouts: gate_proj / up_proj [I, H]
+(kernels.gate_up_silu), so only the activated [T, I] intermediate exists.  The
+down projection of few tokens (kernels.linear_small_pays) streams its weights
+through kernels.linear_small; otherwise it is a plain library GEMM (torch.matmul on the
+step's stream).  Weights keep the reference's layouts: gate_proj / up_proj [I, H]
 or the fused gate_up_proj [2I, H] (gate rows first), down_proj [H, I].
 
 Above FUSED_MAX_TOKENS tokens encode takes the reference's order instead: a
@@ -157,7 +158,11 @@ class EngineMLP:
                     torch.matmul(x, self._gate_proj.t(), out=gu[:, :I])
                     torch.matmul(x, self._up_proj.t(), out=gu[:, I:])
                 kernels.silu_mul(gu[:, :I], gu[:, I:], out=act, stream=s)
-            torch.matmul(act, self._down_proj.t(), out=out)
+            if (kernels.linear_small_ok(act, self._down_proj, out)
+                    and kernels.linear_small_pays(act, self._down_proj)):
+                kernels.linear_small(act, self._down_proj, out, stream=s)
+            else:
+                torch.matmul(act, self._down_proj.t(), out=out)
 
     def get_intermediate_size(self, num_tokens: int) -> int:
         """Bytes of intermediate buffer encode needs: the one activated
