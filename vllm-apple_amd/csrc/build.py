@@ -21,6 +21,7 @@ INCLUDE = REPO / "include"
 OUT_DIR = PKG_ROOT / "vllm_apple_amd"
 LIB_NAME = "libvllm_apple_amd.so"
 OBJ_DIR = PKG_ROOT / "_build"
+HOST_NAME = "_host.so"                      # the Python extension (host_calls.cpp)
 
 SOURCES = [
     "status.hip",
@@ -88,10 +89,36 @@ def _compile(src: str) -> Path:
     return obj
 
 
+def build_host() -> Path:
+    """The wrappers' native host path: a CPython extension over torch's C++
+    headers, plain host code."""
+    import sysconfig
+
+    import torch
+    from torch.utils.cpp_extension import include_paths, library_paths
+
+    out = OUT_DIR / HOST_NAME
+    tmp = OBJ_DIR / (HOST_NAME + ".tmp")
+    cxx = os.environ.get("CXX") or shutil.which("g++") or hipcc()
+    cmd = [cxx, "-O2", "-std=c++17", "-fPIC", "-shared", "-Wall",
+           f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}",
+           f"-I{INCLUDE}", f"-I{sysconfig.get_paths()['include']}",
+           *(f"-isystem{d}" for d in include_paths()), str(HERE / "host_calls.cpp"),
+           "-o", str(tmp), *(f"-L{d}" for d in library_paths()),
+           "-ltorch_python", "-ltorch_cpu", "-lc10", "-ldl"]
+    res = subprocess.run(cmd, capture_output=True, text=True)
+    if res.returncode != 0:
+        raise RuntimeError(f"{cxx} failed for host_calls.cpp:\n{res.stderr}")
+    os.replace(tmp, out)
+    return out
+
+
 def build(verbose: bool = True) -> Path:
     OBJ_DIR.mkdir(parents=True, exist_ok=True)
     with cf.ThreadPoolExecutor(max_workers=min(len(SOURCES), os.cpu_count() or 4)) as ex:
+        host = ex.submit(build_host)
         objs = list(ex.map(_compile, SOURCES))
+        host.result()
     out = OUT_DIR / LIB_NAME
     tmp = out.with_suffix(".so.tmp")
     cmd = [hipcc(), f"--offload-arch={ARCH}", "-shared", "-fPIC", *map(str, objs), "-o", str(tmp)]

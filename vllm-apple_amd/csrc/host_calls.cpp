@@ -1,0 +1,566 @@
+// Native host path of the functional wrappers (vllm_apple_amd/kernels.py and
+// backend.py): each function reads the tensors' metadata, makes the same
+// checks as its Python wrapper and calls the C ABI, in 1 to 3 us instead of 10
+// to 40 (one decode step through the vLLM backend: 43 us of Python for two
+// launches before).  A function returns
+//   True          the work is enqueued;
+//   False         something is not the plain accepted case: nothing is
+//                 enqueued that the wrapper's own path does not repeat, and
+//                 the wrapper goes on from its first line, which converts,
+//                 or raises the same error as ever;
+//   an int n > 0  nothing is enqueued and n bytes of workspace are needed.
+// No state is kept between calls.  The library's entry points are looked up in
+// the handle that _lib.py loaded (bind), so both use one library.
+#define PY_SSIZE_T_CLEAN
+#include <Python.h>
+#include <dlfcn.h>
+#include <torch/csrc/autograd/python_variable.h>
+
+#include "vllm_apple_amd.h"
+
+namespace {
+
+#define VAA_FUNCS(X)                                                                      \
+  X(vaa_kv_write_slots) X(vaa_paged_attention_decode)                                     \
+  X(vaa_paged_attention_decode_workspace_size) X(vaa_paged_attention_prefill)             \
+  X(vaa_build_token_index) X(vaa_rmsnorm) X(vaa_add_rmsnorm) X(vaa_silu_mul)              \
+  X(vaa_qkv_epilogue) X(vaa_topk_logits) X(vaa_topk_workspace_size)                       \
+  X(vaa_gate_up_silu_split) X(vaa_gate_up_silu_workspace_size) X(vaa_linear_small)        \
+  X(vaa_linear_small_workspace_size) X(vaa_attention_no_cache)                            \
+  X(vaa_attention_no_cache_workspace_size)
+#define VAA_DECL(f) decltype(&::f) p_##f = nullptr;
+VAA_FUNCS(VAA_DECL)
+#undef VAA_DECL
+
+using at::Tensor;
+
+// args[i] as a tensor, or null for None (or anything else).
+const Tensor* ten(PyObject* o) {
+  return THPVariable_Check(o) ? &THPVariable_Unpack(o) : nullptr;
+}
+bool none_or_ten(PyObject* o) { return o == Py_None || THPVariable_Check(o); }
+
+void* ptr(const Tensor& t) { return const_cast<void*>(t.const_data_ptr()); }
+uint16_t* p16(const Tensor& t) { return static_cast<uint16_t*>(ptr(t)); }
+
+bool on_gpu(const Tensor& t) { return t.is_cuda() && t.layout() == at::kStrided; }
+
+// VAA_DTYPE_* of a GPU tensor of the two 16-bit types, else -1.
+int dt16(const Tensor& t) {
+  if (!on_gpu(t)) return -1;
+  if (t.scalar_type() == at::kHalf) return VAA_DTYPE_F16;
+  if (t.scalar_type() == at::kBFloat16) return VAA_DTYPE_BF16;
+  return -1;
+}
+bool is_i32(const Tensor& t) {
+  return on_gpu(t) && t.scalar_type() == at::kInt && t.is_contiguous();
+}
+// A slot mapping of at least n entries: VAA_INDEX_*, else -1.
+int slot_type(const Tensor& t, int64_t n) {
+  if (!on_gpu(t) || !t.is_contiguous() || t.numel() < n) return -1;
+  if (t.scalar_type() == at::kLong) return VAA_INDEX_I64;
+  if (t.scalar_type() == at::kInt) return VAA_INDEX_I32;
+  return -1;
+}
+// [tokens, heads, head_size] with a contiguous last dim.
+bool rows3(const Tensor& t) { return t.dim() == 3 && t.stride(2) == 1; }
+bool small(int64_t v) { return v >= 0 && v < (int64_t{1} << 31); }
+
+// Cache fields of p from one K and one V cache tensor of four dims (kernel
+// layout [nb, KV, bs, D], vLLM layout [nb, bs, KV, D]); false when they are not
+// what the wrappers take.
+bool cache4(const Tensor& k, const Tensor& v, bool vllm, vaa_attn_params* p) {
+  if (k.dim() != 4 || v.dim() != 4 || k.stride(3) != 1 || v.stride(3) != 1 ||
+      k.sizes() != v.sizes())
+    return false;
+  const int h = vllm ? 2 : 1, t = vllm ? 1 : 2;
+  if (!small(k.size(h)) || !small(k.size(t)) || !small(k.size(3)) || k.size(h) == 0) return false;
+  p->num_blocks = k.size(0);
+  p->num_kv_heads = k.size(h);
+  p->block_size = k.size(t);
+  p->head_size = k.size(3);
+  p->k_stride_block = k.stride(0);
+  p->k_stride_head = k.stride(h);
+  p->k_stride_token = k.stride(t);
+  p->v_stride_block = v.stride(0);
+  p->v_stride_head = v.stride(h);
+  p->v_stride_token = v.stride(t);
+  return true;
+}
+bool heads(int64_t H, vaa_attn_params* p) {
+  if (!small(H) || H == 0 || H % p->num_kv_heads) return false;
+  p->num_query_heads = H;
+  p->queries_per_kv = H / p->num_kv_heads;
+  return true;
+}
+bool same_rows(const Tensor& a, const Tensor& b) {
+  return a.sizes() == b.sizes() && a.strides() == b.strides();
+}
+
+PyObject* yes(int status) {
+  if (status != VAA_OK) Py_RETURN_FALSE;  // the wrapper repeats the call and raises
+  Py_RETURN_TRUE;
+}
+
+// Arguments by position; any conversion error or exception falls back.
+struct Args {
+  PyObject* const* a;
+  int64_t i(int k) const {
+    const long long v = PyLong_AsLongLong(a[k]);
+    if (v == -1 && PyErr_Occurred()) throw 0;
+    return v;
+  }
+  double f(int k) const {
+    const double v = PyFloat_AsDouble(a[k]);
+    if (v == -1.0 && PyErr_Occurred()) throw 0;
+    return v;
+  }
+  bool b(int k) const { return a[k] == Py_True; }
+  void* s(int k) const { return reinterpret_cast<void*>(static_cast<intptr_t>(i(k))); }
+  const Tensor* t(int k) const { return ten(a[k]); }
+};
+
+template <int N, PyObject* (*F)(const Args&)>
+PyObject* guarded(PyObject*, PyObject* const* args, Py_ssize_t n) {
+  if (n != N) {
+    PyErr_Format(PyExc_TypeError, "expected %d arguments, got %zd", N, n);
+    return nullptr;
+  }
+  if (!p_vaa_rmsnorm) Py_RETURN_FALSE;  // not bound
+  try {
+    return F(Args{args});
+  } catch (...) {
+    PyErr_Clear();
+    Py_RETURN_FALSE;
+  }
+}
+
+// ------------------------------------------------------------ layer ops --
+
+// (x, w, residual or None, out, eps, stream, add)
+PyObject* norm(const Args& a) {
+  const Tensor *x = a.t(0), *w = a.t(1), *r = a.t(2), *o = a.t(3);
+  const bool add = a.b(6);
+  if (!x || !w || !o || !none_or_ten(a.a[2]) || (add && !r)) Py_RETURN_FALSE;
+  const int dt = dt16(*x);
+  if (dt < 0 || dt16(*w) != dt || dt16(*o) != dt || (r && dt16(*r) != dt)) Py_RETURN_FALSE;
+  if (x->dim() != 2 || x->stride(1) != 1 || !w->is_contiguous() || w->numel() != x->size(1) ||
+      o->sizes() != x->sizes() || o->stride(1) != 1 ||
+      (r && (r->sizes() != x->sizes() || r->stride(1) != 1)) || !small(x->size(0)) ||
+      !small(x->size(1)))
+    Py_RETURN_FALSE;
+  const float eps = static_cast<float>(a.f(4));
+  if (add)
+    return yes(p_vaa_add_rmsnorm(p16(*x), p16(*r), p16(*w), p16(*o), x->size(0), x->size(1),
+                                 x->stride(0), r->stride(0), o->stride(0), eps, dt, a.s(5)));
+  return yes(p_vaa_rmsnorm(p16(*x), p16(*o), p16(*w), r ? p16(*r) : nullptr, x->size(0),
+                           x->size(1), x->stride(0), o->stride(0), r ? r->stride(0) : 0, eps, dt,
+                           a.s(5)));
+}
+
+// (gate, up, out, stream): contiguous tensors
+PyObject* silu(const Args& a) {
+  const Tensor *g = a.t(0), *u = a.t(1), *o = a.t(2);
+  if (!g || !u || !o) Py_RETURN_FALSE;
+  const int dt = dt16(*g);
+  if (dt < 0 || dt16(*u) != dt || dt16(*o) != dt || g->sizes() != u->sizes() ||
+      o->sizes() != g->sizes() || !g->is_contiguous() || !u->is_contiguous() ||
+      !o->is_contiguous())
+    Py_RETURN_FALSE;
+  return yes(p_vaa_silu_mul(p16(*g), p16(*u), p16(*o), g->numel(), dt, a.s(3)));
+}
+
+// (q, k, v, pos, cos, sin, slots, k_cache, v_cache, bias or None, rot, vllm, stream)
+PyObject* epilogue(const Args& a) {
+  const Tensor *q = a.t(0), *k = a.t(1), *v = a.t(2), *pos = a.t(3), *c = a.t(4), *s = a.t(5),
+               *sl = a.t(6), *kc = a.t(7), *vc = a.t(8), *b = a.t(9);
+  if (!q || !k || !v || !pos || !c || !s || !sl || !kc || !vc || !none_or_ten(a.a[9]))
+    Py_RETURN_FALSE;
+  const int dt = dt16(*q);
+  if (dt < 0 || dt16(*k) != dt || dt16(*v) != dt || dt16(*kc) != dt || dt16(*vc) != dt ||
+      (b && dt16(*b) != dt))
+    Py_RETURN_FALSE;
+  for (const Tensor* t : {q, k, v})
+    if (!rows3(*t) || t->stride(1) != t->size(2)) Py_RETURN_FALSE;
+  if (!same_rows(*k, *v)) Py_RETURN_FALSE;
+  const int64_t T = q->size(0), H = q->size(1), D = q->size(2), KV = k->size(1), rot = a.i(10);
+  vaa_attn_params p{};
+  if (k->size(0) != T || k->size(2) != D || !small(T) || !is_i32(*pos) || pos->numel() < T ||
+      slot_type(*sl, T) < 0 || !on_gpu(*c) || !on_gpu(*s) || c->scalar_type() != at::kFloat ||
+      s->scalar_type() != at::kFloat || c->dim() != 2 || c->sizes() != s->sizes() ||
+      rot <= 0 || c->size(1) != rot / 2 || !c->is_contiguous() || !s->is_contiguous() ||
+      !small(c->size(0)) || !small(rot) ||
+      (b && (b->dim() != 1 || b->numel() != (H + 2 * KV) * D || !b->is_contiguous())) ||
+      !cache4(*kc, *vc, a.b(11), &p) || !heads(H, &p) || KV != p.num_kv_heads ||
+      D != p.head_size)
+    Py_RETURN_FALSE;
+  p.dtype = dt;
+  p.scale = 1.f;
+  p.q_stride_token = q->stride(0);
+  p.q_stride_head = q->stride(1);
+  p.new_kv_stride_token = k->stride(0);
+  p.new_kv_stride_head = k->stride(1);
+  return yes(p_vaa_qkv_epilogue(&p, p16(*q), p16(*k), p16(*v), b ? p16(*b) : nullptr,
+                                static_cast<float*>(ptr(*c)), static_cast<float*>(ptr(*s)), rot,
+                                c->size(0), static_cast<int32_t*>(ptr(*pos)), ptr(*sl),
+                                slot_type(*sl, T), p16(*kc), p16(*vc), T, a.s(12)));
+}
+
+// (logits, k, indices, values, workspace or None, stream)
+PyObject* topk(const Args& a) {
+  const Tensor *x = a.t(0), *idx = a.t(2), *val = a.t(3), *ws = a.t(4);
+  if (!x || !idx || !val || !none_or_ten(a.a[4])) Py_RETURN_FALSE;
+  const int64_t k = a.i(1);
+  if (dt16(*x) < 0 || dt16(*val) != dt16(*x) || x->dim() != 2 || x->stride(1) != 1 ||
+      !on_gpu(*idx) || idx->scalar_type() != at::kInt || idx->dim() != 2 || val->dim() != 2 ||
+      idx->strides() != val->strides() || idx->stride(1) != 1 || idx->sizes() != val->sizes() ||
+      idx->size(0) != x->size(0) || idx->size(1) != k || k < 1 || k > 256 || k > x->size(1) ||
+      !small(x->size(0)) || !small(x->size(1)))
+    Py_RETURN_FALSE;
+  size_t need = 0;
+  if (p_vaa_topk_workspace_size(x->size(0), x->size(1), k, &need) != VAA_OK) Py_RETURN_FALSE;
+  if (need && (!ws || !on_gpu(*ws) || ws->nbytes() < need)) return PyLong_FromSize_t(need);
+  return yes(p_vaa_topk_logits(p16(*x), x->size(0), x->size(1), x->stride(0), k,
+                               static_cast<int32_t*>(ptr(*idx)), p16(*val), idx->stride(0),
+                               ws ? ptr(*ws) : nullptr, ws ? ws->nbytes() : 0, a.s(5)));
+}
+
+bool mat16(const Tensor& t, int dt) {
+  return dt16(t) == dt && t.dim() == 2 && t.stride(1) == 1 && small(t.size(0)) &&
+         small(t.size(1));
+}
+
+// (x, gate weight or fused gate/up weight, up weight or None, out, workspace or
+// None, stream)
+PyObject* gate_up(const Args& a) {
+  const Tensor *x = a.t(0), *g = a.t(1), *u = a.t(2), *o = a.t(3), *ws = a.t(4);
+  if (!x || !g || !o || !none_or_ten(a.a[2]) || !none_or_ten(a.a[4])) Py_RETURN_FALSE;
+  const int dt = dt16(*x);
+  if (dt < 0 || !mat16(*x, dt) || !mat16(*g, dt) || !mat16(*o, dt) || (u && !mat16(*u, dt)))
+    Py_RETURN_FALSE;
+  const int64_t T = x->size(0), H = x->size(1);
+  int64_t I = g->size(0);
+  const uint16_t* up;
+  if (u) {
+    if (u->sizes() != g->sizes() || u->stride(0) != g->stride(0)) Py_RETURN_FALSE;
+    up = p16(*u);
+  } else {
+    if (I % 2) Py_RETURN_FALSE;
+    I /= 2;
+    up = p16(*g) + I * g->stride(0);
+  }
+  if (g->size(1) != H || o->size(0) != T || o->size(1) != I) Py_RETURN_FALSE;
+  const size_t need = p_vaa_gate_up_silu_workspace_size(T, H, I);
+  if (need && (!ws || !on_gpu(*ws) || ws->nbytes() < need)) return PyLong_FromSize_t(need);
+  return yes(p_vaa_gate_up_silu_split(p16(*x), x->stride(0), p16(*g), up, g->stride(0), p16(*o),
+                                      o->stride(0), T, H, I, dt, ws ? ptr(*ws) : nullptr,
+                                      ws ? ws->nbytes() : 0, a.s(5)));
+}
+
+// (x, weight, out, workspace or None, stream); what linear_small_ok accepts.
+PyObject* linear(const Args& a) {
+  const Tensor *x = a.t(0), *w = a.t(1), *o = a.t(2), *ws = a.t(3);
+  if (!x || !w || !o || !none_or_ten(a.a[3])) Py_RETURN_FALSE;
+  const int dt = dt16(*x);
+  if (dt < 0 || !mat16(*x, dt) || !mat16(*w, dt) || !mat16(*o, dt)) Py_RETURN_FALSE;
+  const int64_t T = x->size(0), K = x->size(1), N = w->size(0);
+  if (w->size(1) != K || o->size(0) != T || o->size(1) != N) Py_RETURN_FALSE;
+  const size_t need = p_vaa_linear_small_workspace_size(T, K, N);
+  if (!need) Py_RETURN_FALSE;
+  if (!ws || !on_gpu(*ws) || ws->nbytes() < need) return PyLong_FromSize_t(need);
+  return yes(p_vaa_linear_small(p16(*x), x->stride(0), p16(*w), w->stride(0), p16(*o),
+                                o->stride(0), T, K, N, dt, ptr(*ws), ws->nbytes(), a.s(4)));
+}
+
+// ------------------------------------------------------------ attention --
+
+// K/V rows key/value[:n] into the cache of p; 0 ok, else fall back.
+int write_rows(vaa_attn_params p, const Tensor& k, const Tensor& v, uint16_t* kc, uint16_t* vc,
+               const Tensor& slots, int64_t n, void* stream) {
+  const int it = slot_type(slots, n);
+  if (it < 0 || !rows3(k) || !same_rows(k, v) || k.size(0) < n || k.size(1) != p.num_kv_heads ||
+      k.size(2) != p.head_size)
+    return 1;
+  p.num_query_heads = p.num_kv_heads;
+  p.queries_per_kv = 1;
+  p.scale = 1.f;
+  p.new_kv_stride_token = k.stride(0);
+  p.new_kv_stride_head = k.stride(1);
+  return p_vaa_kv_write_slots(&p, kc, vc, ptr(slots), it, p16(k), p16(v), n, stream) != VAA_OK;
+}
+
+// (key, value, key_cache, value_cache, slots, vllm, stream)
+PyObject* kv_write(const Args& a) {
+  const Tensor *k = a.t(0), *v = a.t(1), *kc = a.t(2), *vc = a.t(3), *sl = a.t(4);
+  if (!k || !v || !kc || !vc || !sl) Py_RETURN_FALSE;
+  const int dt = dt16(*k);
+  vaa_attn_params p{};
+  if (dt < 0 || dt16(*v) != dt || dt16(*kc) != dt || dt16(*vc) != dt || k->dim() != 3 ||
+      !small(k->size(0)) || !cache4(*kc, *vc, a.b(5), &p))
+    Py_RETURN_FALSE;
+  p.dtype = dt;
+  if (write_rows(p, *k, *v, p16(*kc), p16(*vc), *sl, k->size(0), a.s(6))) Py_RETURN_FALSE;
+  Py_RETURN_TRUE;
+}
+
+// Fills the query, output, table and length fields of a decode over the first
+// n sequences; false: fall back.
+bool decode_params(const Tensor& q, const Tensor& o, const Tensor& bt, const Tensor& sl, int64_t n,
+                   double scale, int64_t max_len, int64_t part, vaa_attn_params* p) {
+  if (!rows3(q) || !rows3(o) || q.size(0) < n || o.size(0) < n || q.size(2) != p->head_size ||
+      !heads(q.size(1), p) || !is_i32(bt) || bt.dim() != 2 || bt.size(0) < n || !is_i32(sl) ||
+      sl.numel() < n || !small(n) || !small(bt.size(1)) || !small(max_len) ||
+      part != static_cast<int32_t>(part))
+    return false;
+  p->scale = static_cast<float>(scale);
+  p->num_seqs = n;
+  p->max_seq_len = max_len;
+  p->max_blocks_per_seq = bt.size(1);
+  p->partition_size = part;
+  p->q_stride_token = q.stride(0);
+  p->q_stride_head = q.stride(1);
+  p->o_stride_token = o.stride(0);
+  p->o_stride_head = o.stride(1);
+  return true;
+}
+
+// (query, key_cache, value_cache, block_table, seq_lens, output, new_keys or
+// None, new_values or None, vllm, scale, max_seq_len, partition_size,
+// workspace or None, stream)
+PyObject* decode(const Args& a) {
+  const Tensor *q = a.t(0), *kc = a.t(1), *vc = a.t(2), *bt = a.t(3), *sl = a.t(4), *o = a.t(5),
+               *nk = a.t(6), *nv = a.t(7), *ws = a.t(12);
+  if (!q || !kc || !vc || !bt || !sl || !o || !none_or_ten(a.a[6]) || !none_or_ten(a.a[7]) ||
+      !none_or_ten(a.a[12]) || !nk != !nv)
+    Py_RETURN_FALSE;
+  const int dt = dt16(*q);
+  vaa_attn_params p{};
+  const int64_t n = sl->numel();
+  if (dt < 0 || dt16(*kc) != dt || dt16(*vc) != dt || dt16(*o) != dt ||
+      !cache4(*kc, *vc, a.b(8), &p) ||
+      !decode_params(*q, *o, *bt, *sl, n, a.f(9), a.i(10), a.i(11), &p))
+    Py_RETURN_FALSE;
+  if (nk) {
+    // The wrapper checks neither the rows' count nor their shape; only the
+    // plain case is taken here.
+    if (dt16(*nk) != dt || dt16(*nv) != dt || !rows3(*nk) || !same_rows(*nk, *nv) ||
+        nk->size(0) < n || nk->size(1) != p.num_kv_heads || nk->size(2) != p.head_size)
+      Py_RETURN_FALSE;
+    p.new_kv_stride_token = nk->stride(0);
+    p.new_kv_stride_head = nk->stride(1);
+  }
+  p.dtype = dt;
+  const size_t need = p_vaa_paged_attention_decode_workspace_size(&p, nullptr);
+  if (need && (!ws || !on_gpu(*ws) || ws->nbytes() < need)) return PyLong_FromSize_t(need);
+  return yes(p_vaa_paged_attention_decode(
+      &p, p16(*q), p16(*kc), p16(*vc), static_cast<int32_t*>(ptr(*bt)),
+      static_cast<int32_t*>(ptr(*sl)), p16(*o), nk ? p16(*nk) : nullptr, nv ? p16(*nv) : nullptr,
+      need ? ptr(*ws) : nullptr, need ? ws->nbytes() : 0, a.s(13)));
+}
+
+// Cache fields of p from vLLM's [2, nb, bs, KV, D] tensor.
+bool cache5(const Tensor& c, vaa_attn_params* p, uint16_t** kc, uint16_t** vc) {
+  if (c.dim() != 5 || c.size(0) != 2 || c.stride(4) != 1 || !small(c.size(2)) ||
+      !small(c.size(3)) || !small(c.size(4)) || c.size(3) == 0)
+    return false;
+  p->num_blocks = c.size(1);
+  p->block_size = c.size(2);
+  p->num_kv_heads = c.size(3);
+  p->head_size = c.size(4);
+  p->k_stride_block = p->v_stride_block = c.stride(1);
+  p->k_stride_token = p->v_stride_token = c.stride(2);
+  p->k_stride_head = p->v_stride_head = c.stride(3);
+  *kc = p16(c);
+  *vc = *kc + c.stride(0);
+  return true;
+}
+
+// One decode step of the backend: the K/V rows of the first n tokens (with
+// write) go to the cache, then n sequences attend.
+// (query, key, value, kv_cache, output, block_table, seq_lens, slots, n, write,
+//  head_size, scale, max_seq_len, partition_size, workspace or None, stream)
+PyObject* step_decode(const Args& a) {
+  const Tensor *q = a.t(0), *k = a.t(1), *v = a.t(2), *c = a.t(3), *o = a.t(4), *bt = a.t(5),
+               *sl = a.t(6), *slots = a.t(7), *ws = a.t(14);
+  const bool write = a.b(9);
+  if (!q || !c || !o || !bt || !sl || (write && (!k || !v || !slots)) || !none_or_ten(a.a[14]))
+    Py_RETURN_FALSE;
+  const int dt = dt16(*q);
+  const int64_t n = a.i(8);
+  vaa_attn_params p{};
+  uint16_t *kc, *vc;
+  if (dt < 0 || n <= 0 || dt16(*c) != dt || dt16(*o) != dt ||
+      (write && (dt16(*k) != dt || dt16(*v) != dt)) || !cache5(*c, &p, &kc, &vc) ||
+      p.head_size != a.i(10) ||
+      !decode_params(*q, *o, *bt, *sl, n, a.f(11), a.i(12), a.i(13), &p))
+    Py_RETURN_FALSE;
+  p.dtype = dt;
+  const size_t need = p_vaa_paged_attention_decode_workspace_size(&p, nullptr);
+  if (need && (!ws || !on_gpu(*ws) || ws->nbytes() < need)) return PyLong_FromSize_t(need);
+  if (write && write_rows(p, *k, *v, kc, vc, *slots, n, a.s(15))) Py_RETURN_FALSE;
+  return yes(p_vaa_paged_attention_decode(&p, p16(*q), kc, vc, static_cast<int32_t*>(ptr(*bt)),
+                                          static_cast<int32_t*>(ptr(*sl)), p16(*o), nullptr,
+                                          nullptr, need ? ptr(*ws) : nullptr,
+                                          need ? ws->nbytes() : 0, a.s(15)));
+}
+
+// Fields of an unsplit prefill of tokens [0, n).
+bool prefill_params(const Tensor& q, const Tensor& o, const Tensor& bt, int64_t n, double scale,
+                    vaa_attn_params* p) {
+  if (!rows3(q) || !rows3(o) || q.size(0) < n || o.size(0) < n || q.size(2) != p->head_size ||
+      o.size(1) != q.size(1) || o.size(2) != q.size(2) || !heads(q.size(1), p) || !is_i32(bt) ||
+      bt.dim() != 2 || !small(bt.size(0)) || !small(bt.size(1)) || !small(n))
+    return false;
+  p->scale = static_cast<float>(scale);
+  p->num_seqs = bt.size(0);
+  p->max_blocks_per_seq = bt.size(1);
+  p->q_stride_token = q.stride(0);
+  p->q_stride_head = q.stride(1);
+  p->o_stride_token = o.stride(0);
+  p->o_stride_head = o.stride(1);
+  return true;
+}
+
+// One prefill-only step of the backend: K/V rows, the token index (into idx,
+// int32 [2 n]) and the unsplit prefill of the first n tokens.
+// (query, key, value, kv_cache, output, block_table, seq_lens, slots,
+//  query_start_loc, idx, n, write, head_size, scale, stream)
+PyObject* step_prefill(const Args& a) {
+  const Tensor *q = a.t(0), *k = a.t(1), *v = a.t(2), *c = a.t(3), *o = a.t(4), *bt = a.t(5),
+               *sl = a.t(6), *slots = a.t(7), *qsl = a.t(8), *idx = a.t(9);
+  const bool write = a.b(11);
+  if (!q || !c || !o || !bt || !sl || !qsl || !idx || (write && (!k || !v || !slots)))
+    Py_RETURN_FALSE;
+  const int dt = dt16(*q);
+  const int64_t n = a.i(10);
+  vaa_attn_params p{};
+  uint16_t *kc, *vc;
+  if (dt < 0 || n <= 0 || dt16(*c) != dt || dt16(*o) != dt ||
+      (write && (dt16(*k) != dt || dt16(*v) != dt)) || !cache5(*c, &p, &kc, &vc) ||
+      p.head_size != a.i(12) || !prefill_params(*q, *o, *bt, n, a.f(13), &p) || !is_i32(*qsl) ||
+      !is_i32(*sl) || qsl->numel() < 1 || !small(qsl->numel()) ||
+      sl->numel() < qsl->numel() - 1 || !is_i32(*idx) || idx->numel() < 2 * n)
+    Py_RETURN_FALSE;
+  p.dtype = dt;
+  void* stream = a.s(14);
+  int32_t* tok = static_cast<int32_t*>(ptr(*idx));
+  if (write && write_rows(p, *k, *v, kc, vc, *slots, n, stream)) Py_RETURN_FALSE;
+  if (p_vaa_build_token_index(static_cast<int32_t*>(ptr(*qsl)), static_cast<int32_t*>(ptr(*sl)),
+                              qsl->numel() - 1, n, tok, tok + n, stream) != VAA_OK)
+    Py_RETURN_FALSE;
+  return yes(p_vaa_paged_attention_prefill(&p, p16(*q), kc, vc, static_cast<int32_t*>(ptr(*bt)),
+                                           tok, tok + n, p16(*o), n, stream));
+}
+
+// (query, key_cache, value_cache, block_table, token_to_seq, positions, output,
+//  vllm, scale, stream): unsplit
+PyObject* prefill(const Args& a) {
+  const Tensor *q = a.t(0), *kc = a.t(1), *vc = a.t(2), *bt = a.t(3), *tok = a.t(4),
+               *pos = a.t(5), *o = a.t(6);
+  if (!q || !kc || !vc || !bt || !tok || !pos || !o) Py_RETURN_FALSE;
+  const int dt = dt16(*q);
+  vaa_attn_params p{};
+  if (dt < 0 || dt16(*kc) != dt || dt16(*vc) != dt || dt16(*o) != dt || q->dim() != 3 ||
+      !cache4(*kc, *vc, a.b(7), &p) || !prefill_params(*q, *o, *bt, q->size(0), a.f(8), &p) ||
+      !is_i32(*tok) || !is_i32(*pos) || tok->numel() < q->size(0) || pos->numel() < q->size(0))
+    Py_RETURN_FALSE;
+  p.dtype = dt;
+  return yes(p_vaa_paged_attention_prefill(&p, p16(*q), p16(*kc), p16(*vc),
+                                           static_cast<int32_t*>(ptr(*bt)),
+                                           static_cast<int32_t*>(ptr(*tok)),
+                                           static_cast<int32_t*>(ptr(*pos)), p16(*o), q->size(0),
+                                           a.s(9)));
+}
+
+// 16-byte aligned rows, which the attention kernels read directly.
+bool aligned_rows(const Tensor& t) {
+  return rows3(t) && t.stride(0) % 8 == 0 && t.stride(1) % 8 == 0 && t.stride(0) >= 0 &&
+         t.stride(1) >= 0 && (reinterpret_cast<uintptr_t>(ptr(t)) & 15u) == 0;
+}
+// Whether the address ranges of two tensors' first T rows meet.
+bool overlap(const Tensor& a, const Tensor& b, int64_t T) {
+  auto end = [T](const Tensor& t) {
+    return p16(t) + (T - 1) * t.stride(0) + (t.size(1) - 1) * t.stride(1) + t.size(2);
+  };
+  return p16(a) < end(b) && p16(b) < end(a);
+}
+
+// Attention of T tokens inside their sequences, K and V read in place; the
+// caller knows that query_start_loc runs from 0 to T without decreasing.
+// (query, key, value, output, query_start_loc, T, num_seqs, head_size, scale,
+//  max_seq_len, causal, workspace or None, stream)
+PyObject* no_cache(const Args& a) {
+  const Tensor *q = a.t(0), *k = a.t(1), *v = a.t(2), *o = a.t(3), *qsl = a.t(4), *ws = a.t(11);
+  if (!q || !k || !v || !o || !qsl || !none_or_ten(a.a[11])) Py_RETURN_FALSE;
+  const int dt = dt16(*q);
+  const int64_t T = a.i(5), S = a.i(6), L = a.i(9);
+  if (dt < 0 || dt16(*k) != dt || dt16(*v) != dt || dt16(*o) != dt || !small(T) || T == 0 ||
+      !small(S) || S == 0 || !small(L) || !is_i32(*qsl) || qsl->numel() != S + 1)
+    Py_RETURN_FALSE;
+  for (const Tensor* t : {q, k, v, o})
+    if (!aligned_rows(*t) || t->size(0) < T || t->size(2) != a.i(7) || t->size(1) == 0)
+      Py_RETURN_FALSE;
+  if (k->sizes() != v->sizes() || k->strides() != v->strides() || o->size(1) != q->size(1) ||
+      q->size(1) % k->size(1) || qsl->get_device() != q->get_device() || overlap(*o, *k, T) ||
+      overlap(*o, *v, T))
+    Py_RETURN_FALSE;
+  vaa_attn_params p{};
+  p.dtype = dt;
+  p.scale = static_cast<float>(a.f(8));
+  p.num_seqs = S;
+  p.max_seq_len = L;
+  p.head_size = q->size(2);
+  p.num_kv_heads = k->size(1);
+  p.num_query_heads = q->size(1);
+  p.queries_per_kv = q->size(1) / k->size(1);
+  p.k_stride_token = p.v_stride_token = k->stride(0);
+  p.k_stride_head = p.v_stride_head = k->stride(1);
+  p.q_stride_token = q->stride(0);
+  p.q_stride_head = q->stride(1);
+  p.o_stride_token = o->stride(0);
+  p.o_stride_head = o->stride(1);
+  const size_t need = p_vaa_attention_no_cache_workspace_size(S, T, L);
+  if (!ws || !on_gpu(*ws) || ws->nbytes() < need) return PyLong_FromSize_t(need);
+  return yes(p_vaa_attention_no_cache(&p, p16(*q), p16(*k), p16(*v),
+                                      static_cast<int32_t*>(ptr(*qsl)), p16(*o), T, a.b(10),
+                                      ptr(*ws), ws->nbytes(), a.s(12)));
+}
+
+// bind(handle): the entry points of the library that _lib.py loaded.
+PyObject* bind(PyObject*, PyObject* arg) {
+  void* h = PyLong_AsVoidPtr(arg);
+  if (PyErr_Occurred()) return nullptr;
+#define VAA_BIND(f)                                                    \
+  p_##f = reinterpret_cast<decltype(p_##f)>(dlsym(h, #f));             \
+  if (!p_##f) {                                                        \
+    p_vaa_rmsnorm = nullptr;                                           \
+    PyErr_SetString(PyExc_RuntimeError, "missing entry point " #f);    \
+    return nullptr;                                                    \
+  }
+  VAA_FUNCS(VAA_BIND)
+#undef VAA_BIND
+  Py_RETURN_NONE;
+}
+
+#define VAA_METHOD(name, n) \
+  {#name, reinterpret_cast<PyCFunction>(guarded<n, name>), METH_FASTCALL, nullptr}
+PyMethodDef methods[] = {{"bind", bind, METH_O, nullptr},
+                         VAA_METHOD(norm, 7),
+                         VAA_METHOD(silu, 4),
+                         VAA_METHOD(epilogue, 13),
+                         VAA_METHOD(topk, 6),
+                         VAA_METHOD(gate_up, 6),
+                         VAA_METHOD(linear, 5),
+                         VAA_METHOD(kv_write, 7),
+                         VAA_METHOD(decode, 14),
+                         VAA_METHOD(step_decode, 16),
+                         VAA_METHOD(step_prefill, 15),
+                         VAA_METHOD(prefill, 10),
+                         VAA_METHOD(no_cache, 13),
+                         {nullptr, nullptr, 0, nullptr}};
+PyModuleDef module = {PyModuleDef_HEAD_INIT, "_host", nullptr, -1, methods,
+                      nullptr,               nullptr, nullptr, nullptr};
+
+}  // namespace
+
+PyMODINIT_FUNC PyInit__host(void) { return PyModule_Create(&module); }

@@ -125,6 +125,7 @@ SIGNATURES = {
 
 _lock = threading.Lock()
 _lib: ctypes.CDLL | None = None
+_host = None  # the native host path (csrc/host_calls.cpp), bound to _lib
 
 
 def library_path() -> Path:
@@ -133,7 +134,7 @@ def library_path() -> Path:
 
 def load() -> ctypes.CDLL:
     """Load (once) and return the library, raising NativeLibraryError if absent."""
-    global _lib
+    global _lib, _host
     if _lib is not None:
         return _lib
     with _lock:
@@ -159,8 +160,22 @@ def load() -> ctypes.CDLL:
             fn = getattr(lib, name)
             fn.restype = res
             fn.argtypes = args
+        try:
+            from . import _host as host_module
+        except ImportError as e:
+            raise NativeLibraryError(
+                f"the host extension is not built ({e}); run vllm_apple_amd.build_library()") from e
+        host_module.bind(lib._handle)
+        _host = host_module
         _lib = lib
         return lib
+
+
+def host():
+    """The native host path of the wrappers, loaded with the library."""
+    if _host is None:
+        load()
+    return _host
 
 
 def last_error() -> str:
@@ -189,5 +204,5 @@ def call(name: str, *args) -> None:
 def stream_handle(stream: "torch.cuda.Stream | None" = None) -> int:
     """Raw hipStream_t of ``stream`` (default: torch's current stream)."""
     if stream is None:
-        stream = torch.cuda.current_stream()
+        return torch._C._cuda_getCurrentRawStream(torch._C._cuda_getDevice())
     return int(stream.cuda_stream)

@@ -244,23 +244,6 @@ def _overlap_enabled() -> bool:
     return os.environ.get(OVERLAP_ENV, "1") != "0"
 
 
-def _rows_ok(t: torch.Tensor) -> bool:
-    """16-byte aligned rows with a contiguous last dim: what the attention
-    kernels read directly."""
-    return (t.dim() == 3 and t.stride(2) == 1 and t.stride(1) % 8 == 0 and t.stride(0) % 8 == 0
-            and t.data_ptr() % 16 == 0)
-
-
-def _overlaps(a: torch.Tensor, b: torch.Tensor) -> bool:
-    """Whether the address ranges that two tensors span meet."""
-    def span(t):
-        n = sum((d - 1) * s for d, s in zip(t.shape, t.stride())) + 1
-        return t.data_ptr(), t.data_ptr() + n * t.element_size()
-
-    (a0, a1), (b0, b1) = span(a), span(b)
-    return a0 < b1 and b0 < a1
-
-
 class HipAttentionImpl(AttentionImpl):
     def __init__(self, num_heads: int, head_size: int, scale: float, num_kv_heads: int,
                  alibi_slopes: Optional[list], sliding_window: Optional[int],
@@ -363,9 +346,12 @@ class HipAttentionImpl(AttentionImpl):
 
         n = attn_metadata.num_actual_tokens
         if self.attn_type in (AttentionType.ENCODER_ONLY, AttentionType.ENCODER):
-            self._attention_no_cache(query[:n], key[:n], value[:n], output[:n], attn_metadata,
-                                     causal=False)
+            self._attention_no_cache(*(t if t.shape[0] == n else t[:n]
+                                       for t in (query, key, value, output)),
+                                     attn_metadata, causal=False)
         else:
+            if not conv and self._step_native(query, key, value, kv_cache, attn_metadata, output, n):
+                return output
             key_cache, value_cache = self._caches(kv_cache)
             if not self._is_kv_shared and key is not None and value is not None and n > 0:
                 kernels.kv_write_slots(key[:n], value[:n], key_cache, value_cache,
@@ -393,15 +379,8 @@ class HipAttentionImpl(AttentionImpl):
                 # decode; C5 attention step 0.61 ms against 0.68-0.79 split).
                 # The pieces are counted over the longest prefill context
                 # (decode contexts do not matter), which bounds the workspace.
-                split, longest = 0, 0
-                lens_host = attn_metadata._seq_lens_cpu
-                qsl_host = attn_metadata._query_start_loc_cpu
-                if lens_host and qsl_host and not overlapped:
-                    ql = [b - a if b - a > 1 else 0 for a, b in zip(qsl_host[:-1], qsl_host[1:])]
-                    split = kernels.choose_prefill_split(
-                        lens_host, ql, self.num_kv_heads, query.shape[1],
-                        kernels.device_cus(query.device), head_size=self.head_size)
-                    longest = max((l for l, q in zip(lens_host, ql) if q > 0), default=0)
+                split, longest = (0, 0) if overlapped else self._prefill_split(attn_metadata,
+                                                                               query)
                 kernels.paged_prefill(query[nd:n], key_cache, value_cache,
                                       attn_metadata.block_table, tok[nd:n], pos[nd:n],
                                       scale=self.scale, layout="vllm", output=output[nd:n],
@@ -425,6 +404,55 @@ class HipAttentionImpl(AttentionImpl):
             return original_output
         return output
 
+    def _step_native(self, query: torch.Tensor, key: Optional[torch.Tensor],
+                     value: Optional[torch.Tensor], kv_cache: torch.Tensor,
+                     md: HipAttentionMetadata, output: torch.Tensor, n: int) -> bool:
+        """A decode-only step, or a prefill-only one without a key split, in one
+        native call: the same launches as forward's own path, without the
+        slices and per-launch parameter blocks.  False, with nothing enqueued
+        that forward's path does not repeat, when the step is anything else."""
+        nd = md.num_decode_tokens
+        if n <= 0 or 0 < nd < n or not query.is_cuda or kv_cache.dim() != 5 or query.dim() != 3:
+            return False
+        kvh = kv_cache.shape[3]
+        if kvh == 0 or query.shape[1] < kvh:
+            return False
+        write = not self._is_kv_shared and key is not None and value is not None
+        lens = md._seq_lens_cpu
+        native, handle = kernels._lib.host(), kernels._lib.stream_handle()
+        if nd >= n:
+            part = kernels._decode_partition(query, kvh, lens[:nd], False) if lens else 0
+            args = (query, key, value, kv_cache, output, md.block_table, md.seq_lens,
+                    md.slot_mapping, nd, write, self.head_size, self.scale, md.max_seq_len, part)
+            if nd != n:
+                return False
+            done = native.step_decode(*args, kernels._decode_ws.current(query.device), handle)
+            if done is not True and done:
+                done = native.step_decode(*args, kernels.decode_workspace(done, query.device),
+                                          handle)
+            return done is True
+        # choose_prefill_split splits no batch whose contexts are all within
+        # 32 key tiles; longer ones are left to forward's path.
+        if lens and md._query_start_loc_cpu and max(lens) > 32 * kernels._PREFILL_KEY_TILE:
+            if self._prefill_split(md, query)[0]:
+                return False
+        idx = torch.empty(2 * n, dtype=torch.int32, device=query.device)
+        return native.step_prefill(query, key, value, kv_cache, output, md.block_table,
+                                   md.seq_lens, md.slot_mapping, md.query_start_loc, idx, n,
+                                   write, self.head_size, self.scale, handle) is True
+
+    def _prefill_split(self, md: HipAttentionMetadata, query: torch.Tensor) -> tuple:
+        """(key split, longest prefill context) of a step's prefill from the
+        host lengths; (0, 0) without them."""
+        lens_host, qsl_host = md._seq_lens_cpu, md._query_start_loc_cpu
+        if not lens_host or not qsl_host:
+            return 0, 0
+        ql = [b - a if b - a > 1 else 0 for a, b in zip(qsl_host[:-1], qsl_host[1:])]
+        split = kernels.choose_prefill_split(
+            lens_host, ql, self.num_kv_heads, query.shape[1],
+            kernels.device_cus(query.device), head_size=self.head_size)
+        return split, max((l for l, q in zip(lens_host, ql) if q > 0), default=0)
+
     def _attention_no_cache(self, query: torch.Tensor, key: torch.Tensor, value: torch.Tensor,
                             output: torch.Tensor, attn_metadata: HipAttentionMetadata,
                             causal: bool) -> torch.Tensor:
@@ -432,7 +460,7 @@ class HipAttentionImpl(AttentionImpl):
         the semantics of _compute_attention_sdpa (base_attn.py:223-306).
 
         Rows that the kernels can read directly, with the sequence starts at
-        hand on the device, run in place (kernels.attention_no_cache).
+        hand on the device, run in place (kernels.try_attention_no_cache).
         Otherwise the tokens are staged into a scratch paged cache, one
         block-aligned range per sequence, and run through the prefill kernel;
         positions are the in-sequence index (causal) or the last index
@@ -444,21 +472,12 @@ class HipAttentionImpl(AttentionImpl):
         if T <= 0:
             return output
         lens_host = [b - a for a, b in zip(qsl[:-1], qsl[1:])]
-        dqsl = attn_metadata.query_start_loc
         if (qsl[0] == 0 and min(lens_host) >= 0 and T == qsl[-1]
-                and isinstance(dqsl, torch.Tensor) and dqsl.dtype == torch.int32
-                and dqsl.device == query.device and dqsl.is_contiguous()
-                and dqsl.numel() == num_seqs + 1
-                and min(key.shape[0], value.shape[0], output.shape[0]) >= T
-                and key.shape == value.shape and key.stride() == value.stride()
-                and key.shape[2] == self.head_size == query.shape[2]
-                and query.shape[1] % key.shape[1] == 0
-                and query.shape[1:] == output.shape[1:]
-                and all(_rows_ok(t) for t in (query, key, value, output))
-                and not _overlaps(output, key) and not _overlaps(output, value)):
-            kernels.attention_no_cache(query[:T], key[:T], value[:T], dqsl, output[:T],
-                                       scale=self.scale, max_seq_len=max(lens_host),
-                                       causal=causal)
+                and isinstance(attn_metadata.query_start_loc, torch.Tensor)
+                and kernels.try_attention_no_cache(
+                    query, key, value, output, attn_metadata.query_start_loc, num_tokens=T,
+                    num_seqs=num_seqs, head_size=self.head_size, scale=self.scale,
+                    max_seq_len=max(lens_host), causal=causal)):
             return output
         bs = 16
         dev = query.device

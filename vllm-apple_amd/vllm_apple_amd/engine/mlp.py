@@ -89,15 +89,16 @@ class EngineMLP:
         return x, 0
 
     def _grow(self, name: str, n: int, like: torch.Tensor,
-              stream: torch.cuda.Stream) -> torch.Tensor:
+              stream: Optional[torch.cuda.Stream], handle: int) -> torch.Tensor:
         """A grow-only scratch of at least n elements kept in attribute
-        `name`, allocated on the stream that writes and reads it.  An outgrown
-        buffer is kept alive, never freed, as kernels._GrowOnlyScratch does: a
-        HIP graph captured while it was current holds its address, and a
-        replay must not write into memory the caching allocator has handed to
-        another tensor.  Sizes grow at least 2x, so the kept buffers sum to
-        less than the current one.  A scratch first made on another stream is
-        marked as used on this one (record_stream)."""
+        `name`, allocated on the stream that writes and reads it (None: the
+        current one; handle: its raw handle).  An outgrown buffer is kept
+        alive, never freed, as kernels._GrowOnlyScratch does: a HIP graph
+        captured while it was current holds its address, and a replay must not
+        write into memory the caching allocator has handed to another tensor.
+        Sizes grow at least 2x, so the kept buffers sum to less than the
+        current one.  A scratch first made on another stream is marked as used
+        on this one (record_stream)."""
         buf, streams = getattr(self, name), getattr(self, name + "_streams")
         if buf is None or buf.numel() < n or buf.dtype != like.dtype or buf.device != like.device:
             size = n
@@ -108,18 +109,19 @@ class EngineMLP:
             with torch.cuda.stream(stream):
                 buf = torch.empty(size, dtype=like.dtype, device=like.device)
             setattr(self, name, buf)
-            setattr(self, name + "_streams", {stream.cuda_stream})
-        elif stream.cuda_stream not in streams:
-            buf.record_stream(stream)
-            streams.add(stream.cuda_stream)
+            setattr(self, name + "_streams", {handle})
+        elif handle not in streams:
+            buf.record_stream(stream if stream is not None
+                              else torch.cuda.current_stream(like.device))
+            streams.add(handle)
         return buf
 
     def _intermediate(self, num_tokens: int, like: torch.Tensor,
-                      stream: torch.cuda.Stream) -> torch.Tensor:
+                      stream: Optional[torch.cuda.Stream], handle: int) -> torch.Tensor:
         """The activated [T, I] scratch."""
         n = num_tokens * self.config.intermediate_size
-        return self._grow("_scratch", n, like, stream)[:n].view(num_tokens,
-                                                                self.config.intermediate_size)
+        return self._grow("_scratch", n, like, stream, handle)[:n].view(
+            num_tokens, self.config.intermediate_size)
 
     def encode(self, step_ctx: Any, hidden_states: Any, output_buffer: Any, num_tokens: int,
                intermediate_buffer: Optional[Any] = None) -> None:
@@ -135,34 +137,47 @@ class EngineMLP:
         ob, oo = self._buf(output_buffer)
         x = view(hb, ho, (num_tokens, H), dtype=hb.dtype)
         out = view(ob, oo, (num_tokens, H), dtype=ob.dtype)
-        s = stream if stream is not None else torch.cuda.current_stream(x.device)
+        if stream is None:
+            # The buffers' device's current stream.
+            handle = torch._C._cuda_getCurrentRawStream(x.device.index) if x.is_cuda else 0
+        else:
+            handle = stream.cuda_stream
         if intermediate_buffer is not None:
             ib, io = self._buf(intermediate_buffer)
             act = view(ib, io, (num_tokens, I), dtype=ib.dtype)
         else:
-            act = self._intermediate(num_tokens, x, s)
-        with torch.cuda.stream(s):
-            if num_tokens <= self.fused_max_tokens:
-                if self._fused_gate_up:
-                    kernels.gate_up_silu(x, self._gate_up_proj, out=act, stream=s)
-                else:
-                    kernels.gate_up_silu(x, self._gate_proj, self._up_proj, out=act, stream=s)
+            act = self._intermediate(num_tokens, x, stream, handle)
+        if stream is None and x.is_cuda and x.device.index == torch.cuda.current_device():
+            self._run(x, act, out, num_tokens, None, handle)
+        else:
+            s = stream if stream is not None else torch.cuda.current_stream(x.device)
+            with torch.cuda.stream(s):
+                self._run(x, act, out, num_tokens, s, handle)
+
+    def _run(self, x: torch.Tensor, act: torch.Tensor, out: torch.Tensor, num_tokens: int,
+             s: Optional[torch.cuda.Stream], handle: int) -> None:
+        """The two halves, enqueued on s, which is the current stream (None:
+        whichever that is)."""
+        I = self.config.intermediate_size
+        if num_tokens <= self.fused_max_tokens:
+            if self._fused_gate_up:
+                kernels.gate_up_silu(x, self._gate_up_proj, out=act, stream=s)
             else:
-                # The reference's order (mlp.py:247-330): both GEMMs into one
-                # [T, 2I] scratch, then silu_mul over its halves.
-                gu = self._grow("_gu", 2 * num_tokens * I, x, s)[:2 * num_tokens * I]
-                gu = gu.view(num_tokens, 2 * I)
-                if self._fused_gate_up:
-                    torch.matmul(x, self._gate_up_proj.t(), out=gu)
-                else:
-                    torch.matmul(x, self._gate_proj.t(), out=gu[:, :I])
-                    torch.matmul(x, self._up_proj.t(), out=gu[:, I:])
-                kernels.silu_mul(gu[:, :I], gu[:, I:], out=act, stream=s)
-            if (kernels.linear_small_ok(act, self._down_proj, out)
-                    and kernels.linear_small_pays(act, self._down_proj)):
-                kernels.linear_small(act, self._down_proj, out, stream=s)
+                kernels.gate_up_silu(x, self._gate_proj, self._up_proj, out=act, stream=s)
+        else:
+            # The reference's order (mlp.py:247-330): both GEMMs into one
+            # [T, 2I] scratch, then silu_mul over its halves.
+            gu = self._grow("_gu", 2 * num_tokens * I, x, s, handle)[:2 * num_tokens * I]
+            gu = gu.view(num_tokens, 2 * I)
+            if self._fused_gate_up:
+                torch.matmul(x, self._gate_up_proj.t(), out=gu)
             else:
-                torch.matmul(act, self._down_proj.t(), out=out)
+                torch.matmul(x, self._gate_proj.t(), out=gu[:, :I])
+                torch.matmul(x, self._up_proj.t(), out=gu[:, I:])
+            kernels.silu_mul(gu[:, :I], gu[:, I:], out=act, stream=s)
+        if not (kernels.linear_small_pays(act, self._down_proj)
+                and kernels.try_linear_small(act, self._down_proj, out, stream=s)):
+            torch.matmul(act, self._down_proj.t(), out=out)
 
     def get_intermediate_size(self, num_tokens: int) -> int:
         """Bytes of intermediate buffer encode needs: the one activated

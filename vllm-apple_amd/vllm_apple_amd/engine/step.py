@@ -66,6 +66,8 @@ def view(buffer: torch.Tensor, byte_offset: int, shape, dtype=torch.float16) -> 
         raise ValueError(f"buffer dtype {buffer.dtype} != {dtype}")
     if not buffer.is_contiguous():
         raise ValueError("engine buffers must be contiguous")
+    if byte_offset == 0 and tuple(buffer.shape) == tuple(shape):
+        return buffer
     esz = buffer.element_size()
     if byte_offset % esz:
         raise ValueError(f"byte offset {byte_offset} not a multiple of {esz}")

@@ -21,6 +21,10 @@ import torch
 from . import _lib
 
 LAYOUTS = ("kernel", "vllm")
+# The hot wrappers first offer a call to their native counterpart
+# (csrc/host_calls.cpp), which takes the plain accepted case whole; anything
+# else goes on below it, where it is converted or refused.
+_IS_VLLM = {"kernel": False, "vllm": True}
 
 
 def _ptr(t: torch.Tensor | None) -> int | None:
@@ -135,6 +139,10 @@ def kv_write_slots(key: torch.Tensor, value: torch.Tensor, key_cache: torch.Tens
     strides with a contiguous last dim); slot_mapping: int32 or int64
     [num_tokens].  Mirrors kv_write.py:118-156 and base_attn.py:308-342.
     """
+    if key.is_cuda and layout in _IS_VLLM and _lib.host().kv_write(
+            key, value, key_cache, value_cache, slot_mapping, _IS_VLLM[layout],
+            _lib.stream_handle(stream)) is True:
+        return
     _require_gpu(key, value, key_cache, value_cache, slot_mapping)
     _attn_dtype(key=key, value=value, key_cache=key_cache, value_cache=value_cache)
     if key.stride() != value.stride() or key.shape != value.shape:
@@ -232,6 +240,10 @@ class _GrowOnlyScratch:
         self._retired: list[torch.Tensor] = []
         self._min = min_bytes
 
+    def current(self, device: torch.device) -> torch.Tensor | None:
+        """The device's present buffer, if any."""
+        return self._cur.get(_dev_index(device))
+
     def get(self, nbytes: int, device: torch.device) -> torch.Tensor:
         idx = _dev_index(device)
         ws = self._cur.get(idx)
@@ -321,6 +333,13 @@ def device_cus(device: torch.device | None = None) -> int:
     return _num_cus[idx]
 
 
+def _int_tuple(values) -> tuple:
+    """The values as a tuple of Python ints (a list of ints, the usual case,
+    without a pass over it in Python)."""
+    t = tuple(values)
+    return t if set(map(type, t)) <= {int} else tuple(int(x) for x in t)
+
+
 def choose_partition_size(seq_lens_host, num_kv_heads: int, num_cus: int,
                           merge_tokens: int = 256, wg_tokens: int = 96) -> int:
     """Split-K mode for known sequence lengths: a partition size in tokens, or
@@ -341,8 +360,7 @@ def choose_partition_size(seq_lens_host, num_kv_heads: int, num_cus: int,
     the balanced split must win by 3 % to be chosen.  Memoised per length
     tuple (the same step is decoded by every layer).
     """
-    key = (tuple(int(x) for x in seq_lens_host), int(num_kv_heads), int(num_cus),
-           merge_tokens, wg_tokens)
+    key = (_int_tuple(seq_lens_host), int(num_kv_heads), int(num_cus), merge_tokens, wg_tokens)
     hit = _partition_cache.get(key)
     if hit is not None:
         return hit
@@ -388,6 +406,15 @@ def choose_partition_size(seq_lens_host, num_kv_heads: int, num_cus: int,
 _partition_cache: dict = {}
 
 
+def _decode_partition(query: torch.Tensor, num_kv_heads: int, seq_lens_host, shared: bool) -> int:
+    """The split-K mode of a decode from its host lengths."""
+    # Groups of more than 16 query heads run one workgroup per chunk of at most
+    # 16 heads: the cost model counts those chunks as kv heads.
+    chunks = -(-(query.shape[1] // num_kv_heads) // 16)
+    part = choose_partition_size(seq_lens_host, num_kv_heads * chunks, device_cus(query.device))
+    return PARTITION_BALANCED_SHARED if shared and part == PARTITION_BALANCED else part
+
+
 def paged_decode(query: torch.Tensor, key_cache: torch.Tensor, value_cache: torch.Tensor,
                  block_table: torch.Tensor, seq_lens: torch.Tensor, *, scale: float,
                  max_seq_len: int, layout: str = "kernel", output: torch.Tensor | None = None,
@@ -409,6 +436,22 @@ def paged_decode(query: torch.Tensor, key_cache: torch.Tensor, value_cache: torc
     half-size workgroups, four per CU's worth of the split, that share CUs
     with the other kernel.
     """
+    if query.is_cuda and output is not None and layout in _IS_VLLM and key_cache.dim() == 4 \
+            and query.dim() == 3:
+        part = partition_size
+        if part == 0 and seq_lens_host is not None:
+            part = _decode_partition(query, key_cache.shape[2 if layout == "vllm" else 1],
+                                     seq_lens_host, shared)
+        args = (query, key_cache, value_cache, block_table, seq_lens, output, new_keys, new_values,
+                _IS_VLLM[layout], scale, max_seq_len, part)
+        handle, native = _lib.stream_handle(stream), _lib.host().decode
+        ws = workspace if workspace is not None else _decode_ws.current(query.device)
+        done = native(*args, ws, handle)
+        if done is True:
+            return output
+        if done and workspace is None and native(
+                *args, decode_workspace(done, query.device), handle) is True:
+            return output
     _require_gpu(query, key_cache, value_cache, block_table, seq_lens, output, new_keys, new_values)
     dt = _attn_dtype(query=query, key_cache=key_cache, value_cache=value_cache, output=output,
                      new_keys=new_keys, new_values=new_values)
@@ -423,14 +466,9 @@ def paged_decode(query: torch.Tensor, key_cache: torch.Tensor, value_cache: torc
     if new_keys is not None and new_keys.stride() != new_values.stride():
         raise ValueError("new_keys and new_values must share strides")
     if partition_size == 0 and seq_lens_host is not None:
-        kvh = key_cache.shape[1] if layout == "kernel" else key_cache.shape[2]
-        # Groups of more than 16 query heads run one workgroup per chunk of
-        # at most 16 heads: the cost model counts those chunks as kv heads.
-        chunks = -(-(query.shape[1] // kvh) // 16)
-        partition_size = choose_partition_size(seq_lens_host, kvh * chunks,
-                                               device_cus(query.device))
-        if shared and partition_size == PARTITION_BALANCED:
-            partition_size = PARTITION_BALANCED_SHARED
+        partition_size = _decode_partition(
+            query, key_cache.shape[1] if layout == "kernel" else key_cache.shape[2],
+            seq_lens_host, shared)
     p = make_params(key_cache=key_cache, value_cache=value_cache, layout=layout,
                     num_query_heads=query.shape[1], scale=scale, num_seqs=num_seqs,
                     max_seq_len=max_seq_len, max_blocks_per_seq=block_table.shape[1],
@@ -586,6 +624,11 @@ def paged_prefill(query: torch.Tensor, key_cache: torch.Tensor, value_cache: tor
     max_seq_len bounds the contexts (default: the block table's capacity) and
     sizes the partials' workspace (grow-only scratch unless given).
     """
+    if query.is_cuda and output is not None and not split_keys and layout in _IS_VLLM \
+            and _lib.host().prefill(query, key_cache, value_cache, block_table, token_to_seq,
+                                    positions, output, _IS_VLLM[layout], scale,
+                                    _lib.stream_handle(stream)) is True:
+        return output
     _require_gpu(query, key_cache, value_cache, block_table, token_to_seq, positions, output)
     dt = _attn_dtype(query=query, key_cache=key_cache, value_cache=value_cache, output=output)
     if block_table.dtype != torch.int32 or block_table.dim() != 2 or not block_table.is_contiguous():
@@ -623,46 +666,28 @@ def paged_prefill(query: torch.Tensor, key_cache: torch.Tensor, value_cache: tor
     return output
 
 
-def attention_no_cache(query: torch.Tensor, key: torch.Tensor, value: torch.Tensor,
-                       query_start_loc: torch.Tensor, output: torch.Tensor, *, scale: float,
-                       max_seq_len: int, causal: bool) -> torch.Tensor:
-    """Attention inside each sequence's own tokens, K and V read in place
-    (vaa_attention_no_cache), on the current stream.
+def try_attention_no_cache(query: torch.Tensor, key: torch.Tensor, value: torch.Tensor,
+                           output: torch.Tensor, query_start_loc: torch.Tensor, *,
+                           num_tokens: int, num_seqs: int, head_size: int, scale: float,
+                           max_seq_len: int, causal: bool) -> bool:
+    """Attention of the first num_tokens tokens inside their own sequences, K
+    and V read in place (vaa_attention_no_cache), on the current stream.
 
-    query/output [T, H, D], key/value [T, KV, D], all fp16 or all bf16, with a
-    contiguous last dim and 16-byte aligned rows; query_start_loc int32
-    [num_seqs + 1] on the device; max_seq_len bounds the sequences' lengths.
-    output must not overlap key or value.
-    """
-    _require_gpu(query, key, value, query_start_loc, output)
-    dt = _attn_dtype(query=query, key=key, value=value, output=output)
-    if query_start_loc.dtype != torch.int32 or not query_start_loc.is_contiguous() \
-            or query_start_loc.numel() < 1:
-        raise ValueError("query_start_loc must be a contiguous int32 [num_seqs + 1] tensor")
-    for t, n in ((query, "query"), (key, "key"), (value, "value"), (output, "output")):
-        if t.dim() != 3 or t.stride(2) != 1:
-            raise ValueError(f"{n} must be [tokens, heads, head_size] with contiguous last dim")
-    T, H, D = query.shape
-    KV = key.shape[1]
-    if key.shape != value.shape or key.shape[0] < T or key.shape[2] != D \
-            or output.shape != query.shape or KV == 0 or H % KV:
-        raise ValueError(f"shapes differ: query {tuple(query.shape)}, key {tuple(key.shape)}, "
-                         f"value {tuple(value.shape)}, output {tuple(output.shape)}")
-    p = _lib.VaaAttnParams()
-    p.dtype = ATTN_DTYPES[dt]
-    p.scale = float(scale)
-    p.num_seqs, p.max_seq_len = query_start_loc.numel() - 1, int(max_seq_len)
-    p.head_size, p.num_kv_heads, p.num_query_heads, p.queries_per_kv = D, KV, H, H // KV
-    p.k_stride_token, p.k_stride_head = key.stride(0), key.stride(1)
-    p.v_stride_token, p.v_stride_head = value.stride(0), value.stride(1)
-    p.q_stride_token, p.q_stride_head = query.stride(0), query.stride(1)
-    p.o_stride_token, p.o_stride_head = output.stride(0), output.stride(1)
-    nbytes = _lib.load().vaa_attention_no_cache_workspace_size(p.num_seqs, T, p.max_seq_len)
-    ws = torch.empty(nbytes, dtype=torch.uint8, device=query.device)
-    _lib.call("vaa_attention_no_cache", ctypes.byref(p), query.data_ptr(), key.data_ptr(),
-              value.data_ptr(), query_start_loc.data_ptr(), output.data_ptr(), T, int(causal),
-              ws.data_ptr(), ws.numel(), _lib.stream_handle())
-    return output
+    Takes [T, H, D] query and output and [T, KV, D] key and value with 16-byte
+    aligned rows, one 16-bit type, key and value of one shape and stride, an
+    output that overlaps neither, and query_start_loc int32 [num_seqs + 1] on
+    their device, which the caller knows to run from 0 to num_tokens without
+    decreasing; max_seq_len is the longest sequence.  False, with nothing
+    done, for anything else."""
+    if not query.is_cuda:
+        return False
+    native, handle = _lib.host().no_cache, _lib.stream_handle()
+    args = (query, key, value, output, query_start_loc, num_tokens, num_seqs, head_size, scale,
+            max_seq_len, causal)
+    done = native(*args, None, handle)
+    if done is not True and done:
+        done = native(*args, torch.empty(done, dtype=torch.uint8, device=query.device), handle)
+    return done is True
 
 
 def build_token_index(query_start_loc: torch.Tensor, seq_lens: torch.Tensor, num_tokens: int,
@@ -710,6 +735,9 @@ def rms_norm(x: torch.Tensor, weight: torch.Tensor, eps: float, *,
              stream=None) -> torch.Tensor:
     """round16(x * rsqrt(mean(x^2) + eps) * w) [+ residual], rows of a 2-D view;
     fp16 or bf16."""
+    if x.is_cuda and out is not None and _lib.host().norm(
+            x, weight, residual, out, eps, _lib.stream_handle(stream), False) is True:
+        return out
     _require_gpu(x, weight, residual, out)
     dt = _layer_dtype(x=x, weight=weight, residual=residual, out=out)
     if x.dim() != 2 or x.stride(1) != 1:
@@ -734,6 +762,9 @@ def add_rms_norm(x: torch.Tensor, residual: torch.Tensor, weight: torch.Tensor, 
     One pass for the reference layer's residual add, copy and norm
     (runner.py:1107-1130).  out may be x itself (the reference's in-place
     hidden buffer) but not residual.  fp16 or bf16."""
+    if x.is_cuda and out is not None and _lib.host().norm(
+            x, weight, residual, out, eps, _lib.stream_handle(stream), True) is True:
+        return out
     _require_gpu(x, residual, weight, out)
     dt = _layer_dtype(x=x, residual=residual, weight=weight, out=out)
     if x.dim() != 2 or x.stride(1) != 1:
@@ -812,6 +843,11 @@ def qkv_epilogue(query: torch.Tensor, key: torch.Tensor, value: torch.Tensor,
     run in turn (engine/ops/qkv.py:391-416, elementwise.py:185-239,
     kv_write.py:118-156).
     """
+    if query.is_cuda and layout in _IS_VLLM and _lib.host().epilogue(
+            query, key, value, positions, cos_cache, sin_cache, slot_mapping, key_cache,
+            value_cache, bias, rotary_dim or query.shape[-1], _IS_VLLM[layout],
+            _lib.stream_handle(stream)) is True:
+        return
     _require_gpu(query, key, value, positions, cos_cache, sin_cache, slot_mapping, key_cache,
                  value_cache, bias)
     _attn_dtype(query=query, key=key, value=value, key_cache=key_cache,
@@ -870,6 +906,14 @@ def topk_logits(logits: torch.Tensor, k: int, *, indices: torch.Tensor | None = 
     EngineTopK, engine/ops/topk.py:40-412).  logits: [T, V] fp16 or bf16 with
     a contiguous last dim.  Without `workspace` a grow-only per-device buffer
     is used, safe for calls ordered on one stream."""
+    if logits.is_cuda and indices is not None and values is not None:
+        handle, native = _lib.stream_handle(stream), _lib.host().topk
+        ws = workspace if workspace is not None else _topk_ws.current(logits.device)
+        done = native(logits, k, indices, values, ws, handle)
+        if done is not True and done and workspace is None:
+            done = native(logits, k, indices, values, _topk_ws.get(done, logits.device), handle)
+        if done is True:
+            return indices, values
     _require_gpu(logits, indices, values, workspace)
     if logits.dtype not in ATTN_DTYPES:
         raise ValueError(f"logits must be float16 or bfloat16, got {logits.dtype}")
@@ -936,6 +980,9 @@ def silu_mul(gate: torch.Tensor, up: torch.Tensor, out: torch.Tensor | None = No
              stream=None) -> torch.Tensor:
     """out = round16(silu(float(gate)) * float(up)); 1-D or row-strided 2-D views;
     fp16 or bf16."""
+    if gate.is_cuda and out is not None and _lib.host().silu(
+            gate, up, out, _lib.stream_handle(stream)) is True:
+        return out
     _require_gpu(gate, up, out)
     dt = _layer_dtype(gate=gate, up=up, out=out)
     if gate.shape != up.shape:
@@ -971,6 +1018,14 @@ def gate_up_silu(x: torch.Tensor, gate_weight: torch.Tensor,
     engine/ops/mlp.py:300-330), or, with up_weight None, gate_weight is the
     fused gate_up_proj [2I, H] (gate rows first, mlp.py:267-296).  H must be a
     multiple of 64 and I of 128.  fp16 or bf16."""
+    if x.is_cuda and out is not None:
+        handle, native = _lib.stream_handle(stream), _lib.host().gate_up
+        done = native(x, gate_weight, up_weight, out, None, handle)
+        if done is not True and done:
+            done = native(x, gate_weight, up_weight, out, _stream_scratch(done, x.device, stream),
+                          handle)
+        if done is True:
+            return out
     _require_gpu(x, gate_weight, up_weight, out)
     if up_weight is None:
         if gate_weight.dim() != 2 or gate_weight.shape[0] % 2:
@@ -1044,10 +1099,25 @@ def linear_small_pays(x: torch.Tensor, weight: torch.Tensor) -> bool:
             or weight.numel() >= _LINEAR_SMALL_MIN_WEIGHTS)
 
 
+def try_linear_small(x: torch.Tensor, weight: torch.Tensor, out: torch.Tensor,
+                     stream=None) -> bool:
+    """linear_small where it takes the tensors (linear_small_ok); False, with
+    nothing done, where it does not."""
+    if not x.is_cuda:
+        return False
+    handle, native = _lib.stream_handle(stream), _lib.host().linear
+    done = native(x, weight, out, None, handle)
+    if done is not True and done:
+        done = native(x, weight, out, _stream_scratch(done, x.device, stream), handle)
+    return done is True
+
+
 def linear_small(x: torch.Tensor, weight: torch.Tensor, out: torch.Tensor,
                  stream=None) -> torch.Tensor:
     """out = round16(x @ weight.T) for few tokens (vaa_linear_small), on
     tensors that linear_small_ok accepts."""
+    if try_linear_small(x, weight, out, stream):
+        return out
     if not linear_small_ok(x, weight, out):
         raise ValueError(f"linear_small: x {tuple(x.shape)}, weight {tuple(weight.shape)}, out "
                          f"{tuple(out.shape)}: not a supported shape, type or layout")
