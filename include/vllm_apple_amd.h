@@ -446,20 +446,20 @@ int vaa_gate_up_silu_split(const uint16_t* x, int64_t x_stride, const uint16_t* 
                            size_t workspace_bytes, void* stream);
 
 /*
- * Plain product of few tokens with a weight matrix, the down projection of a
- * decode batch's MLP (vllm_apple/engine/ops/mlp.py:332-384):
+ * Plain product of up to 1024 tokens with a weight matrix, the down projection
+ * of the MLP (vllm_apple/engine/ops/mlp.py:332-384):
  *   output[t, n] = round16(sum_k x[t, k] w[n, k]),  fp32 accumulation,
- * for num_tokens <= 128, in_features a multiple of 64 and out_features of 128
- * (VAA_ERR_UNSUPPORTED otherwise); strides in elements, multiples of 8, 16-byte
+ * in_features a multiple of 64, out_features of 128 (of 256 above 128 tokens);
+ * VAA_ERR_UNSUPPORTED otherwise; strides in elements, multiples of 8, 16-byte
  * aligned tensors.  The contraction is split over workgroups; workspace:
- * vaa_linear_small_workspace_size bytes (0: shape not supported), 16-byte
- * aligned, not shared by calls that can run concurrently.
+ * vaa_linear_workspace_size bytes (0: shape not supported; at most 64 MiB),
+ * 16-byte aligned, not shared by calls that can run concurrently.
  */
-size_t vaa_linear_small_workspace_size(int num_tokens, int in_features, int out_features);
-int vaa_linear_small(const uint16_t* x, int64_t x_stride, const uint16_t* w, int64_t w_stride,
-                     uint16_t* output, int64_t output_stride, int num_tokens, int in_features,
-                     int out_features, int dtype, void* workspace, size_t workspace_bytes,
-                     void* stream);
+size_t vaa_linear_workspace_size(int num_tokens, int in_features, int out_features);
+int vaa_linear(const uint16_t* x, int64_t x_stride, const uint16_t* w, int64_t w_stride,
+               uint16_t* output, int64_t output_stride, int num_tokens, int in_features,
+               int out_features, int dtype, void* workspace, size_t workspace_bytes,
+               void* stream);
 
 /* ------------------------------------------------------------------------
  * Fused QKV epilogue

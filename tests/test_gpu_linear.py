@@ -1,4 +1,4 @@
-"""The few-token product (vaa_linear_small) and the split gate/up product
+"""The plain product (vaa_linear) and the split gate/up product
 (vaa_gate_up_silu_split) against fp64 products of the same 16-bit values:
 token counts at the edges of the 32-token blocks, one to many splits with short
 last splits, row strides that are and are not multiples of 4 KB (which walk
@@ -23,7 +23,7 @@ def _check(out, ref, dtype, what):
 @pytest.mark.parametrize("T", [1, 31, 32, 33, 64, 65, 96, 97, 127, 128])
 @pytest.mark.parametrize("K,N", [(64, 128), (1024, 256), (2048 + 64, 384), (8192, 128)])
 @pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
-def test_linear_small(gpu, T, K, N, dtype):
+def test_linear_few_tokens(gpu, T, K, N, dtype):
     from vllm_apple_amd import kernels
 
     g = torch.Generator().manual_seed(T + K + N)
@@ -31,10 +31,35 @@ def test_linear_small(gpu, T, K, N, dtype):
     w = (torch.randn(N, K, generator=g) / K ** 0.5).to(dtype)
     buf = torch.full((T + 1, N + 8), 7.0, dtype=dtype, device="cuda")
     out = buf[:T, :N]
-    kernels.linear_small(x.cuda(), w.cuda(), out)
+    kernels.linear(x.cuda(), w.cuda(), out)
     torch.cuda.synchronize()
     _check(out, (x.double() @ w.double().T).numpy(), dtype, f"linear {T}x{K}x{N}")
     assert bool((buf[T:] == 7.0).all()) and bool((buf[:, N:] == 7.0).all()), "padding written"
+
+
+@pytest.mark.parametrize("T", [129, 192, 193, 257, 384, 513, 1024])
+@pytest.mark.parametrize("K,N", [(64, 256), (576, 512), (8192, 256), (2048, 2048)])
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+def test_linear_wide(gpu, T, K, N, dtype):
+    """Token counts at the edges of the 128-, 192- and 256-token tiles, one to
+    many splits."""
+    test_linear_few_tokens(gpu, T, K, N, dtype)
+
+
+@pytest.mark.parametrize("T,I", [(300, 14336), (192, 14336), (384, 32768), (150, 38 * 128)])
+def test_gate_up_silu_tile_heights(gpu, T, I):
+    """Batches that pick 2, 3 and 4 token blocks per wave (by the columns), on
+    rows and columns of the first, a middle and the last tiles."""
+    from vllm_apple_amd import kernels
+
+    H = 192
+    g = torch.Generator(device="cuda").manual_seed(T)
+    x = torch.randn(T, H, generator=g, device="cuda").half()
+    w = (torch.randn(2 * I, H, generator=g, device="cuda") / H ** 0.5).half()
+    out = kernels.gate_up_silu(x, w).double()
+    gu = x.double() @ w.double().T
+    ref = torch.nn.functional.silu(gu[:, :I]) * gu[:, I:]
+    assert bool(((out - ref).abs() <= 2e-3 + 1e-2 * ref.abs()).all())
 
 
 @pytest.mark.parametrize("T", [1, 24, 33, 64, 100, 128])
@@ -51,7 +76,7 @@ def test_gate_up_silu_split(gpu, T, H, I):
     assert_close(host(out), olo.gate_up_silu(host(x), host(w)), what=f"gate_up {T}x{H}x{I}")
 
 
-def test_linear_small_strided_rows_and_refusals(gpu):
+def test_linear_strided_rows_and_refusals(gpu):
     from vllm_apple_amd import kernels
 
     g = torch.Generator().manual_seed(4)
@@ -59,13 +84,15 @@ def test_linear_small_strided_rows_and_refusals(gpu):
     wb = (torch.randn(256, 640, generator=g) / 23).half()
     x, w = xb.cuda()[:, 64:576], wb.cuda()[:, 64:576]
     out = torch.empty(40, 256, dtype=torch.float16, device="cuda")
-    kernels.linear_small(x, w, out)
+    kernels.linear(x, w, out)
     torch.cuda.synchronize()
     assert_close(host(out), (xb[:, 64:].double() @ wb[:, 64:576].double().T).numpy(), what="strided")
-    z = torch.zeros(129, 512, dtype=torch.float16, device="cuda")
-    assert not kernels.linear_small_ok(z, w, torch.empty(129, 256, dtype=z.dtype, device="cuda"))
-    assert not kernels.linear_small_ok(xb.cuda()[:, 1:513], w, out)      # unaligned rows
-    assert not kernels.linear_small_ok(x, w[:200], out[:, :200])         # 200 columns
-    assert not kernels.linear_small_ok(x.bfloat16(), w, out)             # two types
+    z = torch.zeros(1025, 512, dtype=torch.float16, device="cuda")
+    assert not kernels.linear_ok(z, w, torch.empty(1025, 256, dtype=z.dtype, device="cuda"))
+    assert not kernels.linear_ok(z[:129], w[:128],
+                                 torch.empty(129, 128, dtype=z.dtype, device="cuda"))
+    assert not kernels.linear_ok(xb.cuda()[:, 1:513], w, out)      # unaligned rows
+    assert not kernels.linear_ok(x, w[:200], out[:, :200])         # 200 columns
+    assert not kernels.linear_ok(x.bfloat16(), w, out)             # two types
     with pytest.raises(ValueError):
-        kernels.linear_small(x, w[:200], out[:, :200])
+        kernels.linear(x, w[:200], out[:, :200])

@@ -9,12 +9,12 @@
 // accumulators, so neither intermediate is written or read back.
 //
 // Tiling (one 4-wave workgroup per CU, all 160 KB of LDS):
-//   workgroup = 256 tokens x 128 output columns: a 256 x 256 product of the
-//               token rows of x against 256 weight rows (128 gate, then the
-//               128 up rows of the same columns);
-//   wave w    = tokens 128*(w/2) .. +128 x columns 64*(w%2) .. +64, a 4 x 4
+//   workgroup = 64 NB tokens (NB = 2, 3 or 4, wide_blocks) x 128 output columns: a
+//               64 NB x 256 product of the token rows of x against 256 weight
+//               rows (128 gate, then the 128 up rows of the same columns);
+//   wave w    = tokens 32 NB*(w/2) .. +32 NB x columns 64*(w%2) .. +64, a 4 x NB
 //               grid of 32x32 MFMA tiles (two gate and two up row blocks by
-//               four token blocks), so the gate and up values of one output
+//               NB token blocks), so the gate and up values of one output
 //               sit in the same lane, in the same accumulator position;
 //   k-step    = 64 hidden elements.  The product is computed transposed,
 //               W x^T, with v_mfma_f32_32x32x16: the A operand is 8 weights of
@@ -30,6 +30,13 @@
 // M0).  The loads are inline asm, so the compiler does not track them (it
 // would otherwise wait for every one of them before any LDS read); the
 // kernel orders each LDS read behind its own counted vmcnt wait and barrier.
+// What bounds a step is the LDS port beside the MFMAs: the operand reads and
+// the direct loads' writes take 1536 of its cycles against 2048 of MFMA at NB = 4
+// and 1344 against 1536 at NB = 3.
+//
+// The same kernel runs 256 rows of a plain product (kPart: the down projection of
+// 129 to 1024 tokens) with the k-steps split so that one workgroup runs on every
+// CU; the fp32 partials are summed by wide_sum_kernel.
 // Weight tiles go through a ring of three 32 KB stages and activation tiles
 // through two, all of LDS: during step k the wave issues the activation
 // loads of step k + 1 and then the weight loads of step k + 2, one load
@@ -50,7 +57,6 @@
 namespace vaa {
 namespace {
 
-constexpr int kGT = 256;                         // tokens per workgroup
 constexpr int kGI = 128;                         // output columns per workgroup
 constexpr int kGK = 64;                          // hidden elements per k-step
 constexpr int kGWaves = 4;
@@ -125,10 +131,16 @@ struct GluArgs {
 // go; the barrier that follows covers the other waves'.
 __device__ __forceinline__ void glu_wait_tiles() { __builtin_amdgcn_s_waitcnt(0x0078); }
 
-template <typename T, bool kStreamW>
+// NB: 32-token blocks per wave (the workgroup's tile is 64 NB tokens).  kPart:
+// the two matrices are 256 rows of one plain product, the k-steps are split over
+// gridDim.y and the fp32 sums go to a.part.
+template <typename T, bool kStreamW, int NB, bool kPart>
 __global__ void __launch_bounds__(kGThreads) __attribute__((amdgpu_waves_per_eu(1, 1)))
 gate_up_silu_kernel(GluArgs a) {
-  __shared__ __align__(16) char smem[5 * kGTileB];  // W stages 0-2, x stages 0-1
+  constexpr int kTT = 64 * NB;             // tokens per workgroup
+  constexpr int kXTile = kTT * kGRowB;     // activation tile, bytes
+  constexpr int kXLoads = 2 * NB;          // direct loads per wave per activation tile
+  __shared__ __align__(16) char smem[3 * kGTileB + 2 * kXTile];  // W stages 0-2, x stages 0-1
   char* const w0 = smem;
   char* const w1 = smem + kGTileB;
   const uint32_t lds0 = __builtin_amdgcn_readfirstlane(
@@ -138,7 +150,7 @@ gate_up_silu_kernel(GluArgs a) {
   const int logical = (static_cast<int>(blockIdx.x) % kGXcds) * per_xcd +
                       static_cast<int>(blockIdx.x) / kGXcds;
   if (logical >= a.tiles) return;
-  const int t0 = (logical % a.t_tiles) * kGT;
+  const int t0 = (logical % a.t_tiles) * kTT;
   const int i0 = (logical / a.t_tiles) * kGI;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int lane = threadIdx.x & 63;
@@ -150,20 +162,20 @@ gate_up_silu_kernel(GluArgs a) {
   // (waves 2 and 3) the up rows of the same columns, so each wave reads one
   // weight matrix; its load q is 8 rows further on.  Every access stays
   // inside its resource's range (rows of x are clamped to num_tokens - 1).
-  const char* wbase = (wave < 2 ? a.wg : a.wu) + static_cast<int64_t>(i0) * a.ws;
+  const char* wbase = (wave < 2 ? a.wg : a.wu) + (logical / a.t_tiles) * a.w_tile;
   const i32x4v wrs = buffer_rsrc(wbase, static_cast<int>(kGI * a.ws));
   const i32x4v xrs = buffer_rsrc(a.x, static_cast<int>(a.num_tokens * a.xs));
   const int rw = 8 * (wave & 1) * kGLoads + (lane >> 3);  // weight row of load 0, mod 128
   const int lc = (lane & 7) ^ (rw & 7);                    // a wave's rows agree mod 8
   const int woff = rw * static_cast<int>(a.ws) + lc * 16;
   const int wstep = 8 * static_cast<int>(a.ws);
-  int xoff[kGLoads];
+  int xoff[kXLoads];
 #pragma unroll
-  for (int q = 0; q < kGLoads; ++q) {
-    const int R = 8 * (wave * kGLoads + q) + (lane >> 3);
+  for (int q = 0; q < kXLoads; ++q) {
+    const int R = 8 * (wave * kXLoads + q) + (lane >> 3);
     xoff[q] = min(t0 + R, a.num_tokens - 1) * static_cast<int>(a.xs) + lc * 16;
   }
-  const int dst0 = 1024 * wave * kGLoads;
+  const int dst0 = 1024 * wave * kGLoads, xdst0 = 1024 * wave * kXLoads;
 
   // Operand reads: row l % 32 of a 32-row block, logical chunk 4 (l / 32) + s.
   const int l32 = lane & 31, hb = lane >> 5;
@@ -173,99 +185,125 @@ gate_up_silu_kernel(GluArgs a) {
   const int wi = wave & 1, wt = wave >> 1;
   // Weight row blocks: gate 64wi, 64wi + 32; up 128 + 64wi, 128 + 64wi + 32.
   const int wrow[4] = {64 * wi, 64 * wi + 32, kGI + 64 * wi, kGI + 64 * wi + 32};
-  const int xrow0 = 128 * wt;
+  const int xrow0 = 32 * NB * wt;
 
-  f32x16 acc[4][4];
+  f32x16 acc[4][NB];
 #pragma unroll
   for (int f = 0; f < 4; ++f)
 #pragma unroll
-    for (int c = 0; c < 4; ++c)
+    for (int c = 0; c < NB; ++c)
 #pragma unroll
       for (int r = 0; r < 16; ++r) acc[f][c][r] = 0.f;
 
-  // Direct load L of a step: 0-7 the activation tile of k-step kx into the
-  // LDS address xst, 8-15 the weight tile of k-step kw into wst.
+  // Direct load L of a step: the first kXLoads move the activation tile of
+  // k-step kx into the LDS address xst, the next eight the weight tile of
+  // k-step kw into wst.
   auto load1 = [&](int L, int kbx, int kbw, uint32_t xst, uint32_t wst) {
-    if (L < kGLoads)
-      dma16(xrs, xoff[L], kbx, xst + dst0 + 1024 * L);
+    if (L < kXLoads)
+      dma16(xrs, xoff[L], kbx, xst + xdst0 + 1024 * L);
     else if constexpr (kStreamW)
-      dma16_stream(wrs, woff, kbw + (L - kGLoads) * wstep, wst + dst0 + 1024 * (L - kGLoads));
+      dma16_stream(wrs, woff, kbw + (L - kXLoads) * wstep, wst + dst0 + 1024 * (L - kXLoads));
     else
-      dma16(wrs, woff, kbw + (L - kGLoads) * wstep, wst + dst0 + 1024 * (L - kGLoads));
+      dma16(wrs, woff, kbw + (L - kXLoads) * wstep, wst + dst0 + 1024 * (L - kXLoads));
   };
-  auto frags = [&](const char* wt_, const char* xt_, int s, u32x4 (&A)[4], u32x4 (&B)[4]) {
+  auto frags = [&](const char* wt_, const char* xt_, int s, u32x4 (&A)[4], u32x4 (&B)[NB]) {
 #pragma unroll
     for (int f = 0; f < 4; ++f)
       A[f] = *reinterpret_cast<const u32x4*>(wt_ + wrow[f] * kGRowB + rd[s]);
 #pragma unroll
-    for (int c = 0; c < 4; ++c)
+    for (int c = 0; c < NB; ++c)
       B[c] = *reinterpret_cast<const u32x4*>(xt_ + (xrow0 + 32 * c) * kGRowB + rd[s]);
   };
-  auto mfmas = [&](const u32x4 (&A)[4], const u32x4 (&B)[4], bool ld, int L0, int kbx, int kbw,
+  // The 4 NB MFMAs of a sub-step, with nl direct loads from L0 on spread
+  // between them.
+  auto mfmas = [&](const u32x4 (&A)[4], const u32x4 (&B)[NB], int nl, int L0, int kbx, int kbw,
                    uint32_t xst, uint32_t wst) {
 #pragma unroll
-    for (int idx = 0; idx < 16; ++idx) {
-      const int f = idx >> 2, c = idx & 3;
+    for (int idx = 0; idx < 4 * NB; ++idx) {
+      const int f = idx / NB, c = idx % NB;
       acc[f][c] = Elem<T>::mfma32x32x16(__builtin_bit_cast(typename Elem<T>::x8, A[f]),
                                         __builtin_bit_cast(typename Elem<T>::x8, B[c]),
                                         acc[f][c]);
-      if (ld && (idx & 1)) load1(L0 + (idx >> 1), kbx, kbw, xst, wst);
+      if ((idx + 1) * nl / (4 * NB) > idx * nl / (4 * NB))
+        load1(L0 + idx * nl / (4 * NB), kbx, kbw, xst, wst);
       __builtin_amdgcn_sched_barrier(0);
     }
   };
-  const int n = a.ksteps;
+  // Steps k0 .. k0 + n - 1 of this split.
+  const int k0 = kPart ? static_cast<int>(blockIdx.y) * a.k_per : 0;
+  const int n = kPart ? min(a.ksteps - k0, a.k_per) : a.ksteps;
+  // (Starting the column tiles' steps apart, as the few-token kernel does,
+  // measured level here: other tiles' MFMAs spread the loads already.)
+  auto kstep = [&](int ks) { return (k0 + min(ks, n - 1)) * kGRowB; };
   // Step ks: weights in W stage ks % 3, activations in x stage ks % 2; it
   // loads the activations of step ks + 1 and then the weights of ks + 2.
   auto step = [&](int ks) {
     glu_wait_tiles();
     __syncthreads();
     const char* cw = smem + (ks % 3) * kGTileB;
-    const char* cx = smem + (3 + (ks & 1)) * kGTileB;
-    const uint32_t xst = lds0 + (3 + ((ks + 1) & 1)) * kGTileB;
+    const char* cx = smem + 3 * kGTileB + (ks & 1) * kXTile;
+    const uint32_t xst = lds0 + 3 * kGTileB + ((ks + 1) & 1) * kXTile;
     const uint32_t wst = lds0 + ((ks + 2) % 3) * kGTileB;
-    const int kbx = min(ks + 1, n - 1) * kGRowB;
-    const int kbw = min(ks + 2, n - 1) * kGRowB;
-    u32x4 A0[4], B0[4], A1[4], B1[4];
+    const int kbx = kstep(ks + 1);
+    const int kbw = kstep(ks + 2);
+    u32x4 A0[4], B0[NB], A1[4], B1[NB];
     frags(cw, cx, 0, A0, B0);
     frags(cw, cx, 1, A1, B1);
     __builtin_amdgcn_sched_barrier(0);
-    mfmas(A0, B0, true, 0, kbx, kbw, xst, wst);
+    mfmas(A0, B0, kXLoads, 0, kbx, kbw, xst, wst);
     frags(cw, cx, 2, A0, B0);
     __builtin_amdgcn_sched_barrier(0);
-    mfmas(A1, B1, true, 8, kbx, kbw, xst, wst);
+    mfmas(A1, B1, kGLoads, kXLoads, kbx, kbw, xst, wst);
     frags(cw, cx, 3, A1, B1);
     __builtin_amdgcn_sched_barrier(0);
-    mfmas(A0, B0, false, 0, 0, 0, 0, 0);
-    mfmas(A1, B1, false, 0, 0, 0, 0, 0);
+    mfmas(A0, B0, 0, 0, 0, 0, 0, 0);
+    mfmas(A1, B1, 0, 0, 0, 0, 0, 0);
   };
   // Prologue: weights of steps 0 and 1, activations of step 0, issued so
   // that at the top of every step the newest 8 loads are the only ones that
   // may still be in flight (the weights of the next step).
 #pragma unroll
-  for (int q = 0; q < kGLoads; ++q) dma16(wrs, woff, q * wstep, lds0 + dst0 + 1024 * q);
+  for (int q = 0; q < kGLoads; ++q)
+    dma16(wrs, woff, kstep(0) + q * wstep, lds0 + dst0 + 1024 * q);
+#pragma unroll
+  for (int q = 0; q < kXLoads; ++q)
+    dma16(xrs, xoff[q], kstep(0), lds0 + 3 * kGTileB + xdst0 + 1024 * q);
 #pragma unroll
   for (int q = 0; q < kGLoads; ++q)
-    dma16(xrs, xoff[q], 0, lds0 + 3 * kGTileB + dst0 + 1024 * q);
-#pragma unroll
-  for (int q = 0; q < kGLoads; ++q)
-    dma16(wrs, woff, min(1, n - 1) * kGRowB + q * wstep, lds0 + kGTileB + dst0 + 1024 * q);
+    dma16(wrs, woff, kstep(1) + q * wstep, lds0 + kGTileB + dst0 + 1024 * q);
   for (int ks = 0; ks < n; ++ks) step(ks);
   // Every load has landed before the workgroup ends and its LDS is released.
   __builtin_amdgcn_s_waitcnt(0x0070);
 
+  if constexpr (kPart) {
+    // The sums as the lanes hold them: [split][tile][wave][f][c][r4][lane].
+    f32x4* p = reinterpret_cast<f32x4*>(a.part) +
+               ((static_cast<int64_t>(blockIdx.y) * a.tiles + logical) * kGWaves + wave) *
+                   (4 * NB * 4 * kWave) + lane;
+#pragma unroll
+    for (int f = 0; f < 4; ++f)
+#pragma unroll
+      for (int c = 0; c < NB; ++c)
+#pragma unroll
+        for (int r4 = 0; r4 < 4; ++r4)
+          p[((f * NB + c) * 4 + r4) * kWave] =
+              f32x4{acc[f][c][4 * r4], acc[f][c][4 * r4 + 1], acc[f][c][4 * r4 + 2],
+                    acc[f][c][4 * r4 + 3]};
+    return;
+  }
   // Epilogue, staged through LDS so that the output leaves in whole rows.
   // The lane holds token xrow0 + 32c + l32 and, for row block f, columns
   // 8 (r / 4) + 4 hb + r % 4 of that block: four runs of four consecutive
   // columns.  silu(g) u is formed in registers and written as 8-byte pieces
-  // into a [256 tokens][128 columns] tile (token rows 0-127 in w0, 128-255
-  // in w1, 256 bytes each, 16-byte chunks XOR-swizzled by row & 15 so the 32
+  // into a [64 NB tokens][128 columns] tile (the first 32 NB token rows in w0,
+  // the others in w1, 256 bytes each, 16-byte chunks XOR-swizzled by row & 15 so the 32
   // token rows of one write hit distinct banks); then each row goes out as
   // sixteen 16-byte stores.
   __syncthreads();  // every wave is done with the operand tiles
   char* stage = wt == 0 ? w0 : w1;
 #pragma unroll
-  for (int c = 0; c < 4; ++c) {
-    const int row = 32 * c + l32;  // within this wave's 128 token rows
+  for (int c = 0; c < NB; ++c) {
+    const int row = 32 * c + l32;  // within this wave's 32 NB token rows
 #pragma unroll
     for (int j = 0; j < 2; ++j)
 #pragma unroll
@@ -284,15 +322,41 @@ gate_up_silu_kernel(GluArgs a) {
   const int tid = threadIdx.x;
   const int ch = tid & 15;
 #pragma unroll 4
-  for (int r0 = 0; r0 < kGT; r0 += kGThreads / 16) {
+  for (int r0 = 0; r0 < kTT; r0 += kGThreads / 16) {
     const int row = r0 + (tid >> 4);
     const int tok = t0 + row;
     if (tok < a.num_tokens) {
-      const char* src = (row < 128 ? w0 : w1) + (row & 127) * 256 + ((ch ^ (row & 15)) << 4);
+      const int in = row < 32 * NB ? row : row - 32 * NB;
+      const char* src = (row < 32 * NB ? w0 : w1) + in * 256 + ((ch ^ (in & 15)) << 4);
       *reinterpret_cast<u32x4*>(a.out + static_cast<int64_t>(tok) * a.os + 2 * (i0 + 8 * ch)) =
           *reinterpret_cast<const u32x4*>(src);
     }
   }
+}
+
+// Sums the wide kernel's split partials in a fixed order and rounds: a thread
+// owns four consecutive columns of one token, in the partials' order.
+template <typename T, int NB>
+__global__ void __launch_bounds__(256) wide_sum_kernel(GluArgs a, int splits) {
+  constexpr int kPerTile = kGWaves * 4 * NB * 4 * kWave;  // f32x4 of a tile
+  const int tile = blockIdx.x, in = blockIdx.y * 256 + threadIdx.x;
+  const int lane = in % kWave, r4 = in / kWave % 4, c = in / (4 * kWave) % NB;
+  const int f = in / (4 * kWave * NB) % 4, wave = in / (16 * kWave * NB);
+  const int tok = (tile % a.t_tiles) * 64 * NB + 32 * NB * (wave >> 1) + 32 * c + (lane & 31);
+  if (tok >= a.num_tokens) return;
+  const f32x4* p =
+      reinterpret_cast<const f32x4*>(a.part) + static_cast<int64_t>(tile) * kPerTile + in;
+  const int64_t step = static_cast<int64_t>(a.tiles) * kPerTile;
+  f32x4 s = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll 8
+  for (int z = 0; z < splits; ++z) s += p[z * step];
+  T v[4];
+#pragma unroll
+  for (int e = 0; e < 4; ++e) v[e] = Elem<T>::from_f(s[e]);
+  // Row block f of the wave: weight rows 128 (f / 2) + 64 (wave & 1) + 32 (f & 1).
+  const int64_t col = static_cast<int64_t>(tile / a.t_tiles) * 2 * kGI + kGI * (f >> 1) +
+                      64 * (wave & 1) + 32 * (f & 1) + 8 * r4 + 4 * (lane >> 5);
+  *reinterpret_cast<u32x2*>(a.out + tok * a.os + 2 * col) = __builtin_bit_cast(u32x2, v);
 }
 
 // ---------------------------------------------------------------------------
@@ -593,16 +657,107 @@ size_t split_bytes(int tiles, int splits, int num_tokens) {
          sizeof(float);
 }
 
-template <typename T>
-int launch_gate_up_silu(const GluArgs& a0, hipStream_t stream) {
-  GluArgs a = a0;
+// 32-token blocks per wave (2, 3 or 4) for a batch over `cols` column tiles: the
+// fewest rounds of one workgroup per CU (256), a round costing NB + 1/2 (of a
+// k-step's time with one block; 80 k-steps, whole rounds: NB = 2, 3, 4 take 80,
+// 107 and 141 us).  300 tokens, 4096 x 14336: 106.3 us at NB = 4, 90.8 at 3;
+// 192 tokens: 85.0, 72.2 at 2; 2104 tokens, 5120 x 32768: 1170, 1151 at 3.
+inline int wide_blocks(int num_tokens, int cols) {
+  int best = 4, cost = INT32_MAX;
+  for (int nb = 4; nb >= 2; --nb) {
+    const int64_t tiles = static_cast<int64_t>((num_tokens + 64 * nb - 1) / (64 * nb)) * cols;
+    const int c = static_cast<int>((tiles + 255) / 256) * (2 * nb + 1);
+    if (c < cost) {
+      cost = c;
+      best = nb;
+    }
+  }
+  return best;
+}
+
+template <typename T, int NB>
+int launch_gate_up_silu_nb(GluArgs a, hipStream_t stream) {
+  const int cols = a.tiles;
+  a.t_tiles = (a.num_tokens + 64 * NB - 1) / (64 * NB);
+  a.tiles = a.t_tiles * cols;
   const int grid = (a.tiles + kGXcds - 1) / kGXcds * kGXcds;
   // Weight tiles read by at most four token tiles stream with the hint.
   if (a.t_tiles <= 4)
-    hipLaunchKernelGGL((gate_up_silu_kernel<T, true>), dim3(grid), dim3(kGThreads), 0, stream, a);
+    hipLaunchKernelGGL((gate_up_silu_kernel<T, true, NB, false>), dim3(grid), dim3(kGThreads), 0,
+                       stream, a);
   else
-    hipLaunchKernelGGL((gate_up_silu_kernel<T, false>), dim3(grid), dim3(kGThreads), 0, stream, a);
+    hipLaunchKernelGGL((gate_up_silu_kernel<T, false, NB, false>), dim3(grid), dim3(kGThreads), 0,
+                       stream, a);
   return check_launch("gate_up_silu_kernel");
+}
+
+// a.tiles: column tiles.
+template <typename T>
+int launch_gate_up_silu(const GluArgs& a, hipStream_t stream) {
+  switch (wide_blocks(a.num_tokens, a.tiles)) {
+    case 2: return launch_gate_up_silu_nb<T, 2>(a, stream);
+    case 3: return launch_gate_up_silu_nb<T, 3>(a, stream);
+    default: return launch_gate_up_silu_nb<T, 4>(a, stream);
+  }
+}
+
+// How vaa_linear runs a product: on the few-token kernel (nb = 0) or the wide
+// one with nb blocks of 32 tokens per wave, over `splits` ranges of k_per steps.
+struct LinearPlan {
+  int nb, splits, k_per;
+  size_t bytes;  // workspace; 0: shape not supported
+};
+
+// The wide kernel up to kWideTokens tokens: above, the library's GEMM is ahead
+// (us, library / this: 512 tokens, 32768 x 5120 288 / 179, 14336 x 4096 88 / 69,
+// 8192 x 2048 33.5 / 29.6; 1024 tokens 393 / 316, 130 / 117, 49 / 45; 2104
+// tokens 553 / 643, 213 / 256, 83 / 88).
+constexpr int kWideTokens = 1024;
+
+LinearPlan linear_plan(int num_tokens, int ksteps, int out_features) {
+  LinearPlan best{0, 1, ksteps, 0};
+  if (num_tokens <= kSmallTokens) {
+    const int tiles = out_features / (2 * kSCols);
+    best.splits = split_plan(tiles, ksteps, &best.k_per);
+    best.bytes = split_bytes(tiles, best.splits, num_tokens);
+    return best;
+  }
+  if (num_tokens > kWideTokens || out_features % (2 * kGI) != 0) return best;
+  // One workgroup per CU as far as splits of at least kSplitMinSteps steps
+  // allow.  Cost in ns: 0.3 us (NB + 1.2) a step and the partials written and
+  // read at 6 TB/s, as measured.
+  int64_t cost = INT64_MAX;
+  for (int nb = 4; nb >= 2; --nb) {
+    const int64_t tiles = static_cast<int64_t>((num_tokens + 64 * nb - 1) / (64 * nb)) *
+                          (out_features / (2 * kGI));
+    const int64_t want = std::max<int64_t>(
+        1, std::min<int64_t>(256 / tiles, ksteps / kSplitMinSteps));
+    const int k_per = static_cast<int>((ksteps + want - 1) / want);
+    const int splits = (ksteps + k_per - 1) / k_per;
+    const int64_t bytes = tiles * splits * (64 * nb) * (2 * kGI) * 4;
+    const int64_t c = (tiles * splits + 255) / 256 * k_per * (300 * nb + 360) + bytes / 3000;
+    if (c < cost) {
+      cost = c;
+      best = LinearPlan{nb, splits, k_per, static_cast<size_t>(bytes)};
+    }
+  }
+  return best;
+}
+
+// Plain product on the wide kernel, split over `splits` ranges of k-steps.
+template <typename T, int NB>
+int launch_wide_nb(GluArgs a, int splits, hipStream_t stream) {
+  const int cols = a.tiles;
+  a.t_tiles = (a.num_tokens + 64 * NB - 1) / (64 * NB);
+  a.tiles = a.t_tiles * cols;
+  const int grid = (a.tiles + kGXcds - 1) / kGXcds * kGXcds;
+  hipLaunchKernelGGL((gate_up_silu_kernel<T, false, NB, true>), dim3(grid, splits),
+                     dim3(kGThreads), 0, stream, a);
+  const int st = check_launch("gate_up_silu_kernel");
+  if (st) return st;
+  hipLaunchKernelGGL((wide_sum_kernel<T, NB>), dim3(a.tiles, 16 * NB), dim3(256), 0, stream, a,
+                     splits);
+  return check_launch("wide_sum_kernel");
 }
 
 }  // namespace
@@ -647,16 +802,17 @@ int gate_up_silu_impl(const char* what, const uint16_t* x, int64_t x_stride,
   a.os = 2 * output_stride;
   a.num_tokens = num_tokens;
   a.ksteps = hidden_size / kGK;
-  a.t_tiles = (num_tokens + kGT - 1) / kGT;
-  const int64_t tiles = static_cast<int64_t>(a.t_tiles) * (intermediate_size / kGI);
+  a.t_tiles = 1;
+  const int64_t tiles =
+      static_cast<int64_t>((num_tokens + 63) / 64) * (intermediate_size / kGI);
   // Load offsets and buffer ranges are 31-bit: activation rows from x,
   // weight rows from the workgroup's first row.
   if (tiles > (1 << 30) || static_cast<int64_t>(num_tokens) * a.xs >= (int64_t(1) << 31) ||
       static_cast<int64_t>(kGI) * a.ws >= (int64_t(1) << 31))
     return fail(VAA_ERR_UNSUPPORTED, "%s: problem too large", what);
-  a.tiles = static_cast<int>(tiles);
+  a.tiles = intermediate_size / kGI;
   a.k_per = a.ksteps;
-  a.w_tile = kSCols * a.ws;
+  a.w_tile = (num_tokens <= kSmallTokens ? kSCols : kGI) * a.ws;
   a.part = nullptr;
   hipStream_t s = static_cast<hipStream_t>(stream);
   if (num_tokens <= kSmallTokens) {
@@ -715,31 +871,30 @@ extern "C" int vaa_gate_up_silu_split(const uint16_t* x, int64_t x_stride, const
                            workspace_bytes, stream);
 }
 
-extern "C" size_t vaa_linear_small_workspace_size(int num_tokens, int in_features,
-                                                  int out_features) {
-  if (num_tokens <= 0 || num_tokens > kSmallTokens || in_features <= 0 || in_features % kGK ||
-      out_features <= 0 || out_features % (2 * kSCols))
+extern "C" size_t vaa_linear_workspace_size(int num_tokens, int in_features, int out_features) {
+  if (num_tokens <= 0 || in_features <= 0 || in_features % kGK || out_features <= 0 ||
+      out_features % (2 * kSCols))
     return 0;
-  int k_per = 0;
-  const int tiles = out_features / (2 * kSCols);
-  return split_bytes(tiles, split_plan(tiles, in_features / kGK, &k_per), num_tokens);
+  return linear_plan(num_tokens, in_features / kGK, out_features).bytes;
 }
 
-extern "C" int vaa_linear_small(const uint16_t* x, int64_t x_stride, const uint16_t* w,
-                                int64_t w_stride, uint16_t* output, int64_t output_stride,
-                                int num_tokens, int in_features, int out_features, int dtype,
-                                void* workspace, size_t workspace_bytes, void* stream) {
-  const char* what = "vaa_linear_small";
+extern "C" int vaa_linear(const uint16_t* x, int64_t x_stride, const uint16_t* w, int64_t w_stride,
+                          uint16_t* output, int64_t output_stride, int num_tokens,
+                          int in_features, int out_features, int dtype, void* workspace,
+                          size_t workspace_bytes, void* stream) {
+  const char* what = "vaa_linear";
   if (!valid_dtype(dtype)) return fail(VAA_ERR_UNSUPPORTED, "%s: dtype=%d", what, dtype);
   if (num_tokens < 0 || in_features <= 0 || out_features <= 0)
     return fail(VAA_ERR_INVALID_ARG, "%s: num_tokens=%d in_features=%d out_features=%d", what,
                 num_tokens, in_features, out_features);
-  if (num_tokens > kSmallTokens || in_features % kGK || out_features % (2 * kSCols))
+  if (num_tokens == 0) return VAA_OK;
+  const size_t need = vaa_linear_workspace_size(num_tokens, in_features, out_features);
+  if (!need)
     return fail(VAA_ERR_UNSUPPORTED,
                 "%s: num_tokens=%d (at most %d), in_features=%d (a multiple of %d), "
-                "out_features=%d (a multiple of %d)",
-                what, num_tokens, kSmallTokens, in_features, kGK, out_features, 2 * kSCols);
-  if (num_tokens == 0) return VAA_OK;
+                "out_features=%d (a multiple of %d, of %d above %d tokens)",
+                what, num_tokens, kWideTokens, in_features, kGK, out_features, 2 * kSCols,
+                2 * kGI, kSmallTokens);
   if (!x || !w || !output) return fail(VAA_ERR_INVALID_ARG, "%s: null pointer", what);
   if (x_stride < in_features || w_stride < in_features || output_stride < out_features ||
       x_stride % 8 || w_stride % 8 || output_stride % 8)
@@ -747,28 +902,42 @@ extern "C" int vaa_linear_small(const uint16_t* x, int64_t x_stride, const uint1
                 (long long)x_stride, (long long)w_stride, (long long)output_stride);
   if (!aligned16(x) || !aligned16(w) || !aligned16(output))
     return fail(VAA_ERR_INVALID_ARG, "%s: x, weights and output must be 16-byte aligned", what);
+  const LinearPlan plan = linear_plan(num_tokens, in_features / kGK, out_features);
+  const int rows = plan.nb ? kGI : kSCols;  // weight rows of one half of a tile
   GluArgs a;
   a.x = reinterpret_cast<const char*>(x);
   a.wg = reinterpret_cast<const char*>(w);
   a.xs = 2 * x_stride;
   a.ws = 2 * w_stride;
   a.os = 2 * output_stride;
-  a.wu = a.wg + kSCols * a.ws;
-  a.w_tile = 2 * kSCols * a.ws;
+  a.wu = a.wg + rows * a.ws;
+  a.w_tile = 2 * rows * a.ws;
   a.out = reinterpret_cast<char*>(output);
   a.num_tokens = num_tokens;
   a.ksteps = in_features / kGK;
+  a.k_per = plan.k_per;
   a.t_tiles = 1;
-  a.tiles = out_features / (2 * kSCols);
-  if (num_tokens * a.xs >= (int64_t(1) << 31) || kSCols * a.ws >= (int64_t(1) << 31))
+  a.tiles = out_features / (2 * rows);
+  if (num_tokens * a.xs >= (int64_t(1) << 31) || rows * a.ws >= (int64_t(1) << 31))
     return fail(VAA_ERR_UNSUPPORTED, "%s: problem too large", what);
-  const int splits = split_plan(a.tiles, a.ksteps, &a.k_per);
-  const size_t need = split_bytes(a.tiles, splits, num_tokens);
   if (!workspace || workspace_bytes < need || !aligned16(workspace))
     return fail(VAA_ERR_WORKSPACE, "%s: workspace of %zu bytes (16-byte aligned) needed, got %zu",
                 what, need, workspace ? workspace_bytes : static_cast<size_t>(0));
   a.part = static_cast<float*>(workspace);
   hipStream_t s = static_cast<hipStream_t>(stream);
-  return dtype == VAA_DTYPE_F16 ? launch_small<f16, false>(a, splits, s)
-                                : launch_small<bf16, false>(a, splits, s);
+  const bool f = dtype == VAA_DTYPE_F16;
+  switch (plan.nb) {
+    case 0:
+      return f ? launch_small<f16, false>(a, plan.splits, s)
+               : launch_small<bf16, false>(a, plan.splits, s);
+    case 2:
+      return f ? launch_wide_nb<f16, 2>(a, plan.splits, s)
+               : launch_wide_nb<bf16, 2>(a, plan.splits, s);
+    case 3:
+      return f ? launch_wide_nb<f16, 3>(a, plan.splits, s)
+               : launch_wide_nb<bf16, 3>(a, plan.splits, s);
+    default:
+      return f ? launch_wide_nb<f16, 4>(a, plan.splits, s)
+               : launch_wide_nb<bf16, 4>(a, plan.splits, s);
+  }
 }

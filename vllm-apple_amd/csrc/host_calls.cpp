@@ -25,8 +25,8 @@ namespace {
   X(vaa_paged_attention_decode_workspace_size) X(vaa_paged_attention_prefill)             \
   X(vaa_build_token_index) X(vaa_rmsnorm) X(vaa_add_rmsnorm) X(vaa_silu_mul)              \
   X(vaa_qkv_epilogue) X(vaa_topk_logits) X(vaa_topk_workspace_size)                       \
-  X(vaa_gate_up_silu_split) X(vaa_gate_up_silu_workspace_size) X(vaa_linear_small)        \
-  X(vaa_linear_small_workspace_size) X(vaa_attention_no_cache)                            \
+  X(vaa_gate_up_silu_split) X(vaa_gate_up_silu_workspace_size) X(vaa_linear)        \
+  X(vaa_linear_workspace_size) X(vaa_attention_no_cache)                            \
   X(vaa_attention_no_cache_workspace_size)
 #define VAA_DECL(f) decltype(&::f) p_##f = nullptr;
 VAA_FUNCS(VAA_DECL)
@@ -257,7 +257,7 @@ PyObject* gate_up(const Args& a) {
                                       ws ? ws->nbytes() : 0, a.s(5)));
 }
 
-// (x, weight, out, workspace or None, stream); what linear_small_ok accepts.
+// (x, weight, out, workspace or None, stream); what linear_ok accepts.
 PyObject* linear(const Args& a) {
   const Tensor *x = a.t(0), *w = a.t(1), *o = a.t(2), *ws = a.t(3);
   if (!x || !w || !o || !none_or_ten(a.a[3])) Py_RETURN_FALSE;
@@ -265,10 +265,10 @@ PyObject* linear(const Args& a) {
   if (dt < 0 || !mat16(*x, dt) || !mat16(*w, dt) || !mat16(*o, dt)) Py_RETURN_FALSE;
   const int64_t T = x->size(0), K = x->size(1), N = w->size(0);
   if (w->size(1) != K || o->size(0) != T || o->size(1) != N) Py_RETURN_FALSE;
-  const size_t need = p_vaa_linear_small_workspace_size(T, K, N);
+  const size_t need = p_vaa_linear_workspace_size(T, K, N);
   if (!need) Py_RETURN_FALSE;
   if (!ws || !on_gpu(*ws) || ws->nbytes() < need) return PyLong_FromSize_t(need);
-  return yes(p_vaa_linear_small(p16(*x), x->stride(0), p16(*w), w->stride(0), p16(*o),
+  return yes(p_vaa_linear(p16(*x), x->stride(0), p16(*w), w->stride(0), p16(*o),
                                 o->stride(0), T, K, N, dt, ptr(*ws), ws->nbytes(), a.s(4)));
 }
 

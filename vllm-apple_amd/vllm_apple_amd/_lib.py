@@ -113,8 +113,8 @@ SIGNATURES = {
     "vaa_gate_up_silu_workspace_size": (ctypes.c_size_t, [_I, _I, _I]),
     "vaa_gate_up_silu_split": (_I, [_P, _I64, _P, _P, _I64, _P, _I64, _I, _I, _I, _I, _P,
                                     ctypes.c_size_t, _P]),
-    "vaa_linear_small_workspace_size": (ctypes.c_size_t, [_I, _I, _I]),
-    "vaa_linear_small": (_I, [_P, _I64, _P, _I64, _P, _I64, _I, _I, _I, _I, _P, ctypes.c_size_t,
+    "vaa_linear_workspace_size": (ctypes.c_size_t, [_I, _I, _I]),
+    "vaa_linear": (_I, [_P, _I64, _P, _I64, _P, _I64, _I, _I, _I, _I, _P, ctypes.c_size_t,
                               _P]),
     "vaa_topk_workspace_size": (_I, [_I, _I, _I, _P]),
     "vaa_topk_logits": (_I, [_P, _I, _I, _I64, _I, _P, _P, _I64, _P, ctypes.c_size_t, _P]),

@@ -5,8 +5,8 @@ down_proj(silu(gate_proj(x)) * up_proj(x)).  The reference runs the gate and
 up GEMMs into two [T, I] intermediates and a silu_mul pass over them; here
 the first half is one MFMA kernel with the SwiGLU epilogue
 (kernels.gate_up_silu), so only the activated [T, I] intermediate exists.  The
-down projection of few tokens (kernels.linear_small_pays) streams its weights
-through kernels.linear_small; otherwise it is a plain library GEMM (torch.matmul on the
+down projection of up to 1024 tokens runs on kernels.linear where that pays
+(kernels.linear_pays); otherwise it is a plain library GEMM (torch.matmul on the
 step's stream).  Weights keep the reference's layouts: gate_proj / up_proj [I, H]
 or the fused gate_up_proj [2I, H] (gate rows first), down_proj [H, I].
 
@@ -175,8 +175,8 @@ class EngineMLP:
                 torch.matmul(x, self._gate_proj.t(), out=gu[:, :I])
                 torch.matmul(x, self._up_proj.t(), out=gu[:, I:])
             kernels.silu_mul(gu[:, :I], gu[:, I:], out=act, stream=s)
-        if not (kernels.linear_small_pays(act, self._down_proj)
-                and kernels.try_linear_small(act, self._down_proj, out, stream=s)):
+        if not (kernels.linear_pays(act, self._down_proj)
+                and kernels.try_linear(act, self._down_proj, out, stream=s)):
             torch.matmul(act, self._down_proj.t(), out=out)
 
     def get_intermediate_size(self, num_tokens: int) -> int:

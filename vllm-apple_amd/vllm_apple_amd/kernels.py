@@ -1066,42 +1066,44 @@ def _stream_scratch(nbytes: int, device: torch.device, stream) -> torch.Tensor |
         return torch.empty(nbytes, dtype=torch.uint8, device=device)
 
 
-# The few-token product's largest batch (vaa_linear_small).
-LINEAR_SMALL_MAX_TOKENS = 128
+# The plain product's largest batches (vaa_linear): over any multiple of 128
+# output features, and over multiples of 256.
+LINEAR_MAX_TOKENS = 128
+LINEAR_WIDE_MAX_TOKENS = 1024
 
 
-def linear_small_ok(x: torch.Tensor, weight: torch.Tensor, out: torch.Tensor) -> bool:
-    """Whether linear_small takes these: 1 to 128 tokens, features in multiples
-    of 64 (in) and 128 (out), one 16-bit type and 16-byte aligned rows on the
-    GPU."""
+def linear_ok(x: torch.Tensor, weight: torch.Tensor, out: torch.Tensor) -> bool:
+    """Whether linear takes these: 1 to 1024 tokens, input features in multiples
+    of 64 and output features of 128 (of 256 above 128 tokens), one 16-bit
+    type and 16-byte aligned rows on the GPU."""
     if x.dim() != 2 or weight.dim() != 2 or out.dim() != 2:
         return False
     (t, k), n = x.shape, weight.shape[0]
-    return (0 < t <= LINEAR_SMALL_MAX_TOKENS and k > 0 and k % 64 == 0 and n > 0 and n % 128 == 0
+    limit = LINEAR_MAX_TOKENS if n % 256 else LINEAR_WIDE_MAX_TOKENS
+    return (0 < t <= limit and k > 0 and k % 64 == 0 and n > 0 and n % 128 == 0
             and weight.shape[1] == k and tuple(out.shape) == (t, n)
             and x.dtype in ATTN_DTYPES and x.dtype == weight.dtype == out.dtype
             and x.device == weight.device == out.device and x.device.type == "cuda"
             and all(a.stride(1) == 1 and a.stride(0) % 8 == 0 and a.data_ptr() % 16 == 0
-                    and a.shape[1] <= a.stride(0) < 1 << 23 for a in (x, weight, out)))
+                    and a.shape[1] <= a.stride(0) < 1 << 20 for a in (x, weight, out)))
 
 
-# Few-token products that linear_small runs faster than the library's GEMM:
-# up to 64 tokens over any weights, up to 128 over weights of at least 8M
-# elements (us, library against linear_small: 4864 x 896, 64 tokens 13.8 / 10.6,
-# 128 tokens 10.5 / 13.0; 8192 x 2048, 128 tokens 21.4 / 16.8; 14336 x 4096, 128
-# tokens 75 / 34; 32768 x 5120, 128 tokens 194 / 78).
-_LINEAR_SMALL_ANY_TOKENS = 64
-_LINEAR_SMALL_MIN_WEIGHTS = 8 << 20
+# Products that linear runs faster than the library's GEMM: up to 64 tokens over
+# any weights, beyond over weights of at least 8M elements (us, library against
+# linear: 4864 x 896, 64 tokens 13.8 / 10.6, 128 tokens 10.5 / 13.0; 8192 x 2048,
+# 128 tokens 21.4 / 16.8, 512 tokens 33.5 / 29.6; 14336 x 4096, 128 tokens 75 /
+# 34, 512 tokens 88 / 69; 32768 x 5120, 128 tokens 194 / 78, 512 tokens 288 / 179).
+_LINEAR_ANY_TOKENS = 64
+_LINEAR_MIN_WEIGHTS = 8 << 20
 
 
-def linear_small_pays(x: torch.Tensor, weight: torch.Tensor) -> bool:
-    return (x.shape[0] <= _LINEAR_SMALL_ANY_TOKENS
-            or weight.numel() >= _LINEAR_SMALL_MIN_WEIGHTS)
+def linear_pays(x: torch.Tensor, weight: torch.Tensor) -> bool:
+    return x.shape[0] <= _LINEAR_ANY_TOKENS or weight.numel() >= _LINEAR_MIN_WEIGHTS
 
 
-def try_linear_small(x: torch.Tensor, weight: torch.Tensor, out: torch.Tensor,
+def try_linear(x: torch.Tensor, weight: torch.Tensor, out: torch.Tensor,
                      stream=None) -> bool:
-    """linear_small where it takes the tensors (linear_small_ok); False, with
+    """linear where it takes the tensors (linear_ok); False, with
     nothing done, where it does not."""
     if not x.is_cuda:
         return False
@@ -1112,20 +1114,20 @@ def try_linear_small(x: torch.Tensor, weight: torch.Tensor, out: torch.Tensor,
     return done is True
 
 
-def linear_small(x: torch.Tensor, weight: torch.Tensor, out: torch.Tensor,
+def linear(x: torch.Tensor, weight: torch.Tensor, out: torch.Tensor,
                  stream=None) -> torch.Tensor:
-    """out = round16(x @ weight.T) for few tokens (vaa_linear_small), on
-    tensors that linear_small_ok accepts."""
-    if try_linear_small(x, weight, out, stream):
+    """out = round16(x @ weight.T) (vaa_linear), on tensors that linear_ok
+    accepts."""
+    if try_linear(x, weight, out, stream):
         return out
-    if not linear_small_ok(x, weight, out):
-        raise ValueError(f"linear_small: x {tuple(x.shape)}, weight {tuple(weight.shape)}, out "
+    if not linear_ok(x, weight, out):
+        raise ValueError(f"linear: x {tuple(x.shape)}, weight {tuple(weight.shape)}, out "
                          f"{tuple(out.shape)}: not a supported shape, type or layout")
     t, k = x.shape
     n = weight.shape[0]
-    nbytes = _lib.load().vaa_linear_small_workspace_size(t, k, n)
+    nbytes = _lib.load().vaa_linear_workspace_size(t, k, n)
     ws = _stream_scratch(nbytes, x.device, stream)
-    _lib.call("vaa_linear_small", x.data_ptr(), x.stride(0), weight.data_ptr(), weight.stride(0),
+    _lib.call("vaa_linear", x.data_ptr(), x.stride(0), weight.data_ptr(), weight.stride(0),
               out.data_ptr(), out.stride(0), t, k, n, ATTN_DTYPES[x.dtype], _ptr(ws), nbytes,
               _lib.stream_handle(stream))
     return out
