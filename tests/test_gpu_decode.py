@@ -314,3 +314,41 @@ def test_merge_attn_states(gpu, dtype):
     out2 = kernels.merge_attn_states(po_d, lse_d, dtype=dtype)
     torch.cuda.synchronize()
     assert torch.equal(out2, out)
+
+
+@pytest.mark.parametrize("mode", [-1, -2])
+@pytest.mark.parametrize("lens,KV", [
+    ([16] * 90 + [1, 0, 17, 700], 8),          # ranges of many one-tile sequences
+    ([0, 0, 5, 0], 2), ([512], 2), ([511, 1, 513, 2048], 4),
+    ([40] * 300, 32), ([1500, 30] * 16, 32),   # shares above and below the doubled grid's
+    ([1600] * 26, 32),
+])
+def test_balanced_split_units(gpu, mode, lens, KV):
+    """The balanced split's shares: ranges that end inside a sequence's start-up
+    units, sequences whole in a range and over several, coarse and fine grids,
+    empty sequences; every row in 64 bits."""
+    from vllm_apple_amd import kernels
+
+    D, S = 32, len(lens)
+    g = torch.Generator(device="cuda").manual_seed(S + KV)
+    nblk = [-(-n // 16) for n in lens]
+    bt = torch.full((S, max(nblk)), -1, dtype=torch.int32, device="cuda")
+    perm = torch.randperm(sum(nblk) + 1, generator=g, device="cuda").int()
+    off = 0
+    for s, n in enumerate(nblk):
+        bt[s, :n] = perm[off:off + n]
+        off += n
+    kc, vc = (torch.randn(sum(nblk) + 1, KV, 16, D, generator=g, device="cuda").half()
+              for _ in range(2))
+    q = torch.randn(S, 2 * KV, D, generator=g, device="cuda").half()
+    out = kernels.paged_decode(q, kc, vc, bt, torch.tensor(lens, dtype=torch.int32).cuda(),
+                               scale=0.2, max_seq_len=max(lens), partition_size=mode)
+    for s, n in enumerate(lens):
+        ref = torch.zeros(2 * KV, D, dtype=torch.float64, device="cuda")
+        if n:
+            k, v = (c[bt[s, :nblk[s]].long()].transpose(1, 2).reshape(-1, KV, D)[:n].double()
+                    .transpose(0, 1).contiguous() for c in (kc, vc))
+            w = torch.softmax(0.2 * (q[s].double().view(KV, 2, 1, D) * k[:, None]).sum(-1), -1)
+            ref = (w[..., None] * v[:, None]).sum(2).view(2 * KV, D)
+        err = (out[s].double() - ref).abs()
+        assert bool((err <= 2e-3 + 1e-2 * ref.abs()).all()), (s, n, float(err.max()))
