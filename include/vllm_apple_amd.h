@@ -297,6 +297,28 @@ int vaa_paged_attention_prefill_split(const vaa_attn_params* p, const uint16_t* 
                                       size_t workspace_bytes, void* stream);
 
 /*
+ * A prefill-only step in two launches: the KV write of vaa_kv_write_slots (when
+ * new_keys and new_values are non-null) together with the indices of
+ * vaa_build_token_index over num_step_seqs sequences, then
+ * vaa_paged_attention_prefill over them, with the same results.  own_tiles != 0:
+ * every workgroup takes query tokens of one sequence only (up to 1024
+ * sequences), for batches whose sequences end inside a tile of consecutive tokens.
+ * p: as for the prefill, with new_kv_stride_*.  workspace:
+ * vaa_prefill_step_workspace_size bytes, 4-byte aligned, not shared by calls
+ * that can run concurrently.  A refused call may have written the cache rows
+ * and the workspace.
+ */
+size_t vaa_prefill_step_workspace_size(const vaa_attn_params* p, int num_tokens,
+                                       int num_step_seqs);
+int vaa_prefill_step(const vaa_attn_params* p, const uint16_t* query, uint16_t* key_cache,
+                     uint16_t* value_cache, const int32_t* block_table,
+                     const int32_t* seq_lens, const int32_t* query_start_loc,
+                     int num_step_seqs, const uint16_t* new_keys, const uint16_t* new_values,
+                     const void* slot_mapping, int slot_index_type, uint16_t* output,
+                     int num_tokens, int own_tiles, void* workspace, size_t workspace_bytes,
+                     void* stream);
+
+/*
  * Attention inside each sequence's own tokens, without a cache (encoder
  * models; vllm_apple/v1/attention/backends/base_attn.py:223-306): token t of
  * sequence s, the tokens [query_start_loc[s], query_start_loc[s + 1]), attends

@@ -23,7 +23,7 @@ namespace {
 #define VAA_FUNCS(X)                                                                      \
   X(vaa_kv_write_slots) X(vaa_paged_attention_decode)                                     \
   X(vaa_paged_attention_decode_workspace_size) X(vaa_paged_attention_prefill)             \
-  X(vaa_build_token_index) X(vaa_rmsnorm) X(vaa_add_rmsnorm) X(vaa_silu_mul)              \
+  X(vaa_prefill_step) X(vaa_prefill_step_workspace_size) X(vaa_rmsnorm) X(vaa_add_rmsnorm) X(vaa_silu_mul)              \
   X(vaa_qkv_epilogue) X(vaa_topk_logits) X(vaa_topk_workspace_size)                       \
   X(vaa_gate_up_silu_split) X(vaa_gate_up_silu_workspace_size) X(vaa_linear)        \
   X(vaa_linear_workspace_size) X(vaa_attention_no_cache)                            \
@@ -421,35 +421,46 @@ bool prefill_params(const Tensor& q, const Tensor& o, const Tensor& bt, int64_t 
   return true;
 }
 
-// One prefill-only step of the backend: K/V rows, the token index (into idx,
-// int32 [2 n]) and the unsplit prefill of the first n tokens.
+// One prefill-only step of the backend: K/V rows, indices (and, with own_tiles,
+// query tiles of one sequence each) and the unsplit prefill of the first n tokens.
 // (query, key, value, kv_cache, output, block_table, seq_lens, slots,
-//  query_start_loc, idx, n, write, head_size, scale, stream)
+//  query_start_loc, n, write, head_size, scale, own_tiles, workspace or None,
+//  stream)
 PyObject* step_prefill(const Args& a) {
   const Tensor *q = a.t(0), *k = a.t(1), *v = a.t(2), *c = a.t(3), *o = a.t(4), *bt = a.t(5),
-               *sl = a.t(6), *slots = a.t(7), *qsl = a.t(8), *idx = a.t(9);
-  const bool write = a.b(11);
-  if (!q || !c || !o || !bt || !sl || !qsl || !idx || (write && (!k || !v || !slots)))
+               *sl = a.t(6), *slots = a.t(7), *qsl = a.t(8), *ws = a.t(14);
+  const bool write = a.b(10);
+  if (!q || !c || !o || !bt || !sl || !qsl || (write && (!k || !v || !slots)) ||
+      !none_or_ten(a.a[14]))
     Py_RETURN_FALSE;
   const int dt = dt16(*q);
-  const int64_t n = a.i(10);
+  const int64_t n = a.i(9);
   vaa_attn_params p{};
   uint16_t *kc, *vc;
   if (dt < 0 || n <= 0 || dt16(*c) != dt || dt16(*o) != dt ||
       (write && (dt16(*k) != dt || dt16(*v) != dt)) || !cache5(*c, &p, &kc, &vc) ||
-      p.head_size != a.i(12) || !prefill_params(*q, *o, *bt, n, a.f(13), &p) || !is_i32(*qsl) ||
+      p.head_size != a.i(11) || !prefill_params(*q, *o, *bt, n, a.f(12), &p) || !is_i32(*qsl) ||
       !is_i32(*sl) || qsl->numel() < 1 || !small(qsl->numel()) ||
-      sl->numel() < qsl->numel() - 1 || !is_i32(*idx) || idx->numel() < 2 * n)
+      sl->numel() < qsl->numel() - 1)
     Py_RETURN_FALSE;
   p.dtype = dt;
-  void* stream = a.s(14);
-  int32_t* tok = static_cast<int32_t*>(ptr(*idx));
-  if (write && write_rows(p, *k, *v, kc, vc, *slots, n, stream)) Py_RETURN_FALSE;
-  if (p_vaa_build_token_index(static_cast<int32_t*>(ptr(*qsl)), static_cast<int32_t*>(ptr(*sl)),
-                              qsl->numel() - 1, n, tok, tok + n, stream) != VAA_OK)
-    Py_RETURN_FALSE;
-  return yes(p_vaa_paged_attention_prefill(&p, p16(*q), kc, vc, static_cast<int32_t*>(ptr(*bt)),
-                                           tok, tok + n, p16(*o), n, stream));
+  int it = 0;
+  if (write) {
+    it = slot_type(*slots, n);
+    if (it < 0 || !rows3(*k) || !same_rows(*k, *v) || k->size(0) < n ||
+        k->size(1) != p.num_kv_heads || k->size(2) != p.head_size)
+      Py_RETURN_FALSE;
+    p.new_kv_stride_token = k->stride(0);
+    p.new_kv_stride_head = k->stride(1);
+  }
+  const int S = static_cast<int>(qsl->numel() - 1);
+  const size_t need = p_vaa_prefill_step_workspace_size(&p, n, S);
+  if (!ws || !on_gpu(*ws) || ws->nbytes() < need) return PyLong_FromSize_t(need);
+  return yes(p_vaa_prefill_step(&p, p16(*q), kc, vc, static_cast<int32_t*>(ptr(*bt)),
+                                static_cast<int32_t*>(ptr(*sl)),
+                                static_cast<int32_t*>(ptr(*qsl)), S, write ? p16(*k) : nullptr,
+                                write ? p16(*v) : nullptr, write ? ptr(*slots) : nullptr, it,
+                                p16(*o), n, a.b(13), ptr(*ws), ws->nbytes(), a.s(15)));
 }
 
 // (query, key_cache, value_cache, block_table, token_to_seq, positions, output,
@@ -554,7 +565,7 @@ PyMethodDef methods[] = {{"bind", bind, METH_O, nullptr},
                          VAA_METHOD(kv_write, 7),
                          VAA_METHOD(decode, 14),
                          VAA_METHOD(step_decode, 16),
-                         VAA_METHOD(step_prefill, 15),
+                         VAA_METHOD(step_prefill, 16),
                          VAA_METHOD(prefill, 10),
                          VAA_METHOD(no_cache, 13),
                          {nullptr, nullptr, 0, nullptr}};

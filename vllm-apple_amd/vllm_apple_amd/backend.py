@@ -436,10 +436,17 @@ class HipAttentionImpl(AttentionImpl):
         if lens and md._query_start_loc_cpu and max(lens) > 32 * kernels._PREFILL_KEY_TILE:
             if self._prefill_split(md, query)[0]:
                 return False
-        idx = torch.empty(2 * n, dtype=torch.int32, device=query.device)
-        return native.step_prefill(query, key, value, kv_cache, output, md.block_table,
-                                   md.seq_lens, md.slot_mapping, md.query_start_loc, idx, n,
-                                   write, self.head_size, self.scale, handle) is True
+        # Query tiles of one sequence each, where a sequence ends inside a tile of
+        # consecutive tokens (host starts at hand; they only choose the grid).
+        qsl, tile = md._query_start_loc_cpu, kernels._prefill_tile_tokens(query.shape[1] // kvh)
+        own = bool(qsl) and any(b % tile for b in qsl[1:-1])
+        args = (query, key, value, kv_cache, output, md.block_table, md.seq_lens,
+                md.slot_mapping, md.query_start_loc, n, write, self.head_size, self.scale, own)
+        done = native.step_prefill(*args, None, handle)
+        if done is not True and done:
+            ws = torch.empty(done, dtype=torch.uint8, device=query.device)
+            done = native.step_prefill(*args, ws, handle)
+        return done is True
 
     def _prefill_split(self, md: HipAttentionMetadata, query: torch.Tensor) -> tuple:
         """(key split, longest prefill context) of a step's prefill from the

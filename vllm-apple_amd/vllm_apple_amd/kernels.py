@@ -539,6 +539,11 @@ _prefill_split_cache: dict = {}
 PREFILL_SPLIT_MAX_WORKSPACE = 256 << 20
 
 
+def _prefill_tile_tokens(group: int) -> int:
+    """Query tokens of a prefill workgroup for a GQA group of that many heads."""
+    return 32 * (1 if group >= 3 else 4 // max(1, group))
+
+
 def choose_prefill_split(ctx_lens_host, query_lens_host, num_kv_heads: int,
                          num_query_heads: int, num_cus: int, head_size: int = 128,
                          max_workspace_bytes: int = PREFILL_SPLIT_MAX_WORKSPACE) -> int:
@@ -566,7 +571,7 @@ def choose_prefill_split(ctx_lens_host, query_lens_host, num_kv_heads: int,
         return hit
     g = max(1, num_query_heads // max(1, num_kv_heads))
     heads_per_wg = 4 if g >= 4 else (3 if g == 3 else g)
-    tokens_per_wg = 32 * (1 if g >= 3 else 4 // g)
+    tokens_per_wg = _prefill_tile_tokens(g)
     chunks = -(-g // heads_per_wg)
     total, longest = 0, 0
     for ctx, q in zip(key[0], key[1]):
