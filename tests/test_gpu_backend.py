@@ -503,3 +503,64 @@ def test_forward_prefill_split_with_host_lengths(gpu, monkeypatch, dec_lens):
     assert seen and (seen[0] > 0) == (len(dec_lens) == 0)
     ref, kc, vc = _oracle(b, scale)
     assert_close(host(out), ref, what="forward with split prefill")
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+def test_forward_mixed_split_prefill_beside_decode(gpu, monkeypatch, dtype):
+    """A mixed step with one prefill context far longer than the rest splits its
+    keys beside the decode; graph replays give the same rows, which match the
+    oracle in fp16 and the unsplit step in both types (chunk lengths that are no multiple of a
+    tile, contexts that are no multiple of a piece)."""
+    from vllm_apple_amd import kernels
+    from vllm_apple_amd.backend import HipAttentionImpl
+
+    b = _mixed_batch(seed=21, dec_lens=(4000, 37, 300), pre=((12001, 187), (300, 65), (2049, 33)),
+                     dtype=dtype)
+    H, KV, D, T = b["H"], b["KV"], b["D"], b["T"]
+    scale = 1 / math.sqrt(D)
+    impl = HipAttentionImpl(H, D, scale, KV, None, None, "auto")
+    dev = torch.device("cuda")
+    qkv = b["qkv"].to(dev)
+    q = qkv[:, :H * D].view(T, H, D)
+    k = qkv[:, H * D:(H + KV) * D].view(T, KV, D)
+    v = qkv[:, (H + KV) * D:].view(T, KV, D)
+    kv_cache = b["kv_cache"].to(dev)
+    md = _metadata(b, dev)
+    md._seq_lens_cpu = b["lens"].tolist()
+    md._query_start_loc_cpu = b["qsl"].tolist()
+    seen = []
+    real = kernels.paged_prefill
+
+    def spy(*args, **kw):
+        seen.append(kw.get("split_keys", 0))
+        return real(*args, **kw)
+
+    monkeypatch.setattr(kernels, "paged_prefill", spy)
+    out = torch.zeros((T, H, D), dtype=dtype, device=dev)
+    impl.forward(None, q, k, v, kv_cache, md, output=out)
+    torch.cuda.synchronize()
+    assert seen == [2048]
+    if dtype == torch.float16:
+        ref, _, _ = _oracle(b, scale)
+        assert_close(host(out), ref, what="mixed step, prefill split beside the decode")
+    monkeypatch.setattr(kernels, "_SPLIT_BESIDE_TOKENS", 1 << 30)
+    kernels._prefill_split_cache.clear()
+    whole = torch.zeros_like(out)
+    impl.forward(None, q, k, v, kv_cache, md, output=whole)
+    torch.cuda.synchronize()
+    assert seen == [2048, 0]
+    # Half an ulp of rounding each, at most 2^-7 of the value in bf16.
+    assert_close(host(out.float()), host(whole.float()), what="split against whole")
+    monkeypatch.setattr(kernels, "_SPLIT_BESIDE_TOKENS", 4096)
+    kernels._prefill_split_cache.clear()
+    g = torch.cuda.CUDAGraph()
+    again = torch.zeros_like(out)
+    with torch.cuda.graph(g):
+        impl.forward(None, q, k, v, kv_cache, md, output=again)
+    for r in range(3):
+        again.zero_()
+        torch.cuda.synchronize()
+        g.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(again, out), f"replay {r}"
+        _ = (again.float() * 2).sum().item()

@@ -293,6 +293,32 @@ def test_prefill_split_choice():
     assert K.choose_prefill_split([2000, 100], [64, 64], 8, 32, 256) == 0
 
 
+@pytest.mark.parametrize("ctx,q,dec,want", [
+    # One context outlasts the other chunks and the decode: split, and only it
+    # where more pieces would not fit the chip's 512 slots and an eighth.
+    ([1671, 10219, 2192, 637, 16317, 2347, 694, 9274], 256, 237_883, 10240),
+    ([8166, 1807, 272, 316, 2713, 11009], 187, 65_983, 3072),
+    ([805, 7792, 8236, 733, 14652, 4049, 510, 1132], 64, 113_776, 3072),
+    ([7178, 2440, 2631], 211, 32_288, 2048),
+    # The decode, or the chunks together, last as long.
+    ([3687, 12930, 3786, 15986, 16351, 2973, 14549, 2983], 256, 465_892, 0),
+    ([5722, 3260, 278, 3370], 256, 113_288, 0),
+    ([3072, 40], 64, 5000, 0),         # within 48 key tiles
+    ([3073, 40], 64, 5000, 2048),      # just past them
+    ([9000, 40], 64, 4096, 2048),      # the fewest decode tokens that split
+    ([9000, 40], 64, 4095, 0),
+    ([131072], 2, 5000, 2048),         # pieces up to the slots: 64 x 8 workgroups
+    ([1 << 20], 2, 5000, 15360),       # 69 x 8: the slots and an eighth
+    ([16384] * 64, 512, 5000, 0),      # more workgroups than slots, all equal
+])
+def test_prefill_split_beside_decode(ctx, q, dec, want):
+    from vllm_apple_amd import kernels as K
+
+    K._prefill_split_cache.clear()
+    sp = K.choose_prefill_split(ctx, [q] * len(ctx), 8, 32, 256, beside_decode_tokens=dec)
+    assert sp == want and sp % 1024 == 0
+
+
 def test_prefill_split_workspace_is_bounded():
     """One 256-token chunk at a 128k context beside 31 short 248-token
     prefills: the share-based piece (10240 keys, 13 pieces over 7944 tokens)

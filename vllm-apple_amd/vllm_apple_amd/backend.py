@@ -373,18 +373,26 @@ class HipAttentionImpl(AttentionImpl):
 
             def prefill():
                 # Split long contexts when the host lengths are at hand (never
-                # a device sync for them) and no decode runs beside the
-                # prefill: next to a decode the unsplit prefill is better (its
-                # long workgroups hold a few CUs and leave the rest to the
-                # decode; C5 attention step 0.61 ms against 0.68-0.79 split).
+                # a device sync for them).  Next to a decode the unsplit
+                # prefill is better (its long workgroups hold a few CUs and
+                # leave the rest to the decode; C5 attention step 0.61 ms
+                # against 0.68-0.79 split) unless one context outlasts all
+                # else: choose_prefill_split has a rule for each.
                 # The pieces are counted over the longest prefill context
                 # (decode contexts do not matter), which bounds the workspace.
-                split, longest = (0, 0) if overlapped else self._prefill_split(attn_metadata,
-                                                                               query)
+                split, longest = self._prefill_split(attn_metadata, query, overlapped)
+                # Beside a decode the partials are the call's own memory: steps
+                # of several streams may be in flight.
+                ws = None
+                if split and overlapped:
+                    ws = torch.empty((n - nd) * query.shape[1] * -(-longest // split)
+                                     * (self.head_size + 2), dtype=torch.float32,
+                                     device=query.device)
                 kernels.paged_prefill(query[nd:n], key_cache, value_cache,
                                       attn_metadata.block_table, tok[nd:n], pos[nd:n],
                                       scale=self.scale, layout="vllm", output=output[nd:n],
-                                      split_keys=split, max_seq_len=longest if split else 0)
+                                      split_keys=split, max_seq_len=longest if split else 0,
+                                      workspace=ws)
 
             if n > nd:
                 tok, pos = kernels.build_token_index(attn_metadata.query_start_loc,
@@ -448,16 +456,24 @@ class HipAttentionImpl(AttentionImpl):
             done = native.step_prefill(*args, ws, handle)
         return done is True
 
-    def _prefill_split(self, md: HipAttentionMetadata, query: torch.Tensor) -> tuple:
+    def _prefill_split(self, md: HipAttentionMetadata, query: torch.Tensor,
+                       overlapped: bool = False) -> tuple:
         """(key split, longest prefill context) of a step's prefill from the
-        host lengths; (0, 0) without them."""
+        host lengths; (0, 0) without them.  overlapped: the step's decodes run
+        beside it."""
         lens_host, qsl_host = md._seq_lens_cpu, md._query_start_loc_cpu
         if not lens_host or not qsl_host:
             return 0, 0
+        if overlapped and max(lens_host) <= kernels._SPLIT_BESIDE_TILES * kernels._PREFILL_KEY_TILE:
+            return 0, 0  # nothing that the rule below splits
         ql = [b - a if b - a > 1 else 0 for a, b in zip(qsl_host[:-1], qsl_host[1:])]
+        # A query of one token is a decode only in front of the prefills.
+        beside = sum(l for l, b in zip(lens_host, qsl_host[1:])
+                     if b <= md.num_decode_tokens) if overlapped else None
         split = kernels.choose_prefill_split(
             lens_host, ql, self.num_kv_heads, query.shape[1],
-            kernels.device_cus(query.device), head_size=self.head_size)
+            kernels.device_cus(query.device), head_size=self.head_size,
+            beside_decode_tokens=beside)
         return split, max((l for l, q in zip(lens_host, ql) if q > 0), default=0)
 
     def _attention_no_cache(self, query: torch.Tensor, key: torch.Tensor, value: torch.Tensor,

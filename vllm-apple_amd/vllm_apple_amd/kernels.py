@@ -531,6 +531,8 @@ def merge_attn_states(partial_out: torch.Tensor, partial_lse: torch.Tensor, *,
 _prefill_ws = _GrowOnlyScratch()
 _PREFILL_KEY_TILE = 64      # keys per prefill tile (paged_prefill.hip)
 _PREFILL_SPLIT_QUANTUM = 1024  # split sizes in multiples of 16 key tiles
+_SPLIT_BESIDE_TILES = 48     # key tiles past which a prefill beside a decode may split
+_SPLIT_BESIDE_TOKENS = 4096  # decode tokens from which a prefill beside them may split
 _prefill_split_cache: dict = {}
 # Largest split-K prefill workspace choose_prefill_split plans for: the
 # partials take num_tokens * H * pieces * (D + 2) * 4 bytes, so a long
@@ -546,7 +548,8 @@ def _prefill_tile_tokens(group: int) -> int:
 
 def choose_prefill_split(ctx_lens_host, query_lens_host, num_kv_heads: int,
                          num_query_heads: int, num_cus: int, head_size: int = 128,
-                         max_workspace_bytes: int = PREFILL_SPLIT_MAX_WORKSPACE) -> int:
+                         max_workspace_bytes: int = PREFILL_SPLIT_MAX_WORKSPACE,
+                         beside_decode_tokens: int | None = None) -> int:
     """Key split for a prefill batch (0: none), from the host lengths.
 
     The prefill kernel gives each workgroup a query tile (32 tokens of 4
@@ -561,11 +564,30 @@ def choose_prefill_split(ctx_lens_host, query_lens_host, num_kv_heads: int,
     paged_prefill's max_seq_len), and the partials of all prefill tokens
     (sum of the query lengths) must fit max_workspace_bytes: otherwise the
     pieces grow until they do, or the split is dropped.
+
+    beside_decode_tokens (cached tokens that a decode running beside the
+    prefill reads) applies the rule for an overlapped step instead.  There the
+    longest workgroup may last as long as everything else, since the decode
+    fills the other CUs, and a split that adds workgroups past the chip's slots
+    holds the decode back; below that it shortens the step.  In key tiles: the
+    prefill's share counts 1.4 per tile and the decode's tokens 5.8e-5 per kv
+    head (HBM time over 1.6 us a tile).  A split is chosen when the longest
+    workgroup exceeds 1.1x their sum; the pieces are the shortest of at least
+    half the sum whose workgroups stay within an eighth over the slots (or
+    over the unsplit grid).  Beside fewer than 4096 decode tokens a step stays
+    unsplit: tests/test_gpu_backend.py pins that for two short decodes (a split
+    would be faster there too).  Overlapped steps of 32/8 heads, D 128, unsplit ->
+    this rule, us: 8 chunks of 256 up to 16317 keys beside 238k decode tokens
+    407 -> 343 (bf16 484 -> 425); 6 of 187 up to 11009 beside 66k 309 -> 180;
+    8 of 64 up to 14652 beside 114k, bf16, 413 -> 182; 2 of 38 up to 9519 beside
+    184k 432 -> 228.  On the other side of
+    the line: 8 of 256 up to 16351 beside 466k 557, split 606 at the least;
+    4 of 256 up to 5722 beside 113k 154, split 154 to 188.
     Memoised per length tuple (every layer of a step sees the same batch).
     """
     key = (tuple(int(x) for x in ctx_lens_host), tuple(int(x) for x in query_lens_host),
            int(num_kv_heads), int(num_query_heads), int(num_cus), int(head_size),
-           int(max_workspace_bytes))
+           int(max_workspace_bytes), beside_decode_tokens)
     hit = _prefill_split_cache.get(key)
     if hit is not None:
         return hit
@@ -573,17 +595,25 @@ def choose_prefill_split(ctx_lens_host, query_lens_host, num_kv_heads: int,
     heads_per_wg = 4 if g >= 4 else (3 if g == 3 else g)
     tokens_per_wg = _prefill_tile_tokens(g)
     chunks = -(-g // heads_per_wg)
-    total, longest = 0, 0
-    for ctx, q in zip(key[0], key[1]):
-        if q <= 0 or ctx <= 0:
-            continue
-        tiles = -(-ctx // _PREFILL_KEY_TILE)
-        total += -(-q // tokens_per_wg) * tiles
-        longest = max(longest, tiles)
-    total *= num_kv_heads * chunks
-    share = total / max(1, 2 * num_cus)
+    work = [(-(-q // tokens_per_wg), -(-ctx // _PREFILL_KEY_TILE))
+            for ctx, q in zip(key[0], key[1]) if q > 0 and ctx > 0]
+    longest = max((tiles for _, tiles in work), default=0)
+    heads_grid = num_kv_heads * chunks
+    slots = max(1, 2 * num_cus)
+    share = sum(q * tiles for q, tiles in work) * heads_grid / slots
     split = 0
-    if longest > 32 and longest > 1.5 * share:
+    if beside_decode_tokens is not None:
+        rest = 1.4 * share + 5.8e-5 * beside_decode_tokens * num_kv_heads
+        if beside_decode_tokens >= _SPLIT_BESIDE_TOKENS \
+                and longest > max(_SPLIT_BESIDE_TILES, 1.1 * rest):
+            quantum = _PREFILL_SPLIT_QUANTUM // _PREFILL_KEY_TILE
+            most = max(slots, sum(q for q, _ in work) * heads_grid) + slots // 8
+            piece = max(2, -(-int(rest / 2) // quantum)) * quantum
+            while piece < longest and \
+                    sum(q * -(-tiles // piece) for q, tiles in work) * heads_grid > most:
+                piece += quantum
+            split = piece * _PREFILL_KEY_TILE if piece < longest else 0
+    elif longest > 32 and longest > 1.5 * share:
         piece = max(_PREFILL_SPLIT_QUANTUM, int(share / 2) * _PREFILL_KEY_TILE)
         split = -(-piece // _PREFILL_SPLIT_QUANTUM) * _PREFILL_SPLIT_QUANTUM
         if split >= longest * _PREFILL_KEY_TILE:
