@@ -319,6 +319,29 @@ int vaa_prefill_step(const vaa_attn_params* p, const uint16_t* query, uint16_t* 
                      void* stream);
 
 /*
+ * The prefill with query tiles of one sequence each, for sequences that end inside
+ * a tile of consecutive tokens; results as vaa_paged_attention_prefill (split_keys
+ * 0) or _prefill_split over the same indices.  vaa_build_prefill_tiles writes the
+ * indices of vaa_build_token_index for the tokens [first_token, first_token +
+ * num_tokens) of the step, counted from first_token, over num_seqs sequences
+ * (query_start_loc holds the step's positions, num_seqs + 1 entries from the first of
+ * these sequences on), and tiles, 2 * num_tiles entries, where num_tiles is
+ * vaa_prefill_tile_count's (0: unsupported, more than 1024 sequences).  The prefill
+ * takes these tiles only.  Split: workspace as for vaa_paged_attention_prefill_split.
+ */
+int vaa_prefill_tile_count(int num_tokens, int num_seqs, int queries_per_kv);
+int vaa_build_prefill_tiles(const int32_t* query_start_loc, const int32_t* seq_lens, int num_seqs,
+                            int first_token, int num_tokens, int queries_per_kv,
+                            int32_t* token_to_seq, int32_t* positions, int32_t* tiles,
+                            int num_tiles, void* stream);
+int vaa_paged_attention_prefill_tiles(const vaa_attn_params* p, const uint16_t* query,
+                                      const uint16_t* key_cache, const uint16_t* value_cache,
+                                      const int32_t* block_table, const int32_t* token_to_seq,
+                                      const int32_t* positions, uint16_t* output, int num_tokens,
+                                      const int32_t* tiles, int num_tiles, int split_keys,
+                                      void* workspace, size_t workspace_bytes, void* stream);
+
+/*
  * Attention inside each sequence's own tokens, without a cache (encoder
  * models; vllm_apple/v1/attention/backends/base_attn.py:223-306): token t of
  * sequence s, the tokens [query_start_loc[s], query_start_loc[s + 1]), attends

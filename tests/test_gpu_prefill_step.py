@@ -65,6 +65,46 @@ def test_step(gpu, lens, prefix, H, KV, D, own, write):
     assert bool((ws[n // 4:] == -77).all()), "workspace overrun"
 
 
+@pytest.mark.parametrize("split", [0, 64, 128])
+@pytest.mark.parametrize("lens,H,KV,D", [
+    ([33], 8, 2, 128), ([187, 1, 65, 0, 31], 32, 8, 128), ([127, 129, 3], 4, 4, 64),
+    ([65, 63, 2], 8, 4, 96),
+])
+def test_tiles_behind_decodes(gpu, lens, H, KV, D, split):
+    """The prefill of a mixed step's chunks over a tile table: the same bits as
+    over consecutive tokens, the decodes' rows untouched."""
+    from vllm_apple_amd import kernels
+
+    nd, prefix = 5, 300
+    new = [1] * nd + lens
+    S, T = len(new), sum(new)
+    g = torch.Generator().manual_seed(T)
+    total = [prefix + 17 * i + n if n else 0 for i, n in enumerate(new)]
+    nb = -(-max(total) // 16)
+    bt = torch.randperm(S * nb, generator=g).int().view(S, nb).cuda()
+    cache = torch.randn(2, S * nb, 16, KV, D, generator=g).half().cuda()
+    q = torch.randn(T, H, D, generator=g).half().cuda()
+    qsl = torch.tensor([0] + torch.tensor(new).cumsum(0).tolist(), dtype=torch.int32).cuda()
+    sl = torch.tensor(total, dtype=torch.int32).cuda()
+    tok, pos = kernels.build_token_index(qsl, sl, T)
+    ref, out = torch.full_like(q, 7.0), torch.full_like(q, 7.0)
+    kw = dict(scale=0.1, layout="vllm", split_keys=split, max_seq_len=max(total) if split else 0)
+    kernels.paged_prefill(q[nd:], cache[0], cache[1], bt, tok[nd:], pos[nd:], output=ref[nd:], **kw)
+    t, p, tiles = kernels.build_prefill_tiles(qsl[nd:], sl[nd:], nd, T - nd, H // KV)
+    assert torch.equal(t + nd, tok[nd:]) and torch.equal(p, pos[nd:])
+    per = kernels._prefill_tile_tokens(H // KV)
+    want, at = [], 0
+    for n in lens:
+        want += [(at + i, min(per, n - i)) for i in range(0, n, per)]
+        at += n
+    want += [(0, 0)] * (tiles.shape[0] - len(want))
+    assert [tuple(x) for x in tiles.tolist()] == want
+    kernels.paged_prefill(q[nd:], cache[0], cache[1], bt[nd:], t, p, output=out[nd:], tiles=tiles,
+                          **kw)
+    torch.cuda.synchronize()
+    assert torch.equal(out.view(torch.int16), ref.view(torch.int16))
+
+
 def test_step_workspace_refused(gpu):
     from vllm_apple_amd import _lib
 

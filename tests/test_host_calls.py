@@ -9,7 +9,7 @@ from vllm_apple_amd import _lib, backend, kernels
 NAMES = ["norm", "silu", "epilogue", "topk", "gate_up", "linear", "kv_write", "decode",
          "step_decode", "step_prefill", "prefill", "no_cache"]
 COUNTS = dict(norm=7, silu=4, epilogue=13, topk=6, gate_up=6, linear=5, kv_write=7, decode=14,
-              step_decode=16, step_prefill=16, prefill=10, no_cache=13)
+              step_decode=16, step_prefill=16, prefill=14, no_cache=13)
 
 
 @pytest.mark.parametrize("name", NAMES)

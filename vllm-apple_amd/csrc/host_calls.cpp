@@ -23,7 +23,9 @@ namespace {
 #define VAA_FUNCS(X)                                                                      \
   X(vaa_kv_write_slots) X(vaa_paged_attention_decode)                                     \
   X(vaa_paged_attention_decode_workspace_size) X(vaa_paged_attention_prefill)             \
-  X(vaa_prefill_step) X(vaa_prefill_step_workspace_size) X(vaa_rmsnorm) X(vaa_add_rmsnorm) X(vaa_silu_mul)              \
+  X(vaa_paged_attention_prefill_split) X(vaa_paged_attention_prefill_tiles)               \
+  X(vaa_paged_attention_prefill_workspace_size) X(vaa_prefill_step)                       \
+  X(vaa_prefill_step_workspace_size) X(vaa_rmsnorm) X(vaa_add_rmsnorm) X(vaa_silu_mul)    \
   X(vaa_qkv_epilogue) X(vaa_topk_logits) X(vaa_topk_workspace_size)                       \
   X(vaa_gate_up_silu_split) X(vaa_gate_up_silu_workspace_size) X(vaa_linear)        \
   X(vaa_linear_workspace_size) X(vaa_attention_no_cache)                            \
@@ -464,23 +466,46 @@ PyObject* step_prefill(const Args& a) {
 }
 
 // (query, key_cache, value_cache, block_table, token_to_seq, positions, output,
-//  vllm, scale, stream): unsplit
+//  vllm, scale, tiles or None, split_keys, max_seq_len, workspace or None, stream)
 PyObject* prefill(const Args& a) {
   const Tensor *q = a.t(0), *kc = a.t(1), *vc = a.t(2), *bt = a.t(3), *tok = a.t(4),
-               *pos = a.t(5), *o = a.t(6);
-  if (!q || !kc || !vc || !bt || !tok || !pos || !o) Py_RETURN_FALSE;
+               *pos = a.t(5), *o = a.t(6), *tiles = a.t(9), *ws = a.t(12);
+  if (!q || !kc || !vc || !bt || !tok || !pos || !o || !none_or_ten(a.a[9]) ||
+      !none_or_ten(a.a[12]))
+    Py_RETURN_FALSE;
   const int dt = dt16(*q);
+  const int64_t split = a.i(10), max_len = a.i(11);
   vaa_attn_params p{};
   if (dt < 0 || dt16(*kc) != dt || dt16(*vc) != dt || dt16(*o) != dt || q->dim() != 3 ||
       !cache4(*kc, *vc, a.b(7), &p) || !prefill_params(*q, *o, *bt, q->size(0), a.f(8), &p) ||
-      !is_i32(*tok) || !is_i32(*pos) || tok->numel() < q->size(0) || pos->numel() < q->size(0))
+      !is_i32(*tok) || !is_i32(*pos) || tok->numel() < q->size(0) || pos->numel() < q->size(0) ||
+      !small(split) || !small(max_len) || (split && !max_len) ||
+      (tiles && (!is_i32(*tiles) || tiles->dim() != 2 || tiles->size(1) != 2 ||
+                 !small(tiles->size(0)))))
     Py_RETURN_FALSE;
   p.dtype = dt;
-  return yes(p_vaa_paged_attention_prefill(&p, p16(*q), p16(*kc), p16(*vc),
-                                           static_cast<int32_t*>(ptr(*bt)),
-                                           static_cast<int32_t*>(ptr(*tok)),
-                                           static_cast<int32_t*>(ptr(*pos)), p16(*o), q->size(0),
-                                           a.s(9)));
+  const int n = static_cast<int>(q->size(0));
+  size_t need = 0;
+  if (split) {
+    p.max_seq_len = max_len;
+    need = p_vaa_paged_attention_prefill_workspace_size(&p, n, split);
+    if (need && (!ws || !on_gpu(*ws) || ws->nbytes() < need)) return PyLong_FromSize_t(need);
+  }
+  auto* btp = static_cast<int32_t*>(ptr(*bt));
+  auto* tp = static_cast<int32_t*>(ptr(*tok));
+  auto* pp = static_cast<int32_t*>(ptr(*pos));
+  void* wp = need ? ptr(*ws) : nullptr;
+  if (tiles)
+    return yes(p_vaa_paged_attention_prefill_tiles(
+        &p, p16(*q), p16(*kc), p16(*vc), btp, tp, pp, p16(*o), n,
+        static_cast<int32_t*>(ptr(*tiles)), static_cast<int>(tiles->size(0)), split, wp,
+        need ? ws->nbytes() : 0, a.s(13)));
+  if (split)
+    return yes(p_vaa_paged_attention_prefill_split(&p, p16(*q), p16(*kc), p16(*vc), btp, tp, pp,
+                                                   p16(*o), n, split, wp, need ? ws->nbytes() : 0,
+                                                   a.s(13)));
+  return yes(p_vaa_paged_attention_prefill(&p, p16(*q), p16(*kc), p16(*vc), btp, tp, pp, p16(*o),
+                                           n, a.s(13)));
 }
 
 // 16-byte aligned rows, which the attention kernels read directly.
@@ -566,7 +591,7 @@ PyMethodDef methods[] = {{"bind", bind, METH_O, nullptr},
                          VAA_METHOD(decode, 14),
                          VAA_METHOD(step_decode, 16),
                          VAA_METHOD(step_prefill, 16),
-                         VAA_METHOD(prefill, 10),
+                         VAA_METHOD(prefill, 14),
                          VAA_METHOD(no_cache, 13),
                          {nullptr, nullptr, 0, nullptr}};
 PyModuleDef module = {PyModuleDef_HEAD_INIT, "_host", nullptr, -1, methods,

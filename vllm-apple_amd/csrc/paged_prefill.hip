@@ -642,7 +642,7 @@ paged_prefill_kernel(PrefillArgs a) {
   // Per-lane query token (lanes l and l+32 share token qj).
   int first = tile_x * (kQT * a.subtiles), count = kQT * a.subtiles;
   if (a.tiles) {
-    first = scalar_load_i32(a.tiles + 2 * tile_x);
+    first = max(scalar_load_i32(a.tiles + 2 * tile_x), 0);
     count = scalar_load_i32(a.tiles + 2 * tile_x + 1);
     if (count <= 0) return;
   }
@@ -1150,6 +1150,7 @@ struct IndexArgs {
   const int32_t* qsl;
   const int32_t* seq_lens;  // positions end at seq_lens[s] - 1; null: no-cache
   int num_seqs, num_tokens, causal;
+  int first;                // with seq_lens: the token that the indices count from
   int32_t* tok;
   int32_t* pos;
   int32_t* bt;              // no-cache block table [num_seqs, max_blocks], or null
@@ -1172,7 +1173,7 @@ __device__ __forceinline__ void index_block(const IndexArgs& a, int64_t blk, Ind
   // No-cache starts are clamped to the tensors' rows, so that no entry lets the
   // prefill read past them whatever query_start_loc holds (its paged reads are
   // checked by block).
-  auto raw = [&](int s) { return a.seq_lens ? a.qsl[s] : clamp(a.qsl[s]); };
+  auto raw = [&](int s) { return a.seq_lens ? a.qsl[s] - a.first : clamp(a.qsl[s]); };
   if (lds) {
     for (int i = tid; i <= S; i += kIdxThreads) sm.start[i] = raw(i);
     __syncthreads();
@@ -1308,6 +1309,63 @@ int launch_index(const IndexArgs& a, hipStream_t stream) {
 
 }  // namespace
 }  // namespace vaa
+
+// Indices and query tiles of a mixed step's prefill sequences, built in front of the
+// fork to the decode's stream, and the prefill over them.
+//
+// Chunks that are no multiple of a tile (what a token budget leaves) made tiles that
+// walk two contexts: five chunks of 201 tokens over 1318 to 9715 keys beside 14
+// decodes, split in pieces of 4096 keys, 228 us a step, 152 with the table; two of 113
+// over up to 4454 beside 19, bf16, 160 -> 112; aligned chunks (no table) the same.
+extern "C" int vaa_prefill_tile_count(int num_tokens, int num_seqs, int queries_per_kv) {
+  if (num_tokens <= 0 || num_seqs < 0 || num_seqs > kIdxSeqs || queries_per_kv <= 0) return 0;
+  const int64_t n = tile_bound(num_tokens, num_seqs, tile_tokens(queries_per_kv));
+  return n <= INT32_MAX / 2 ? static_cast<int>(n) : 0;
+}
+
+extern "C" int vaa_build_prefill_tiles(const int32_t* query_start_loc, const int32_t* seq_lens,
+                                       int num_seqs, int first_token, int num_tokens,
+                                       int queries_per_kv, int32_t* token_to_seq,
+                                       int32_t* positions, int32_t* tiles, int num_tiles,
+                                       void* stream) {
+  const char* what = "vaa_build_prefill_tiles";
+  const int need = vaa_prefill_tile_count(num_tokens, num_seqs, queries_per_kv);
+  if (num_tokens < 0 || num_seqs < 0 || first_token < 0 || queries_per_kv <= 0)
+    return fail(VAA_ERR_INVALID_ARG, "%s: num_seqs=%d first_token=%d num_tokens=%d", what,
+                num_seqs, first_token, num_tokens);
+  if (num_tokens == 0) return VAA_OK;
+  if (need == 0)
+    return fail(VAA_ERR_UNSUPPORTED, "%s: num_seqs=%d (at most %d)", what, num_seqs, kIdxSeqs);
+  if (num_tiles != need)
+    return fail(VAA_ERR_INVALID_ARG, "%s: num_tiles=%d, not %d", what, num_tiles, need);
+  if (!query_start_loc || !seq_lens || !token_to_seq || !positions || !tiles)
+    return fail(VAA_ERR_INVALID_ARG, "%s: null pointer", what);
+  IndexArgs ia{};
+  ia.qsl = query_start_loc;
+  ia.seq_lens = seq_lens;
+  ia.num_seqs = num_seqs;
+  ia.num_tokens = num_tokens;
+  ia.first = first_token;
+  ia.tok = token_to_seq;
+  ia.pos = positions;
+  ia.tiles = tiles;
+  ia.per = tile_tokens(queries_per_kv);
+  ia.num_tiles = need;
+  return launch_index(ia, static_cast<hipStream_t>(stream));
+}
+
+extern "C" int vaa_paged_attention_prefill_tiles(
+    const vaa_attn_params* p, const uint16_t* query, const uint16_t* key_cache,
+    const uint16_t* value_cache, const int32_t* block_table, const int32_t* token_to_seq,
+    const int32_t* positions, uint16_t* output, int num_tokens, const int32_t* tiles,
+    int num_tiles, int split_keys, void* workspace, size_t workspace_bytes, void* stream) {
+  const char* what = "vaa_paged_attention_prefill_tiles";
+  if (!tiles || num_tiles <= 0 || num_tiles > INT32_MAX / 2)
+    return fail(VAA_ERR_INVALID_ARG, "%s: num_tiles=%d", what, num_tiles);
+  return prefill_impl(what, p, query, key_cache, value_cache, block_table, token_to_seq, positions,
+                      output, num_tokens, split_keys, workspace, workspace_bytes, stream, tiles,
+                      num_tiles);
+}
 
 // One prefill-only step: KV write, indices, prefill.
 extern "C" size_t vaa_prefill_step_workspace_size(const vaa_attn_params* p, int num_tokens,

@@ -100,6 +100,10 @@ SIGNATURES = {
     "vaa_prefill_step_workspace_size": (ctypes.c_size_t, [_PARAMS, _I, _I]),
     "vaa_prefill_step": (_I, [_PARAMS, _P, _P, _P, _P, _P, _P, _I, _P, _P, _P, _I, _P, _I, _I, _P,
                               ctypes.c_size_t, _P]),
+    "vaa_prefill_tile_count": (_I, [_I, _I, _I]),
+    "vaa_build_prefill_tiles": (_I, [_P, _P, _I, _I, _I, _I, _P, _P, _P, _I, _P]),
+    "vaa_paged_attention_prefill_tiles": (_I, [_PARAMS, _P, _P, _P, _P, _P, _P, _P, _I, _P, _I, _I,
+                                               _P, ctypes.c_size_t, _P]),
     "vaa_attention_no_cache_workspace_size": (ctypes.c_size_t, [_I, _I, _I]),
     "vaa_attention_no_cache": (_I, [_PARAMS, _P, _P, _P, _P, _P, _I, _I, _P, ctypes.c_size_t, _P]),
     "vaa_paged_attention_decode_noalloc_max_workspace": (ctypes.c_size_t, []),

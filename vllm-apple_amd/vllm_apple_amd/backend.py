@@ -388,15 +388,25 @@ class HipAttentionImpl(AttentionImpl):
                     ws = torch.empty((n - nd) * query.shape[1] * -(-longest // split)
                                      * (self.head_size + 2), dtype=torch.float32,
                                      device=query.device)
-                kernels.paged_prefill(query[nd:n], key_cache, value_cache,
-                                      attn_metadata.block_table, tok[nd:n], pos[nd:n],
+                kernels.paged_prefill(query[nd:n], key_cache, value_cache, bt, tok, pos,
                                       scale=self.scale, layout="vllm", output=output[nd:n],
                                       split_keys=split, max_seq_len=longest if split else 0,
-                                      workspace=ws)
+                                      workspace=ws, tiles=tiles)
 
-            if n > nd:
+            # Where a mixed step's chunk ends inside a query tile, tiles of one
+            # sequence each; sequence i < nd is decode token i.
+            own = None
+            if overlapped and self._own_tiles(attn_metadata, query, nd):
+                own = kernels.build_prefill_tiles(attn_metadata.query_start_loc[nd:],
+                                                  attn_metadata.seq_lens[nd:], nd, n - nd,
+                                                  query.shape[1] // key_cache.shape[2])
+            if own is not None:
+                tok, pos, tiles = own
+                bt = attn_metadata.block_table[nd:]
+            elif n > nd:
                 tok, pos = kernels.build_token_index(attn_metadata.query_start_loc,
                                                      attn_metadata.seq_lens, n)
+                tok, pos, tiles, bt = tok[nd:n], pos[nd:n], None, attn_metadata.block_table
             if overlapped:
                 # Mixed step: prefill (MFMA-bound, current stream, dispatched
                 # first) and decode (HBM-bound, side stream, shared split) run
@@ -444,10 +454,7 @@ class HipAttentionImpl(AttentionImpl):
         if lens and md._query_start_loc_cpu and max(lens) > 32 * kernels._PREFILL_KEY_TILE:
             if self._prefill_split(md, query)[0]:
                 return False
-        # Query tiles of one sequence each, where a sequence ends inside a tile of
-        # consecutive tokens (host starts at hand; they only choose the grid).
-        qsl, tile = md._query_start_loc_cpu, kernels._prefill_tile_tokens(query.shape[1] // kvh)
-        own = bool(qsl) and any(b % tile for b in qsl[1:-1])
+        own = self._own_tiles(md, query, 0)
         args = (query, key, value, kv_cache, output, md.block_table, md.seq_lens,
                 md.slot_mapping, md.query_start_loc, n, write, self.head_size, self.scale, own)
         done = native.step_prefill(*args, None, handle)
@@ -455,6 +462,16 @@ class HipAttentionImpl(AttentionImpl):
             ws = torch.empty(done, dtype=torch.uint8, device=query.device)
             done = native.step_prefill(*args, ws, handle)
         return done is True
+
+    def _own_tiles(self, md: HipAttentionMetadata, query: torch.Tensor, nd: int) -> bool:
+        """Whether a prefill sequence behind the first nd, decodes of one token
+        each, ends inside a query tile of consecutive tokens (host starts at hand;
+        they only choose the grid)."""
+        qsl = md._query_start_loc_cpu
+        if not qsl or len(qsl) <= nd + 1 or qsl[nd] != nd:
+            return False
+        tile = kernels._prefill_tile_tokens(query.shape[1] // self.num_kv_heads)
+        return any((b - nd) % tile for b in qsl[nd + 1:-1])
 
     def _prefill_split(self, md: HipAttentionMetadata, query: torch.Tensor,
                        overlapped: bool = False) -> tuple:

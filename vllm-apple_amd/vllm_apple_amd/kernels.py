@@ -647,7 +647,7 @@ def paged_prefill(query: torch.Tensor, key_cache: torch.Tensor, value_cache: tor
                   positions: torch.Tensor, *, scale: float, layout: str = "kernel",
                   output: torch.Tensor | None = None, split_keys: int = 0,
                   max_seq_len: int = 0, workspace: torch.Tensor | None = None,
-                  stream=None) -> torch.Tensor:
+                  stream=None, tiles: torch.Tensor | None = None) -> torch.Tensor:
     """Chunked-prefill attention: token t attends to cache positions [0, positions[t]].
 
     query [num_tokens, H, D] fp16 or bf16, as the caches and output; the
@@ -658,10 +658,13 @@ def paged_prefill(query: torch.Tensor, key_cache: torch.Tensor, value_cache: tor
     multiple of 64; see choose_prefill_split) merged by log-sum-exp;
     max_seq_len bounds the contexts (default: the block table's capacity) and
     sizes the partials' workspace (grow-only scratch unless given).
+    tiles: build_prefill_tiles' table for these tokens.
     """
-    if query.is_cuda and output is not None and not split_keys and layout in _IS_VLLM \
+    if query.is_cuda and output is not None and layout in _IS_VLLM \
+            and (not split_keys or (max_seq_len and workspace is not None)) \
             and _lib.host().prefill(query, key_cache, value_cache, block_table, token_to_seq,
-                                    positions, output, _IS_VLLM[layout], scale,
+                                    positions, output, _IS_VLLM[layout], scale, tiles,
+                                    split_keys, max_seq_len, workspace,
                                     _lib.stream_handle(stream)) is True:
         return output
     _require_gpu(query, key_cache, value_cache, block_table, token_to_seq, positions, output)
@@ -679,14 +682,17 @@ def paged_prefill(query: torch.Tensor, key_cache: torch.Tensor, value_cache: tor
     p = make_params(key_cache=key_cache, value_cache=value_cache, layout=layout,
                     num_query_heads=query.shape[1], scale=scale, num_seqs=block_table.shape[0],
                     max_blocks_per_seq=block_table.shape[1], query=query, output=output)
-    if not split_keys:
+    if tiles is not None and (tiles.dtype != torch.int32 or tiles.dim() != 2 or tiles.shape[1] != 2
+                              or not tiles.is_contiguous() or tiles.device != query.device):
+        raise ValueError("tiles must be a contiguous int32 [n, 2] tensor on the query's device")
+    if not split_keys and tiles is None:
         _lib.call("vaa_paged_attention_prefill", ctypes.byref(p), query.data_ptr(),
                   key_cache.data_ptr(), value_cache.data_ptr(), block_table.data_ptr(),
                   token_to_seq.data_ptr(), positions.data_ptr(), output.data_ptr(), num_tokens,
                   _lib.stream_handle(stream))
         return output
     p.max_seq_len = int(max_seq_len) if max_seq_len else block_table.shape[1] * p.block_size
-    nbytes = prefill_workspace_size(p, num_tokens, split_keys)
+    nbytes = prefill_workspace_size(p, num_tokens, split_keys) if split_keys else 0
     ws_ptr = None
     if nbytes:
         if workspace is None:
@@ -694,6 +700,13 @@ def paged_prefill(query: torch.Tensor, key_cache: torch.Tensor, value_cache: tor
         if workspace.numel() * workspace.element_size() < nbytes:
             raise ValueError(f"workspace smaller than {nbytes} bytes")
         ws_ptr = workspace.data_ptr()
+    if tiles is not None:
+        _lib.call("vaa_paged_attention_prefill_tiles", ctypes.byref(p), query.data_ptr(),
+                  key_cache.data_ptr(), value_cache.data_ptr(), block_table.data_ptr(),
+                  token_to_seq.data_ptr(), positions.data_ptr(), output.data_ptr(), num_tokens,
+                  tiles.data_ptr(), tiles.shape[0], int(split_keys), ws_ptr, nbytes,
+                  _lib.stream_handle(stream))
+        return output
     _lib.call("vaa_paged_attention_prefill_split", ctypes.byref(p), query.data_ptr(),
               key_cache.data_ptr(), value_cache.data_ptr(), block_table.data_ptr(),
               token_to_seq.data_ptr(), positions.data_ptr(), output.data_ptr(), num_tokens,
@@ -740,6 +753,31 @@ def build_token_index(query_start_loc: torch.Tensor, seq_lens: torch.Tensor, num
     _lib.call("vaa_build_token_index", query_start_loc.data_ptr(), seq_lens.data_ptr(), num_seqs,
               num_tokens, tok.data_ptr(), pos.data_ptr(), _lib.stream_handle(stream))
     return tok, pos
+
+
+def build_prefill_tiles(query_start_loc: torch.Tensor, seq_lens: torch.Tensor, first_token: int,
+                        num_tokens: int, queries_per_kv: int, stream=None) -> tuple | None:
+    """(token_to_seq, positions, tiles) of the tokens [first_token, first_token +
+    num_tokens) of a step, whose sequences' starts (one more entry than sequences)
+    and lengths are given: the indices count tokens from first_token and sequences
+    from the first given, and each tile holds tokens of one sequence.  None for
+    more than 1024 sequences."""
+    _require_gpu(query_start_loc, seq_lens)
+    for t, n in ((query_start_loc, "query_start_loc"), (seq_lens, "seq_lens")):
+        if t.dtype != torch.int32 or not t.is_contiguous():
+            raise ValueError(f"{n} must be a contiguous int32 tensor")
+    num_seqs = query_start_loc.numel() - 1
+    if num_seqs < 0 or seq_lens.numel() < num_seqs:
+        raise ValueError("query_start_loc must have num_seqs + 1 entries")
+    nt = int(_lib.load().vaa_prefill_tile_count(num_tokens, num_seqs, queries_per_kv))
+    if nt <= 0:
+        return None
+    buf = torch.empty(2 * (num_tokens + nt), dtype=torch.int32, device=query_start_loc.device)
+    tok, pos, tiles = buf.split([num_tokens, num_tokens, 2 * nt])
+    _lib.call("vaa_build_prefill_tiles", query_start_loc.data_ptr(), seq_lens.data_ptr(), num_seqs,
+              first_token, num_tokens, queries_per_kv, tok.data_ptr(), pos.data_ptr(),
+              tiles.data_ptr(), nt, _lib.stream_handle(stream))
+    return tok, pos, tiles.view(nt, 2)
 
 
 def build_slot_mapping(block_table: torch.Tensor, block_size: int, token_to_seq: torch.Tensor,
