@@ -1,6 +1,10 @@
 """The wrappers' native host path (csrc/host_calls.cpp): on the GPU, every form
 of call gives the same bits and the same errors with it as without it; on the
 CPU, it declines whatever is not a GPU tensor."""
+import ctypes
+import shutil
+import subprocess
+
 import pytest
 import torch
 
@@ -20,6 +24,132 @@ def test_declines_other_objects(name):
         assert fn(*[a] * COUNTS[name]) is False
     with pytest.raises(TypeError):
         fn(t)
+
+
+# Entry points that only count their calls; every size query asks for 64 bytes.
+_STUB = """
+#include <stddef.h>
+int calls;
+int vaa_topk_workspace_size(int t, int v, int k, size_t* n) { *n = 64; return 0; }
+""" + "".join(f"size_t {f}() {{ return 64; }}\n" for f in (
+    "decode_workspace", "prefill_workspace", "step_workspace", "gate_workspace",
+    "linear_workspace", "no_cache_workspace")) + "int launch() { ++calls; return 0; }\n"
+_STUB_NAMES = {
+    "decode_workspace": ["vaa_paged_attention_decode_workspace_size"],
+    "prefill_workspace": ["vaa_paged_attention_prefill_workspace_size"],
+    "step_workspace": ["vaa_prefill_step_workspace_size"],
+    "gate_workspace": ["vaa_gate_up_silu_workspace_size"],
+    "linear_workspace": ["vaa_linear_workspace_size"],
+    "no_cache_workspace": ["vaa_attention_no_cache_workspace_size"],
+    "launch": ["vaa_kv_write_slots", "vaa_paged_attention_decode", "vaa_paged_attention_prefill",
+               "vaa_paged_attention_prefill_split", "vaa_paged_attention_prefill_tiles",
+               "vaa_prefill_step", "vaa_rmsnorm", "vaa_add_rmsnorm", "vaa_silu_mul",
+               "vaa_qkv_epilogue", "vaa_topk_logits", "vaa_gate_up_silu_split", "vaa_linear",
+               "vaa_attention_no_cache"]}
+
+
+@pytest.fixture(scope="module")
+def stub_lib(tmp_path_factory):
+    if shutil.which("gcc") is None:
+        pytest.skip("gcc not available")
+    d = tmp_path_factory.mktemp("stub")
+    so = d / "stub.so"
+    (d / "stub.c").write_text(_STUB)
+    alias = [f"-Wl,--defsym={n}={f}" for f, ns in _STUB_NAMES.items() for n in ns]
+    subprocess.run(["gcc", "-shared", "-fPIC", str(d / "stub.c"), "-o", str(so), *alias],
+                   check=True)
+    return ctypes.CDLL(str(so))
+
+
+@pytest.fixture
+def stub(stub_lib):
+    """The native path bound to entry points that launch nothing."""
+    host = _lib.host()
+    host.bind(stub_lib._handle)
+    yield host, ctypes.c_int.in_dll(stub_lib, "calls")
+    host.bind(_lib.load()._handle)
+
+
+_memory = ctypes.create_string_buffer(1 << 20)
+
+
+def _on(device, shape, dtype=torch.float16):
+    """A tensor that says it lives on cuda:`device` (its memory is the host's
+    and is never read)."""
+    base = (ctypes.addressof(_memory) + 255) // 256 * 256
+    storage = torch._C._construct_storage_from_data_pointer(
+        base, torch.device("cuda", device), len(_memory) - 256)
+    strides = [1] * len(shape)
+    for i in range(len(shape) - 1, 0, -1):
+        strides[i - 1] = strides[i] * shape[i]
+    return torch._C._construct_CUDA_Tensor_From_Storage_And_Metadata(
+        dict(dtype=dtype, device=torch.device("cuda", device), size=tuple(shape),
+             stride=tuple(strides), storage_offset=0), storage)
+
+
+def _apart(t, elements):
+    """The same tensor `elements` further on in the memory."""
+    return t.as_strided(t.shape, t.stride(), elements)
+
+
+def _accepted(name, dev=lambda i: 0):
+    """Arguments that `name` takes whole; dev(i): the device of argument i."""
+    n, H, KV, D, i32, i64 = 4, 4, 2, 64, torch.int32, torch.int64
+
+    def t(i, *shape, dtype=torch.float16):
+        return _on(dev(i), shape, dtype)
+    ws = lambda i: t(i, 64, dtype=torch.uint8)  # noqa: E731
+    kv = lambda i: t(i, 8, 16, KV, D)  # noqa: E731
+    if name == "norm":
+        return [t(0, n, D), t(1, D), t(2, n, D), t(3, n, D), 1e-5, 0, False]
+    if name == "silu":
+        return [t(0, n, D), t(1, n, D), t(2, n, D), 0]
+    if name == "epilogue":
+        return [t(0, n, H, D), t(1, n, KV, D), t(2, n, KV, D), t(3, n, dtype=i32),
+                t(4, 9, D // 2, dtype=torch.float32), t(5, 9, D // 2, dtype=torch.float32),
+                t(6, n, dtype=i64), kv(7), kv(8), t(9, (H + 2 * KV) * D), D, True, 0]
+    if name == "topk":
+        return [t(0, n, 9000), 5, t(2, n, 5, dtype=i32), t(3, n, 5), ws(4), 0]
+    if name == "gate_up":
+        return [t(0, n, D), t(1, 128, D), t(2, 128, D), t(3, n, 128), ws(4), 0]
+    if name == "linear":
+        return [t(0, n, D), t(1, 128, D), t(2, n, 128), ws(3), 0]
+    if name == "kv_write":
+        return [t(0, n, KV, D), t(1, n, KV, D), kv(2), kv(3), t(4, n, dtype=i64), True, 0]
+    if name == "decode":
+        return [t(0, n, H, D), kv(1), kv(2), t(3, n, 3, dtype=i32), t(4, n, dtype=i32),
+                t(5, n, H, D), t(6, n, KV, D), t(7, n, KV, D), True, 0.1, 40, 0, ws(12), 0]
+    if name == "step_decode":
+        return [t(0, n, H, D), t(1, n, KV, D), t(2, n, KV, D), t(3, 2, 8, 16, KV, D),
+                t(4, n, H, D), t(5, n, 3, dtype=i32), t(6, n, dtype=i32), t(7, n, dtype=i64), n,
+                True, D, 0.1, 40, 0, ws(14), 0]
+    if name == "step_prefill":
+        return [t(0, n, H, D), t(1, n, KV, D), t(2, n, KV, D), t(3, 2, 8, 16, KV, D),
+                t(4, n, H, D), t(5, 2, 3, dtype=i32), t(6, 2, dtype=i32), t(7, n, dtype=i64),
+                t(8, 3, dtype=i32), n, True, D, 0.1, True, ws(14), 0]
+    if name == "prefill":
+        return [t(0, n, H, D), kv(1), kv(2), t(3, 2, 3, dtype=i32), t(4, n, dtype=i32),
+                t(5, n, dtype=i32), t(6, n, H, D), True, 0.1, t(9, 2, 2, dtype=i32), 64, 40,
+                ws(12), 0]
+    return [t(0, n, H, D), t(1, n, KV, D), t(2, n, KV, D), _apart(t(3, n, H, D), 4096),
+            t(4, 3, dtype=i32), n, 2, D, 0.1, 3, False, ws(11), 0]
+
+
+@pytest.mark.parametrize("name", NAMES)
+def test_tensors_of_two_devices_are_declined(stub, name):
+    """A call whose tensors are on one device is taken; with any one of them on
+    another device nothing is launched."""
+    host, calls = stub
+    fn, args = getattr(host, name), _accepted(name)
+    assert len(args) == COUNTS[name]
+    assert fn(*args) is True
+    for i, a in enumerate(args):
+        if not isinstance(a, torch.Tensor):
+            continue
+        calls.value = 0
+        done = fn(*_accepted(name, lambda j, i=i: int(j == i)))
+        assert done is not True and calls.value == 0, f"argument {i}"
+    assert fn(*_accepted(name, lambda j: 1)) is True
 
 
 class _Declines:

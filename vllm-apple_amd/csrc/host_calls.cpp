@@ -16,6 +16,8 @@
 #include <dlfcn.h>
 #include <torch/csrc/autograd/python_variable.h>
 
+#include <initializer_list>
+
 #include "vllm_apple_amd.h"
 
 namespace {
@@ -46,6 +48,21 @@ void* ptr(const Tensor& t) { return const_cast<void*>(t.const_data_ptr()); }
 uint16_t* p16(const Tensor& t) { return static_cast<uint16_t*>(ptr(t)); }
 
 bool on_gpu(const Tensor& t) { return t.is_cuda() && t.layout() == at::kStrided; }
+// Whether the tensors (null: absent) are all on one device.  A kernel given
+// another device's pointers would read them over the peer mapping or fault.
+bool one_device(std::initializer_list<const Tensor*> ts) {
+  const Tensor* first = nullptr;
+  for (const Tensor* t : ts) {
+    if (!t) continue;
+    if (!first) first = t;
+    if (t->device() != first->device()) return false;
+  }
+  return true;
+}
+// Whether ws is a workspace of `need` bytes on the tensor's device.
+bool room(const Tensor* ws, size_t need, const Tensor& like) {
+  return ws && on_gpu(*ws) && ws->device() == like.device() && ws->nbytes() >= need;
+}
 
 // VAA_DTYPE_* of a GPU tensor of the two 16-bit types, else -1.
 int dt16(const Tensor& t) {
@@ -143,7 +160,8 @@ PyObject* guarded(PyObject*, PyObject* const* args, Py_ssize_t n) {
 PyObject* norm(const Args& a) {
   const Tensor *x = a.t(0), *w = a.t(1), *r = a.t(2), *o = a.t(3);
   const bool add = a.b(6);
-  if (!x || !w || !o || !none_or_ten(a.a[2]) || (add && !r)) Py_RETURN_FALSE;
+  if (!x || !w || !o || !none_or_ten(a.a[2]) || (add && !r) || !one_device({x, w, r, o}))
+    Py_RETURN_FALSE;
   const int dt = dt16(*x);
   if (dt < 0 || dt16(*w) != dt || dt16(*o) != dt || (r && dt16(*r) != dt)) Py_RETURN_FALSE;
   if (x->dim() != 2 || x->stride(1) != 1 || !w->is_contiguous() || w->numel() != x->size(1) ||
@@ -163,7 +181,7 @@ PyObject* norm(const Args& a) {
 // (gate, up, out, stream): contiguous tensors
 PyObject* silu(const Args& a) {
   const Tensor *g = a.t(0), *u = a.t(1), *o = a.t(2);
-  if (!g || !u || !o) Py_RETURN_FALSE;
+  if (!g || !u || !o || !one_device({g, u, o})) Py_RETURN_FALSE;
   const int dt = dt16(*g);
   if (dt < 0 || dt16(*u) != dt || dt16(*o) != dt || g->sizes() != u->sizes() ||
       o->sizes() != g->sizes() || !g->is_contiguous() || !u->is_contiguous() ||
@@ -176,7 +194,8 @@ PyObject* silu(const Args& a) {
 PyObject* epilogue(const Args& a) {
   const Tensor *q = a.t(0), *k = a.t(1), *v = a.t(2), *pos = a.t(3), *c = a.t(4), *s = a.t(5),
                *sl = a.t(6), *kc = a.t(7), *vc = a.t(8), *b = a.t(9);
-  if (!q || !k || !v || !pos || !c || !s || !sl || !kc || !vc || !none_or_ten(a.a[9]))
+  if (!q || !k || !v || !pos || !c || !s || !sl || !kc || !vc || !none_or_ten(a.a[9]) ||
+      !one_device({q, k, v, pos, c, s, sl, kc, vc, b}))
     Py_RETURN_FALSE;
   const int dt = dt16(*q);
   if (dt < 0 || dt16(*k) != dt || dt16(*v) != dt || dt16(*kc) != dt || dt16(*vc) != dt ||
@@ -211,7 +230,8 @@ PyObject* epilogue(const Args& a) {
 // (logits, k, indices, values, workspace or None, stream)
 PyObject* topk(const Args& a) {
   const Tensor *x = a.t(0), *idx = a.t(2), *val = a.t(3), *ws = a.t(4);
-  if (!x || !idx || !val || !none_or_ten(a.a[4])) Py_RETURN_FALSE;
+  if (!x || !idx || !val || !none_or_ten(a.a[4]) || !one_device({x, idx, val, ws}))
+    Py_RETURN_FALSE;
   const int64_t k = a.i(1);
   if (dt16(*x) < 0 || dt16(*val) != dt16(*x) || x->dim() != 2 || x->stride(1) != 1 ||
       !on_gpu(*idx) || idx->scalar_type() != at::kInt || idx->dim() != 2 || val->dim() != 2 ||
@@ -221,7 +241,7 @@ PyObject* topk(const Args& a) {
     Py_RETURN_FALSE;
   size_t need = 0;
   if (p_vaa_topk_workspace_size(x->size(0), x->size(1), k, &need) != VAA_OK) Py_RETURN_FALSE;
-  if (need && (!ws || !on_gpu(*ws) || ws->nbytes() < need)) return PyLong_FromSize_t(need);
+  if (need && !room(ws, need, *x)) return PyLong_FromSize_t(need);
   return yes(p_vaa_topk_logits(p16(*x), x->size(0), x->size(1), x->stride(0), k,
                                static_cast<int32_t*>(ptr(*idx)), p16(*val), idx->stride(0),
                                ws ? ptr(*ws) : nullptr, ws ? ws->nbytes() : 0, a.s(5)));
@@ -236,7 +256,9 @@ bool mat16(const Tensor& t, int dt) {
 // None, stream)
 PyObject* gate_up(const Args& a) {
   const Tensor *x = a.t(0), *g = a.t(1), *u = a.t(2), *o = a.t(3), *ws = a.t(4);
-  if (!x || !g || !o || !none_or_ten(a.a[2]) || !none_or_ten(a.a[4])) Py_RETURN_FALSE;
+  if (!x || !g || !o || !none_or_ten(a.a[2]) || !none_or_ten(a.a[4]) ||
+      !one_device({x, g, u, o}))
+    Py_RETURN_FALSE;
   const int dt = dt16(*x);
   if (dt < 0 || !mat16(*x, dt) || !mat16(*g, dt) || !mat16(*o, dt) || (u && !mat16(*u, dt)))
     Py_RETURN_FALSE;
@@ -253,7 +275,7 @@ PyObject* gate_up(const Args& a) {
   }
   if (g->size(1) != H || o->size(0) != T || o->size(1) != I) Py_RETURN_FALSE;
   const size_t need = p_vaa_gate_up_silu_workspace_size(T, H, I);
-  if (need && (!ws || !on_gpu(*ws) || ws->nbytes() < need)) return PyLong_FromSize_t(need);
+  if (need && !room(ws, need, *x)) return PyLong_FromSize_t(need);
   return yes(p_vaa_gate_up_silu_split(p16(*x), x->stride(0), p16(*g), up, g->stride(0), p16(*o),
                                       o->stride(0), T, H, I, dt, ws ? ptr(*ws) : nullptr,
                                       ws ? ws->nbytes() : 0, a.s(5)));
@@ -262,14 +284,14 @@ PyObject* gate_up(const Args& a) {
 // (x, weight, out, workspace or None, stream); what linear_ok accepts.
 PyObject* linear(const Args& a) {
   const Tensor *x = a.t(0), *w = a.t(1), *o = a.t(2), *ws = a.t(3);
-  if (!x || !w || !o || !none_or_ten(a.a[3])) Py_RETURN_FALSE;
+  if (!x || !w || !o || !none_or_ten(a.a[3]) || !one_device({x, w, o})) Py_RETURN_FALSE;
   const int dt = dt16(*x);
   if (dt < 0 || !mat16(*x, dt) || !mat16(*w, dt) || !mat16(*o, dt)) Py_RETURN_FALSE;
   const int64_t T = x->size(0), K = x->size(1), N = w->size(0);
   if (w->size(1) != K || o->size(0) != T || o->size(1) != N) Py_RETURN_FALSE;
   const size_t need = p_vaa_linear_workspace_size(T, K, N);
   if (!need) Py_RETURN_FALSE;
-  if (!ws || !on_gpu(*ws) || ws->nbytes() < need) return PyLong_FromSize_t(need);
+  if (!room(ws, need, *x)) return PyLong_FromSize_t(need);
   return yes(p_vaa_linear(p16(*x), x->stride(0), p16(*w), w->stride(0), p16(*o),
                                 o->stride(0), T, K, N, dt, ptr(*ws), ws->nbytes(), a.s(4)));
 }
@@ -294,7 +316,7 @@ int write_rows(vaa_attn_params p, const Tensor& k, const Tensor& v, uint16_t* kc
 // (key, value, key_cache, value_cache, slots, vllm, stream)
 PyObject* kv_write(const Args& a) {
   const Tensor *k = a.t(0), *v = a.t(1), *kc = a.t(2), *vc = a.t(3), *sl = a.t(4);
-  if (!k || !v || !kc || !vc || !sl) Py_RETURN_FALSE;
+  if (!k || !v || !kc || !vc || !sl || !one_device({k, v, kc, vc, sl})) Py_RETURN_FALSE;
   const int dt = dt16(*k);
   vaa_attn_params p{};
   if (dt < 0 || dt16(*v) != dt || dt16(*kc) != dt || dt16(*vc) != dt || k->dim() != 3 ||
@@ -333,7 +355,7 @@ PyObject* decode(const Args& a) {
   const Tensor *q = a.t(0), *kc = a.t(1), *vc = a.t(2), *bt = a.t(3), *sl = a.t(4), *o = a.t(5),
                *nk = a.t(6), *nv = a.t(7), *ws = a.t(12);
   if (!q || !kc || !vc || !bt || !sl || !o || !none_or_ten(a.a[6]) || !none_or_ten(a.a[7]) ||
-      !none_or_ten(a.a[12]) || !nk != !nv)
+      !none_or_ten(a.a[12]) || !nk != !nv || !one_device({q, kc, vc, bt, sl, o, nk, nv}))
     Py_RETURN_FALSE;
   const int dt = dt16(*q);
   vaa_attn_params p{};
@@ -353,7 +375,7 @@ PyObject* decode(const Args& a) {
   }
   p.dtype = dt;
   const size_t need = p_vaa_paged_attention_decode_workspace_size(&p, nullptr);
-  if (need && (!ws || !on_gpu(*ws) || ws->nbytes() < need)) return PyLong_FromSize_t(need);
+  if (need && !room(ws, need, *q)) return PyLong_FromSize_t(need);
   return yes(p_vaa_paged_attention_decode(
       &p, p16(*q), p16(*kc), p16(*vc), static_cast<int32_t*>(ptr(*bt)),
       static_cast<int32_t*>(ptr(*sl)), p16(*o), nk ? p16(*nk) : nullptr, nv ? p16(*nv) : nullptr,
@@ -385,7 +407,8 @@ PyObject* step_decode(const Args& a) {
   const Tensor *q = a.t(0), *k = a.t(1), *v = a.t(2), *c = a.t(3), *o = a.t(4), *bt = a.t(5),
                *sl = a.t(6), *slots = a.t(7), *ws = a.t(14);
   const bool write = a.b(9);
-  if (!q || !c || !o || !bt || !sl || (write && (!k || !v || !slots)) || !none_or_ten(a.a[14]))
+  if (!q || !c || !o || !bt || !sl || (write && (!k || !v || !slots)) || !none_or_ten(a.a[14]) ||
+      !one_device({q, c, o, bt, sl}) || (write && !one_device({q, k, v, slots})))
     Py_RETURN_FALSE;
   const int dt = dt16(*q);
   const int64_t n = a.i(8);
@@ -398,7 +421,7 @@ PyObject* step_decode(const Args& a) {
     Py_RETURN_FALSE;
   p.dtype = dt;
   const size_t need = p_vaa_paged_attention_decode_workspace_size(&p, nullptr);
-  if (need && (!ws || !on_gpu(*ws) || ws->nbytes() < need)) return PyLong_FromSize_t(need);
+  if (need && !room(ws, need, *q)) return PyLong_FromSize_t(need);
   if (write && write_rows(p, *k, *v, kc, vc, *slots, n, a.s(15))) Py_RETURN_FALSE;
   return yes(p_vaa_paged_attention_decode(&p, p16(*q), kc, vc, static_cast<int32_t*>(ptr(*bt)),
                                           static_cast<int32_t*>(ptr(*sl)), p16(*o), nullptr,
@@ -433,7 +456,8 @@ PyObject* step_prefill(const Args& a) {
                *sl = a.t(6), *slots = a.t(7), *qsl = a.t(8), *ws = a.t(14);
   const bool write = a.b(10);
   if (!q || !c || !o || !bt || !sl || !qsl || (write && (!k || !v || !slots)) ||
-      !none_or_ten(a.a[14]))
+      !none_or_ten(a.a[14]) || !one_device({q, c, o, bt, sl, qsl}) ||
+      (write && !one_device({q, k, v, slots})))
     Py_RETURN_FALSE;
   const int dt = dt16(*q);
   const int64_t n = a.i(9);
@@ -457,7 +481,7 @@ PyObject* step_prefill(const Args& a) {
   }
   const int S = static_cast<int>(qsl->numel() - 1);
   const size_t need = p_vaa_prefill_step_workspace_size(&p, n, S);
-  if (!ws || !on_gpu(*ws) || ws->nbytes() < need) return PyLong_FromSize_t(need);
+  if (!room(ws, need, *q)) return PyLong_FromSize_t(need);
   return yes(p_vaa_prefill_step(&p, p16(*q), kc, vc, static_cast<int32_t*>(ptr(*bt)),
                                 static_cast<int32_t*>(ptr(*sl)),
                                 static_cast<int32_t*>(ptr(*qsl)), S, write ? p16(*k) : nullptr,
@@ -471,7 +495,7 @@ PyObject* prefill(const Args& a) {
   const Tensor *q = a.t(0), *kc = a.t(1), *vc = a.t(2), *bt = a.t(3), *tok = a.t(4),
                *pos = a.t(5), *o = a.t(6), *tiles = a.t(9), *ws = a.t(12);
   if (!q || !kc || !vc || !bt || !tok || !pos || !o || !none_or_ten(a.a[9]) ||
-      !none_or_ten(a.a[12]))
+      !none_or_ten(a.a[12]) || !one_device({q, kc, vc, bt, tok, pos, o, tiles}))
     Py_RETURN_FALSE;
   const int dt = dt16(*q);
   const int64_t split = a.i(10), max_len = a.i(11);
@@ -489,7 +513,7 @@ PyObject* prefill(const Args& a) {
   if (split) {
     p.max_seq_len = max_len;
     need = p_vaa_paged_attention_prefill_workspace_size(&p, n, split);
-    if (need && (!ws || !on_gpu(*ws) || ws->nbytes() < need)) return PyLong_FromSize_t(need);
+    if (need && !room(ws, need, *q)) return PyLong_FromSize_t(need);
   }
   auto* btp = static_cast<int32_t*>(ptr(*bt));
   auto* tp = static_cast<int32_t*>(ptr(*tok));
@@ -527,7 +551,8 @@ bool overlap(const Tensor& a, const Tensor& b, int64_t T) {
 //  max_seq_len, causal, workspace or None, stream)
 PyObject* no_cache(const Args& a) {
   const Tensor *q = a.t(0), *k = a.t(1), *v = a.t(2), *o = a.t(3), *qsl = a.t(4), *ws = a.t(11);
-  if (!q || !k || !v || !o || !qsl || !none_or_ten(a.a[11])) Py_RETURN_FALSE;
+  if (!q || !k || !v || !o || !qsl || !none_or_ten(a.a[11]) || !one_device({q, k, v, o, qsl}))
+    Py_RETURN_FALSE;
   const int dt = dt16(*q);
   const int64_t T = a.i(5), S = a.i(6), L = a.i(9);
   if (dt < 0 || dt16(*k) != dt || dt16(*v) != dt || dt16(*o) != dt || !small(T) || T == 0 ||
@@ -537,8 +562,7 @@ PyObject* no_cache(const Args& a) {
     if (!aligned_rows(*t) || t->size(0) < T || t->size(2) != a.i(7) || t->size(1) == 0)
       Py_RETURN_FALSE;
   if (k->sizes() != v->sizes() || k->strides() != v->strides() || o->size(1) != q->size(1) ||
-      q->size(1) % k->size(1) || qsl->get_device() != q->get_device() || overlap(*o, *k, T) ||
-      overlap(*o, *v, T))
+      q->size(1) % k->size(1) || overlap(*o, *k, T) || overlap(*o, *v, T))
     Py_RETURN_FALSE;
   vaa_attn_params p{};
   p.dtype = dt;
@@ -556,7 +580,7 @@ PyObject* no_cache(const Args& a) {
   p.o_stride_token = o->stride(0);
   p.o_stride_head = o->stride(1);
   const size_t need = p_vaa_attention_no_cache_workspace_size(S, T, L);
-  if (!ws || !on_gpu(*ws) || ws->nbytes() < need) return PyLong_FromSize_t(need);
+  if (!room(ws, need, *q)) return PyLong_FromSize_t(need);
   return yes(p_vaa_attention_no_cache(&p, p16(*q), p16(*k), p16(*v),
                                       static_cast<int32_t*>(ptr(*qsl)), p16(*o), T, a.b(10),
                                       ptr(*ws), ws->nbytes(), a.s(12)));
