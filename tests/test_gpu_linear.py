@@ -96,3 +96,47 @@ def test_linear_strided_rows_and_refusals(gpu):
     assert not kernels.linear_ok(x.bfloat16(), w, out)             # two types
     with pytest.raises(ValueError):
         kernels.linear(x, w[:200], out[:, :200])
+
+
+@pytest.mark.parametrize("which", ["down_proj", "out"])
+def test_mlp_refuses_gradients_as_the_library_product_does(gpu, which):
+    """encode writes into a given buffer, which autograd cannot follow: a down
+    projection or output that needs a gradient is refused while gradients are
+    on, by the own product as by torch.matmul, and taken without them.  A
+    forward-mode tangent goes to torch.matmul too, and the output's version
+    moves either way."""
+    import torch.autograd.forward_ad as fwd
+
+    from vllm_apple_amd.engine import EngineMLP
+
+    H, I, T = 256, 512, 5
+    g = torch.Generator().manual_seed(3)
+    x, w1, w2 = ((torch.randn(s, generator=g) * 0.1).half().cuda()
+                 for s in ((T, H), (2 * I, H), (H, I)))
+    out = torch.zeros(T, H, dtype=torch.float16, device="cuda")
+    m = EngineMLP(None, H, I)
+    m.set_weights(gate_up_proj=w1, down_proj=w2)
+    m.encode(None, x, out, T)
+    want, version = out.clone(), out._version
+    m.encode(None, x, out, T)
+    assert torch.equal(out, want) and out._version > version
+    with fwd.dual_level():
+        dual = fwd.make_dual(w2, torch.ones_like(w2))
+        kinds = []
+        m.set_weights(gate_up_proj=w1, down_proj=dual)
+        act = torch.zeros(T, I, dtype=torch.float16, device="cuda")
+        for call in (lambda: torch.matmul(act, dual.t(), out=out),
+                     lambda: m.encode(None, x, out, T)):
+            try:
+                call()
+                kinds.append(None)
+            except Exception as e:  # noqa: BLE001
+                kinds.append(type(e))
+        assert kinds[0] == kinds[1]
+    m.set_weights(gate_up_proj=w1, down_proj=w2)
+    (w2 if which == "down_proj" else out).requires_grad_()
+    with pytest.raises(RuntimeError, match="automatic differentiation"):
+        m.encode(None, x, out, T)
+    with torch.no_grad():
+        m.encode(None, x, out, T)
+    assert torch.equal(out.detach(), want)

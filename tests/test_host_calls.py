@@ -152,6 +152,33 @@ def test_tensors_of_two_devices_are_declined(stub, name):
     assert fn(*_accepted(name, lambda j: 1)) is True
 
 
+def test_product_is_left_to_torch_where_it_would_do_more(stub):
+    """The product that stands in for torch.matmul(out=) declines what the
+    library call refuses or hands on: a gradient to record, a dispatch mode.  It
+    counts as a write to its output."""
+    from torch.utils._python_dispatch import TorchDispatchMode
+
+    host, calls = stub
+    for i in range(3):
+        args = _accepted("linear")
+        args[i].requires_grad_()
+        calls.value = 0
+        assert host.linear(*args) is False and calls.value == 0
+        with torch.no_grad():
+            assert host.linear(*args) is True
+    args = _accepted("linear")
+    version = args[2]._version
+    assert host.linear(*args) is True and args[2]._version == version + 1
+
+    class Sees(TorchDispatchMode):
+        def __torch_dispatch__(self, func, types, args=(), kwargs=None):
+            return func(*args, **(kwargs or {}))
+    args = _accepted("linear")
+    with Sees():
+        assert host.linear(*args) is False
+    assert host.linear(*args) is True
+
+
 class _Declines:
     """A native path that declines everything: the wrappers' own path runs."""
 

@@ -14,6 +14,8 @@
 #define PY_SSIZE_T_CLEAN
 #include <Python.h>
 #include <dlfcn.h>
+#include <c10/core/GradMode.h>
+#include <c10/core/impl/TorchDispatchModeTLS.h>
 #include <torch/csrc/autograd/python_variable.h>
 
 #include <initializer_list>
@@ -281,10 +283,29 @@ PyObject* gate_up(const Args& a) {
                                       ws ? ws->nbytes() : 0, a.s(5)));
 }
 
-// (x, weight, out, workspace or None, stream); what linear_ok accepts.
+// Whether torch.matmul(out=) would do nothing but the product on these: no
+// gradient to record or refuse (reverse or forward mode), no tensor whose
+// operations Python or a transform implements, no dispatch mode that would see
+// the call.
+bool plain_matmul(std::initializer_list<const Tensor*> ts) {
+  if (c10::impl::dispatch_mode_enabled()) return false;
+  const bool grad = c10::GradMode::is_enabled();
+  for (const Tensor* t : ts)
+    if ((grad && t->requires_grad()) || t->_fw_grad(0).defined() ||
+        t->key_set().has_any(c10::DispatchKeySet({c10::DispatchKey::Python,
+                                                  c10::DispatchKey::FuncTorchBatched,
+                                                  c10::DispatchKey::FuncTorchGradWrapper})))
+      return false;
+  return true;
+}
+
+// (x, weight, out, workspace or None, stream); what linear_ok accepts, in a call
+// that stands in for torch.matmul(out=): like it, it counts as a write to out.
 PyObject* linear(const Args& a) {
   const Tensor *x = a.t(0), *w = a.t(1), *o = a.t(2), *ws = a.t(3);
-  if (!x || !w || !o || !none_or_ten(a.a[3]) || !one_device({x, w, o})) Py_RETURN_FALSE;
+  if (!x || !w || !o || !none_or_ten(a.a[3]) || !one_device({x, w, o}) ||
+      !plain_matmul({x, w, o}))
+    Py_RETURN_FALSE;
   const int dt = dt16(*x);
   if (dt < 0 || !mat16(*x, dt) || !mat16(*w, dt) || !mat16(*o, dt)) Py_RETURN_FALSE;
   const int64_t T = x->size(0), K = x->size(1), N = w->size(0);
@@ -292,8 +313,12 @@ PyObject* linear(const Args& a) {
   const size_t need = p_vaa_linear_workspace_size(T, K, N);
   if (!need) Py_RETURN_FALSE;
   if (!room(ws, need, *x)) return PyLong_FromSize_t(need);
-  return yes(p_vaa_linear(p16(*x), x->stride(0), p16(*w), w->stride(0), p16(*o),
-                                o->stride(0), T, K, N, dt, ptr(*ws), ws->nbytes(), a.s(4)));
+  void* const stream = a.s(4);
+  if (p_vaa_linear(p16(*x), x->stride(0), p16(*w), w->stride(0), p16(*o), o->stride(0), T, K, N,
+                   dt, ptr(*ws), ws->nbytes(), stream) != VAA_OK)
+    Py_RETURN_FALSE;
+  if (!o->is_inference()) o->unsafeGetTensorImpl()->bump_version();
+  Py_RETURN_TRUE;
 }
 
 // ------------------------------------------------------------ attention --
