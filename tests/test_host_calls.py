@@ -4,6 +4,7 @@ CPU, it declines whatever is not a GPU tensor."""
 import ctypes
 import shutil
 import subprocess
+import threading
 
 import pytest
 import torch
@@ -29,11 +30,20 @@ def test_declines_other_objects(name):
 # Entry points that only count their calls; every size query asks for 64 bytes.
 _STUB = """
 #include <stddef.h>
-int calls;
+#include <unistd.h>
+int calls, delay_ms, inside;
 int vaa_topk_workspace_size(int t, int v, int k, size_t* n) { *n = 64; return 0; }
 """ + "".join(f"size_t {f}() {{ return 64; }}\n" for f in (
     "decode_workspace", "prefill_workspace", "step_workspace", "gate_workspace",
-    "linear_workspace", "no_cache_workspace")) + "int launch() { ++calls; return 0; }\n"
+    "linear_workspace", "no_cache_workspace")) + """
+int launch() {
+  ++calls;
+  inside = 1;
+  usleep(1000 * delay_ms);
+  inside = 0;
+  return 0;
+}
+"""
 _STUB_NAMES = {
     "decode_workspace": ["vaa_paged_attention_decode_workspace_size"],
     "prefill_workspace": ["vaa_paged_attention_prefill_workspace_size"],
@@ -67,6 +77,7 @@ def stub(stub_lib):
     host = _lib.host()
     host.bind(stub_lib._handle)
     yield host, ctypes.c_int.in_dll(stub_lib, "calls")
+    ctypes.c_int.in_dll(stub_lib, "delay_ms").value = 0
     host.bind(_lib.load()._handle)
 
 
@@ -177,6 +188,23 @@ def test_product_is_left_to_torch_where_it_would_do_more(stub):
     with Sees():
         assert host.linear(*args) is False
     assert host.linear(*args) is True
+
+
+@pytest.mark.parametrize("name", NAMES)
+def test_launches_leave_the_interpreter_to_other_threads(stub, stub_lib, name):
+    """While one thread's launch blocks (a full queue), another runs Python."""
+    host, _ = stub
+    ctypes.c_int.in_dll(stub_lib, "delay_ms").value = 150
+    inside = ctypes.c_int.in_dll(stub_lib, "inside")
+    done = []
+    worker = threading.Thread(
+        target=lambda: done.append(getattr(host, name)(*_accepted(name))))
+    worker.start()
+    seen = 0
+    while not done:
+        seen |= inside.value
+    worker.join()
+    assert done == [True] and seen == 1
 
 
 class _Declines:

@@ -118,6 +118,19 @@ bool same_rows(const Tensor& a, const Tensor& b) {
   return a.sizes() == b.sizes() && a.strides() == b.strides();
 }
 
+// Calls an entry point without the interpreter lock, as ctypes does: a launch
+// into a full queue blocks until the GPU takes one, and other Python threads run
+// meanwhile.  The arguments are evaluated by the caller, with the lock; the
+// tensors live as long as the caller's argument list.
+template <typename... P, typename... A>
+int launch(int (*f)(P...), A... args) {
+  struct Unlocked {
+    PyThreadState* state = PyEval_SaveThread();
+    ~Unlocked() { PyEval_RestoreThread(state); }
+  } unlocked;
+  return f(args...);
+}
+
 PyObject* yes(int status) {
   if (status != VAA_OK) Py_RETURN_FALSE;  // the wrapper repeats the call and raises
   Py_RETURN_TRUE;
@@ -173,11 +186,10 @@ PyObject* norm(const Args& a) {
     Py_RETURN_FALSE;
   const float eps = static_cast<float>(a.f(4));
   if (add)
-    return yes(p_vaa_add_rmsnorm(p16(*x), p16(*r), p16(*w), p16(*o), x->size(0), x->size(1),
-                                 x->stride(0), r->stride(0), o->stride(0), eps, dt, a.s(5)));
-  return yes(p_vaa_rmsnorm(p16(*x), p16(*o), p16(*w), r ? p16(*r) : nullptr, x->size(0),
-                           x->size(1), x->stride(0), o->stride(0), r ? r->stride(0) : 0, eps, dt,
-                           a.s(5)));
+    return yes(launch(p_vaa_add_rmsnorm, p16(*x), p16(*r), p16(*w), p16(*o), x->size(0), x->size(1),
+                      x->stride(0), r->stride(0), o->stride(0), eps, dt, a.s(5)));
+  return yes(launch(p_vaa_rmsnorm, p16(*x), p16(*o), p16(*w), r ? p16(*r) : nullptr, x->size(0),
+                    x->size(1), x->stride(0), o->stride(0), r ? r->stride(0) : 0, eps, dt, a.s(5)));
 }
 
 // (gate, up, out, stream): contiguous tensors
@@ -189,7 +201,7 @@ PyObject* silu(const Args& a) {
       o->sizes() != g->sizes() || !g->is_contiguous() || !u->is_contiguous() ||
       !o->is_contiguous())
     Py_RETURN_FALSE;
-  return yes(p_vaa_silu_mul(p16(*g), p16(*u), p16(*o), g->numel(), dt, a.s(3)));
+  return yes(launch(p_vaa_silu_mul, p16(*g), p16(*u), p16(*o), g->numel(), dt, a.s(3)));
 }
 
 // (q, k, v, pos, cos, sin, slots, k_cache, v_cache, bias or None, rot, vllm, stream)
@@ -223,10 +235,10 @@ PyObject* epilogue(const Args& a) {
   p.q_stride_head = q->stride(1);
   p.new_kv_stride_token = k->stride(0);
   p.new_kv_stride_head = k->stride(1);
-  return yes(p_vaa_qkv_epilogue(&p, p16(*q), p16(*k), p16(*v), b ? p16(*b) : nullptr,
-                                static_cast<float*>(ptr(*c)), static_cast<float*>(ptr(*s)), rot,
-                                c->size(0), static_cast<int32_t*>(ptr(*pos)), ptr(*sl),
-                                slot_type(*sl, T), p16(*kc), p16(*vc), T, a.s(12)));
+  return yes(launch(p_vaa_qkv_epilogue, &p, p16(*q), p16(*k), p16(*v), b ? p16(*b) : nullptr,
+                    static_cast<float*>(ptr(*c)), static_cast<float*>(ptr(*s)), rot, c->size(0),
+                    static_cast<int32_t*>(ptr(*pos)), ptr(*sl), slot_type(*sl, T), p16(*kc),
+                    p16(*vc), T, a.s(12)));
 }
 
 // (logits, k, indices, values, workspace or None, stream)
@@ -244,9 +256,9 @@ PyObject* topk(const Args& a) {
   size_t need = 0;
   if (p_vaa_topk_workspace_size(x->size(0), x->size(1), k, &need) != VAA_OK) Py_RETURN_FALSE;
   if (need && !room(ws, need, *x)) return PyLong_FromSize_t(need);
-  return yes(p_vaa_topk_logits(p16(*x), x->size(0), x->size(1), x->stride(0), k,
-                               static_cast<int32_t*>(ptr(*idx)), p16(*val), idx->stride(0),
-                               ws ? ptr(*ws) : nullptr, ws ? ws->nbytes() : 0, a.s(5)));
+  return yes(launch(p_vaa_topk_logits, p16(*x), x->size(0), x->size(1), x->stride(0), k,
+                    static_cast<int32_t*>(ptr(*idx)), p16(*val), idx->stride(0),
+                    ws ? ptr(*ws) : nullptr, ws ? ws->nbytes() : 0, a.s(5)));
 }
 
 bool mat16(const Tensor& t, int dt) {
@@ -278,9 +290,9 @@ PyObject* gate_up(const Args& a) {
   if (g->size(1) != H || o->size(0) != T || o->size(1) != I) Py_RETURN_FALSE;
   const size_t need = p_vaa_gate_up_silu_workspace_size(T, H, I);
   if (need && !room(ws, need, *x)) return PyLong_FromSize_t(need);
-  return yes(p_vaa_gate_up_silu_split(p16(*x), x->stride(0), p16(*g), up, g->stride(0), p16(*o),
-                                      o->stride(0), T, H, I, dt, ws ? ptr(*ws) : nullptr,
-                                      ws ? ws->nbytes() : 0, a.s(5)));
+  return yes(launch(p_vaa_gate_up_silu_split, p16(*x), x->stride(0), p16(*g), up, g->stride(0),
+                    p16(*o), o->stride(0), T, H, I, dt, ws ? ptr(*ws) : nullptr,
+                    ws ? ws->nbytes() : 0, a.s(5)));
 }
 
 // Whether torch.matmul(out=) would do nothing but the product on these: no
@@ -314,8 +326,8 @@ PyObject* linear(const Args& a) {
   if (!need) Py_RETURN_FALSE;
   if (!room(ws, need, *x)) return PyLong_FromSize_t(need);
   void* const stream = a.s(4);
-  if (p_vaa_linear(p16(*x), x->stride(0), p16(*w), w->stride(0), p16(*o), o->stride(0), T, K, N,
-                   dt, ptr(*ws), ws->nbytes(), stream) != VAA_OK)
+  if (launch(p_vaa_linear, p16(*x), x->stride(0), p16(*w), w->stride(0), p16(*o), o->stride(0), T,
+             K, N, dt, ptr(*ws), ws->nbytes(), stream) != VAA_OK)
     Py_RETURN_FALSE;
   if (!o->is_inference()) o->unsafeGetTensorImpl()->bump_version();
   Py_RETURN_TRUE;
@@ -335,7 +347,8 @@ int write_rows(vaa_attn_params p, const Tensor& k, const Tensor& v, uint16_t* kc
   p.scale = 1.f;
   p.new_kv_stride_token = k.stride(0);
   p.new_kv_stride_head = k.stride(1);
-  return p_vaa_kv_write_slots(&p, kc, vc, ptr(slots), it, p16(k), p16(v), n, stream) != VAA_OK;
+  return launch(p_vaa_kv_write_slots, &p, kc, vc, ptr(slots), it, p16(k), p16(v), n,
+                stream) != VAA_OK;
 }
 
 // (key, value, key_cache, value_cache, slots, vllm, stream)
@@ -401,10 +414,10 @@ PyObject* decode(const Args& a) {
   p.dtype = dt;
   const size_t need = p_vaa_paged_attention_decode_workspace_size(&p, nullptr);
   if (need && !room(ws, need, *q)) return PyLong_FromSize_t(need);
-  return yes(p_vaa_paged_attention_decode(
-      &p, p16(*q), p16(*kc), p16(*vc), static_cast<int32_t*>(ptr(*bt)),
-      static_cast<int32_t*>(ptr(*sl)), p16(*o), nk ? p16(*nk) : nullptr, nv ? p16(*nv) : nullptr,
-      need ? ptr(*ws) : nullptr, need ? ws->nbytes() : 0, a.s(13)));
+  return yes(launch(p_vaa_paged_attention_decode, &p, p16(*q), p16(*kc), p16(*vc),
+                    static_cast<int32_t*>(ptr(*bt)), static_cast<int32_t*>(ptr(*sl)), p16(*o),
+                    nk ? p16(*nk) : nullptr, nv ? p16(*nv) : nullptr, need ? ptr(*ws) : nullptr,
+                    need ? ws->nbytes() : 0, a.s(13)));
 }
 
 // Cache fields of p from vLLM's [2, nb, bs, KV, D] tensor.
@@ -448,10 +461,9 @@ PyObject* step_decode(const Args& a) {
   const size_t need = p_vaa_paged_attention_decode_workspace_size(&p, nullptr);
   if (need && !room(ws, need, *q)) return PyLong_FromSize_t(need);
   if (write && write_rows(p, *k, *v, kc, vc, *slots, n, a.s(15))) Py_RETURN_FALSE;
-  return yes(p_vaa_paged_attention_decode(&p, p16(*q), kc, vc, static_cast<int32_t*>(ptr(*bt)),
-                                          static_cast<int32_t*>(ptr(*sl)), p16(*o), nullptr,
-                                          nullptr, need ? ptr(*ws) : nullptr,
-                                          need ? ws->nbytes() : 0, a.s(15)));
+  return yes(launch(p_vaa_paged_attention_decode, &p, p16(*q), kc, vc,
+                    static_cast<int32_t*>(ptr(*bt)), static_cast<int32_t*>(ptr(*sl)), p16(*o),
+                    nullptr, nullptr, need ? ptr(*ws) : nullptr, need ? ws->nbytes() : 0, a.s(15)));
 }
 
 // Fields of an unsplit prefill of tokens [0, n).
@@ -507,11 +519,11 @@ PyObject* step_prefill(const Args& a) {
   const int S = static_cast<int>(qsl->numel() - 1);
   const size_t need = p_vaa_prefill_step_workspace_size(&p, n, S);
   if (!room(ws, need, *q)) return PyLong_FromSize_t(need);
-  return yes(p_vaa_prefill_step(&p, p16(*q), kc, vc, static_cast<int32_t*>(ptr(*bt)),
-                                static_cast<int32_t*>(ptr(*sl)),
-                                static_cast<int32_t*>(ptr(*qsl)), S, write ? p16(*k) : nullptr,
-                                write ? p16(*v) : nullptr, write ? ptr(*slots) : nullptr, it,
-                                p16(*o), n, a.b(13), ptr(*ws), ws->nbytes(), a.s(15)));
+  return yes(launch(p_vaa_prefill_step, &p, p16(*q), kc, vc, static_cast<int32_t*>(ptr(*bt)),
+                    static_cast<int32_t*>(ptr(*sl)), static_cast<int32_t*>(ptr(*qsl)), S,
+                    write ? p16(*k) : nullptr, write ? p16(*v) : nullptr,
+                    write ? ptr(*slots) : nullptr, it, p16(*o), n, a.b(13), ptr(*ws), ws->nbytes(),
+                    a.s(15)));
 }
 
 // (query, key_cache, value_cache, block_table, token_to_seq, positions, output,
@@ -545,16 +557,15 @@ PyObject* prefill(const Args& a) {
   auto* pp = static_cast<int32_t*>(ptr(*pos));
   void* wp = need ? ptr(*ws) : nullptr;
   if (tiles)
-    return yes(p_vaa_paged_attention_prefill_tiles(
-        &p, p16(*q), p16(*kc), p16(*vc), btp, tp, pp, p16(*o), n,
-        static_cast<int32_t*>(ptr(*tiles)), static_cast<int>(tiles->size(0)), split, wp,
-        need ? ws->nbytes() : 0, a.s(13)));
+    return yes(launch(p_vaa_paged_attention_prefill_tiles, &p, p16(*q), p16(*kc), p16(*vc), btp, tp,
+                      pp, p16(*o), n, static_cast<int32_t*>(ptr(*tiles)),
+                      static_cast<int>(tiles->size(0)), split, wp, need ? ws->nbytes() : 0,
+                      a.s(13)));
   if (split)
-    return yes(p_vaa_paged_attention_prefill_split(&p, p16(*q), p16(*kc), p16(*vc), btp, tp, pp,
-                                                   p16(*o), n, split, wp, need ? ws->nbytes() : 0,
-                                                   a.s(13)));
-  return yes(p_vaa_paged_attention_prefill(&p, p16(*q), p16(*kc), p16(*vc), btp, tp, pp, p16(*o),
-                                           n, a.s(13)));
+    return yes(launch(p_vaa_paged_attention_prefill_split, &p, p16(*q), p16(*kc), p16(*vc), btp, tp,
+                      pp, p16(*o), n, split, wp, need ? ws->nbytes() : 0, a.s(13)));
+  return yes(launch(p_vaa_paged_attention_prefill, &p, p16(*q), p16(*kc), p16(*vc), btp, tp, pp,
+                    p16(*o), n, a.s(13)));
 }
 
 // 16-byte aligned rows, which the attention kernels read directly.
@@ -606,9 +617,9 @@ PyObject* no_cache(const Args& a) {
   p.o_stride_head = o->stride(1);
   const size_t need = p_vaa_attention_no_cache_workspace_size(S, T, L);
   if (!room(ws, need, *q)) return PyLong_FromSize_t(need);
-  return yes(p_vaa_attention_no_cache(&p, p16(*q), p16(*k), p16(*v),
-                                      static_cast<int32_t*>(ptr(*qsl)), p16(*o), T, a.b(10),
-                                      ptr(*ws), ws->nbytes(), a.s(12)));
+  return yes(launch(p_vaa_attention_no_cache, &p, p16(*q), p16(*k), p16(*v),
+                    static_cast<int32_t*>(ptr(*qsl)), p16(*o), T, a.b(10), ptr(*ws), ws->nbytes(),
+                    a.s(12)));
 }
 
 // bind(handle): the entry points of the library that _lib.py loaded.
