@@ -387,3 +387,25 @@ def test_decode_wrapper(gpu, monkeypatch):
                 (a, b), used = _both(monkeypatch, run)
                 _same(a, b)
                 assert used is (native and table is bt), kw
+
+
+@pytest.mark.gpu
+def test_lazy_clones_are_not_written_through(gpu):
+    """A lazy clone (torch._lazy_clone) shares its original's memory until one of
+    the two is written: kernels that write a clone leave the original alone."""
+    n, KV, D = 5, 2, 64
+    x, w = _rand(n, D), _rand(D)
+    base = torch.full((n, D), 7.0, dtype=x.dtype, device="cuda")
+    out = torch._lazy_clone(base)
+    assert torch._C._is_cow_tensor(out)
+    kernels.rms_norm(x, w, 1e-5, out=out)
+    _same(base, torch.full_like(base, 7.0))
+    _same(out, kernels.rms_norm(x, w, 1e-5))
+    cache = torch.zeros(2, 3, 16, KV, D, dtype=x.dtype, device="cuda")
+    clone = torch._lazy_clone(cache)
+    kv = _rand(n, KV, D)
+    slots = torch.arange(n, device="cuda")
+    kernels.kv_write_slots(kv, kv, clone[0], clone[1], slots, layout="vllm")
+    torch.cuda.synchronize()
+    assert not cache.any()
+    _same(clone[:, 0, :n], kv.expand(2, n, KV, D))

@@ -46,7 +46,9 @@ const Tensor* ten(PyObject* o) {
 }
 bool none_or_ten(PyObject* o) { return o == Py_None || THPVariable_Check(o); }
 
-void* ptr(const Tensor& t) { return const_cast<void*>(t.const_data_ptr()); }
+// As Tensor.data_ptr(): a lazy clone that still shares its memory gets its own
+// first, also where the kernel only reads (two views of one storage then agree).
+void* ptr(const Tensor& t) { return t.mutable_data_ptr(); }
 uint16_t* p16(const Tensor& t) { return static_cast<uint16_t*>(ptr(t)); }
 
 bool on_gpu(const Tensor& t) { return t.is_cuda() && t.layout() == at::kStrided; }
