@@ -495,9 +495,13 @@ int vaa_gate_up_silu_split(const uint16_t* x, int64_t x_stride, const uint16_t* 
  *   output[t, n] = round16(sum_k x[t, k] w[n, k]),  fp32 accumulation,
  * in_features a multiple of 64, out_features of 128 (of 256 above 128 tokens);
  * VAA_ERR_UNSUPPORTED otherwise; strides in elements, multiples of 8, 16-byte
- * aligned tensors.  The contraction is split over workgroups; workspace:
- * vaa_linear_workspace_size bytes (0: shape not supported; at most 64 MiB),
- * 16-byte aligned, not shared by calls that can run concurrently.
+ * aligned tensors.  The contraction is split over workgroups where the output
+ * has fewer tiles than the GPU has CUs; workspace: vaa_linear_workspace_size
+ * bytes (0: shape not supported), 16-byte aligned, not shared by calls that can
+ * run concurrently.  It holds the fp32 sums of every split, also of a single
+ * one: at most 64 MiB, or 4 * out_features bytes a token, with the tokens
+ * rounded up to whole tiles (of 32 up to 128 tokens, of at most 256 above),
+ * where that is more (1024 tokens: above 16384 output features).
  */
 size_t vaa_linear_workspace_size(int num_tokens, int in_features, int out_features);
 int vaa_linear(const uint16_t* x, int64_t x_stride, const uint16_t* w, int64_t w_stride,

@@ -210,6 +210,27 @@ def test_topk_workspace_size(lib):
         assert S * k <= 4096 and -(-V // S) <= 16384
 
 
+def test_linear_workspace_size(lib):
+    """Never more than 64 MiB or the fp32 output of whole token tiles, whichever
+    is more; 0 exactly where the product is not supported."""
+    size = lib.vaa_linear_workspace_size
+    largest = 0
+    for t in (1, 31, 32, 33, 127, 128, 129, 192, 193, 255, 256, 257, 511, 768, 1000, 1023, 1024):
+        for k in (64, 512, 4096, 14336, 32768):
+            for n in (128, 256, 4096, 5120, 8192, 16384, 32768, 128256, 151936):
+                got = size(t, k, n)
+                if t > 128 and n % 256:
+                    assert got == 0
+                    continue
+                whole = 4 * n * (-(-t // 32) * 32 if t <= 128 else t + 255)
+                assert 4 * n * t <= got <= max(64 << 20, whole), (t, k, n)
+                largest = max(largest, got)
+    assert largest > 64 << 20
+    assert size(1024, 8192, 32768) == 128 << 20 and size(1024, 8192, 16384) == 64 << 20
+    for t, k, n in ((0, 64, 128), (1025, 64, 256), (4, 96, 128), (4, 64, 192), (4, 0, 128)):
+        assert size(t, k, n) == 0
+
+
 def test_add_rmsnorm_argument_errors(lib):
     """Output over the residual, short strides and null pointers are refused
     before any launch; zero tokens is a no-op."""
