@@ -218,7 +218,13 @@ int vaa_paged_attention_decode(const vaa_attn_params* p, const uint16_t* query,
  * device array of vaa_paged_attention_decode_noalloc_max_workspace() bytes
  * (32 MiB), one per GPU, held until the process ends; a split that needs
  * more (vaa_paged_attention_decode_workspace_size) is refused with
- * VAA_ERR_WORKSPACE before anything is enqueued.  The stream must belong to
+ * VAA_ERR_WORKSPACE before anything is enqueued.  VAA_PARTITION_BALANCED alone
+ * has a smaller form to fall back to: a grid of two workgroups per CU's worth
+ * and shares by tiles alone, taken where only its partials fit (32 query and 8
+ * kv heads, head size 128, 256 CUs: from 1890 to 1952 sequences).  Its pieces
+ * differ from the workspace entry point's, so its rows agree with that one's to
+ * rounding and not bit for bit; it is refused in turn where it does not fit
+ * either.  The stream must belong to
  * the current device.  All calls on one GPU share its array: calls that can
  * overlap on one GPU (different streams, no ordering) race and must not be
  * made.

@@ -990,7 +990,8 @@ inline int heads_per_chunk(int G) {
 // How a call splits its sequences.
 struct Split {
   bool balanced;     // balanced split over the actual lengths
-  bool shared;       // balanced, kSharedPerCu (else kBalPerCu) workgroups per CU's worth
+  bool shared;       // balanced: shares by tiles alone over the grid as it is (the shared
+                     // mode, and the coarse grid of a limited workspace)
   int part;          // fixed: tokens per partition (balanced: -1)
   int max_parts;     // fixed: partitions per sequence; balanced: workgroups per kv head
                      // and head chunk
