@@ -132,8 +132,8 @@ struct GluArgs {
 __device__ __forceinline__ void glu_wait_tiles() { __builtin_amdgcn_s_waitcnt(0x0078); }
 
 // NB: 32-token blocks per wave (the workgroup's tile is 64 NB tokens).  kPart:
-// the two matrices are 256 rows of one plain product, the k-steps are split over
-// gridDim.y and the fp32 sums go to a.part.
+// the two matrices are 256 rows of one plain product, the k-steps are split and
+// the fp32 sums go to a.part.
 template <typename T, bool kStreamW, int NB, bool kPart>
 __global__ void __launch_bounds__(kGThreads) __attribute__((amdgpu_waves_per_eu(1, 1)))
 gate_up_silu_kernel(GluArgs a) {
@@ -147,9 +147,20 @@ gate_up_silu_kernel(GluArgs a) {
       static_cast<uint32_t>(reinterpret_cast<uintptr_t>(smem)));
 
   const int per_xcd = static_cast<int>(gridDim.x) / kGXcds;
-  const int logical = (static_cast<int>(blockIdx.x) % kGXcds) * per_xcd +
-                      static_cast<int>(blockIdx.x) / kGXcds;
-  if (logical >= a.tiles) return;
+  int logical = (static_cast<int>(blockIdx.x) % kGXcds) * per_xcd +
+                static_cast<int>(blockIdx.x) / kGXcds;
+  // kPart: the tiles of all splits, one split after the other, are dealt over
+  // the XCDs together.  (Dealt split by split, a tile count that is no multiple
+  // of 8 leaves the same XCDs short in every split and the others with more
+  // workgroups than CUs: 18 tiles in 12 splits made 36 on six XCDs of 32 CUs.)
+  int split = 0;
+  if constexpr (kPart) {
+    split = logical / a.tiles;
+    if (split * a.k_per >= a.ksteps) return;
+    logical -= split * a.tiles;
+  } else if (logical >= a.tiles) {
+    return;
+  }
   const int t0 = (logical % a.t_tiles) * kTT;
   const int i0 = (logical / a.t_tiles) * kGI;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -230,7 +241,7 @@ gate_up_silu_kernel(GluArgs a) {
     }
   };
   // Steps k0 .. k0 + n - 1 of this split.
-  const int k0 = kPart ? static_cast<int>(blockIdx.y) * a.k_per : 0;
+  const int k0 = kPart ? split * a.k_per : 0;
   const int n = kPart ? min(a.ksteps - k0, a.k_per) : a.ksteps;
   // (Starting the column tiles' steps apart, as the few-token kernel does,
   // measured level here: other tiles' MFMAs spread the loads already.)
@@ -278,7 +289,7 @@ gate_up_silu_kernel(GluArgs a) {
   if constexpr (kPart) {
     // The sums as the lanes hold them: [split][tile][wave][f][c][r4][lane].
     f32x4* p = reinterpret_cast<f32x4*>(a.part) +
-               ((static_cast<int64_t>(blockIdx.y) * a.tiles + logical) * kGWaves + wave) *
+               ((static_cast<int64_t>(split) * a.tiles + logical) * kGWaves + wave) *
                    (4 * NB * 4 * kWave) + lane;
 #pragma unroll
     for (int f = 0; f < 4; ++f)
@@ -750,9 +761,9 @@ int launch_wide_nb(GluArgs a, int splits, hipStream_t stream) {
   const int cols = a.tiles;
   a.t_tiles = (a.num_tokens + 64 * NB - 1) / (64 * NB);
   a.tiles = a.t_tiles * cols;
-  const int grid = (a.tiles + kGXcds - 1) / kGXcds * kGXcds;
-  hipLaunchKernelGGL((gate_up_silu_kernel<T, false, NB, true>), dim3(grid, splits),
-                     dim3(kGThreads), 0, stream, a);
+  const int grid = (a.tiles * splits + kGXcds - 1) / kGXcds * kGXcds;
+  hipLaunchKernelGGL((gate_up_silu_kernel<T, false, NB, true>), dim3(grid), dim3(kGThreads), 0,
+                     stream, a);
   const int st = check_launch("gate_up_silu_kernel");
   if (st) return st;
   hipLaunchKernelGGL((wide_sum_kernel<T, NB>), dim3(a.tiles, 16 * NB), dim3(256), 0, stream, a,
