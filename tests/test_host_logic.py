@@ -319,6 +319,24 @@ def test_prefill_split_beside_decode(ctx, q, dec, want):
     assert sp == want and sp % 1024 == 0
 
 
+@pytest.mark.parametrize("t,n,k,want", [
+    (1, 128, 64, True), (64, 8192, 1024, True),        # few tokens: any weights
+    (65, 1024, 3072, False), (128, 896, 4864, False),  # more: from 8M elements
+    (65, 1024, 8192, True), (128, 14336, 4096, True),
+    (129, 2048, 4096, False), (1024, 8192, 2048, False),   # beyond 128: a long contraction,
+    (512, 14336, 4096, False), (1024, 5120, 5120, False), (129, 512, 8192, False),  # 8M elements
+    (129, 2048, 5632, True), (300, 4096, 14336, True), (1024, 5120, 32768, True),
+    (768, 6144, 16384, True), (1024, 6144, 16384, False),  # and at most 5M outputs
+    (512, 8192, 28672, True), (768, 8192, 28672, False),
+])
+def test_linear_pays(t, n, k, want):
+    """Both sides of each line of the rule, at sizes that were measured."""
+    from vllm_apple_amd import kernels as K
+
+    x, w = torch.empty(t, k, device="meta"), torch.empty(n, k, device="meta")
+    assert K.linear_pays(x, w) is want
+
+
 def test_prefill_split_workspace_is_bounded():
     """One 256-token chunk at a 128k context beside 31 short 248-token
     prefills: the share-based piece (10240 keys, 13 pieces over 7944 tokens)

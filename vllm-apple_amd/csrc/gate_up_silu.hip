@@ -720,9 +720,10 @@ struct LinearPlan {
 };
 
 // The wide kernel up to kWideTokens tokens: above, the library's GEMM is ahead
-// (us, library / this: 512 tokens, 32768 x 5120 288 / 179, 14336 x 4096 88 / 69,
-// 8192 x 2048 33.5 / 29.6; 1024 tokens 393 / 316, 130 / 117, 49 / 45; 2104
-// tokens 553 / 643, 213 / 256, 83 / 88).
+// (us, library / this: 512 tokens, 32768 x 5120 289 / 181, 14336 x 4096 91 / 70,
+// 8192 x 2048 35 / 31; 1024 tokens 395 / 311, 132 / 117, 53 / 46; 2104
+// tokens 553 / 643, 213 / 256, 83 / 88).  Short contractions and wide outputs are
+// the library's below that too (kernels.linear_pays).
 constexpr int kWideTokens = 1024;
 
 LinearPlan linear_plan(int num_tokens, int ksteps, int out_features) {

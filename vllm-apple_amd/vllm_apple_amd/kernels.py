@@ -1161,17 +1161,33 @@ def linear_ok(x: torch.Tensor, weight: torch.Tensor, out: torch.Tensor) -> bool:
                     and a.shape[1] <= a.stride(0) < 1 << 20 for a in (x, weight, out)))
 
 
-# Products that linear runs faster than the library's GEMM: up to 64 tokens over
-# any weights, beyond over weights of at least 8M elements (us, library against
-# linear: 4864 x 896, 64 tokens 13.8 / 10.6, 128 tokens 10.5 / 13.0; 8192 x 2048,
-# 128 tokens 21.4 / 16.8, 512 tokens 33.5 / 29.6; 14336 x 4096, 128 tokens 75 /
-# 34, 512 tokens 88 / 69; 32768 x 5120, 128 tokens 194 / 78, 512 tokens 288 / 179).
+# Products that linear runs no slower than the library's GEMM (device us, library
+# / linear, K x N bf16, weights beyond the caches):
+#  - up to 64 tokens any weights (4864 x 896, 64 tokens 18.4 / 11.5; 256 x 256
+#    8.5 / 7.0; behind only at K 1024 and few tokens, 8192 outputs 8.8 / 9.6, where
+#    an eager call still gains from its shorter host path, 18.5 / 10);
+#  - up to 128 tokens weights of at least 8M elements (8192 x 1024 14.8 / 13.1;
+#    32768 x 5120 195 / 78; the least 4096 x 14336 34.0 / 34.3 and 2048 x 8192
+#    16.2 / 17.4; below, 3072 x 1024 9.1 / 11.1);
+#  - beyond, where the library leaves CUs idle on a long contraction: 8M elements,
+#    K from 5632 and at most 5M outputs.  5632 x 2048, 129 and 1024 tokens 20.1 /
+#    19.7, 39.9 / 36.4; 14336 x 4096 55 / 44, 132 / 117; 16384 x 6144, 768 tokens
+#    170 / 157; 32768 x 5120, 1024 tokens 395 / 311.  Past the lines: 4096 x 2048
+#    15.4 / 18.1, 28.6 / 30.8; 5120 x 5120, 1024 tokens 64.1 / 68.1; 2048 x 8192
+#    35 / 48; 8192 x 512, 192 tokens 14.8 / 15.9; 16384 x 6144, 1024 tokens 191 /
+#    203; 28672 x 8192, 768 tokens 303 / 336.
 _LINEAR_ANY_TOKENS = 64
 _LINEAR_MIN_WEIGHTS = 8 << 20
+_LINEAR_WIDE_MIN_K = 5632
+_LINEAR_WIDE_MAX_OUT = 5 << 20
 
 
 def linear_pays(x: torch.Tensor, weight: torch.Tensor) -> bool:
-    return x.shape[0] <= _LINEAR_ANY_TOKENS or weight.numel() >= _LINEAR_MIN_WEIGHTS
+    t, (n, k) = x.shape[0], weight.shape
+    if t <= _LINEAR_ANY_TOKENS:
+        return True
+    return n * k >= _LINEAR_MIN_WEIGHTS and (
+        t <= LINEAR_MAX_TOKENS or (k >= _LINEAR_WIDE_MIN_K and t * n <= _LINEAR_WIDE_MAX_OUT))
 
 
 def try_linear(x: torch.Tensor, weight: torch.Tensor, out: torch.Tensor,
