@@ -468,10 +468,9 @@ def test_forward_mixed_overlap_balanced_shared_split(gpu, monkeypatch):
 
 @pytest.mark.parametrize("dec_lens", [(), (37, 300)])
 def test_forward_prefill_split_with_host_lengths(gpu, monkeypatch, dec_lens):
-    """With the host lengths in the metadata, a prefill-only batch with one
-    long context next to short ones runs the split-K prefill (the chooser's
-    split); beside decodes (run concurrently) the prefill stays unsplit.
-    Every row matches the oracle either way."""
+    """With the host lengths in the metadata, a batch with one long context next
+    to short ones runs the split-K prefill with the chooser's split, alone and
+    beside decodes (run concurrently).  Every row matches the oracle."""
     from vllm_apple_amd import kernels
     from vllm_apple_amd.backend import HipAttentionImpl
 
@@ -500,7 +499,11 @@ def test_forward_prefill_split_with_host_lengths(gpu, monkeypatch, dec_lens):
     out = torch.zeros((T, H, D), dtype=torch.float16, device=dev)
     impl.forward(None, q, k, v, kv_cache, md, output=out)
     torch.cuda.synchronize()
-    assert seen and (seen[0] > 0) == (len(dec_lens) == 0)
+    ql = [0] * len(dec_lens) + [256] * 3
+    want = kernels.choose_prefill_split(
+        md._seq_lens_cpu, ql, KV, H, kernels.device_cus(dev), head_size=D,
+        beside_decode_tokens=sum(dec_lens) if dec_lens else None)
+    assert seen == [want] and want > 0
     ref, kc, vc = _oracle(b, scale)
     assert_close(host(out), ref, what="forward with split prefill")
 
@@ -543,7 +546,8 @@ def test_forward_mixed_split_prefill_beside_decode(gpu, monkeypatch, dtype):
     if dtype == torch.float16:
         ref, _, _ = _oracle(b, scale)
         assert_close(host(out), ref, what="mixed step, prefill split beside the decode")
-    monkeypatch.setattr(kernels, "_SPLIT_BESIDE_TOKENS", 1 << 30)
+    tiles = kernels._SPLIT_BESIDE_TILES
+    monkeypatch.setattr(kernels, "_SPLIT_BESIDE_TILES", 1 << 30)
     kernels._prefill_split_cache.clear()
     whole = torch.zeros_like(out)
     impl.forward(None, q, k, v, kv_cache, md, output=whole)
@@ -551,7 +555,7 @@ def test_forward_mixed_split_prefill_beside_decode(gpu, monkeypatch, dtype):
     assert seen == [2048, 0]
     # Half an ulp of rounding each, at most 2^-7 of the value in bf16.
     assert_close(host(out.float()), host(whole.float()), what="split against whole")
-    monkeypatch.setattr(kernels, "_SPLIT_BESIDE_TOKENS", 4096)
+    monkeypatch.setattr(kernels, "_SPLIT_BESIDE_TILES", tiles)
     kernels._prefill_split_cache.clear()
     g = torch.cuda.CUDAGraph()
     again = torch.zeros_like(out)

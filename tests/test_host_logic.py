@@ -305,8 +305,7 @@ def test_prefill_split_choice():
     ([5722, 3260, 278, 3370], 256, 113_288, 0),
     ([3072, 40], 64, 5000, 0),         # within 48 key tiles
     ([3073, 40], 64, 5000, 2048),      # just past them
-    ([9000, 40], 64, 4096, 2048),      # the fewest decode tokens that split
-    ([9000, 40], 64, 4095, 0),
+    ([9000, 40], 64, 1, 2048),         # beside the shortest decode too
     ([131072], 2, 5000, 2048),         # pieces up to the slots: 64 x 8 workgroups
     ([1 << 20], 2, 5000, 15360),       # 69 x 8: the slots and an eighth
     ([16384] * 64, 512, 5000, 0),      # more workgroups than slots, all equal

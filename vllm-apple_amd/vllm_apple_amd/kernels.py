@@ -532,7 +532,6 @@ _prefill_ws = _GrowOnlyScratch()
 _PREFILL_KEY_TILE = 64      # keys per prefill tile (paged_prefill.hip)
 _PREFILL_SPLIT_QUANTUM = 1024  # split sizes in multiples of 16 key tiles
 _SPLIT_BESIDE_TILES = 48     # key tiles past which a prefill beside a decode may split
-_SPLIT_BESIDE_TOKENS = 4096  # decode tokens from which a prefill beside them may split
 _prefill_split_cache: dict = {}
 # Largest split-K prefill workspace choose_prefill_split plans for: the
 # partials take num_tokens * H * pieces * (D + 2) * 4 bytes, so a long
@@ -574,15 +573,19 @@ def choose_prefill_split(ctx_lens_host, query_lens_host, num_kv_heads: int,
     head (HBM time over 1.6 us a tile).  A split is chosen when the longest
     workgroup exceeds 1.1x their sum; the pieces are the shortest of at least
     half the sum whose workgroups stay within an eighth over the slots (or
-    over the unsplit grid).  Beside fewer than 4096 decode tokens a step stays
-    unsplit: tests/test_gpu_backend.py pins that for two short decodes (a split
-    would be faster there too).  Overlapped steps of 32/8 heads, D 128, unsplit ->
+    over the unsplit grid).  Contexts within 48 key tiles stay whole: below about
+    2700 keys a split took 1.0 to 1.16 of the unsplit time, from 3200 keys it takes
+    less.  Overlapped steps of 32/8 heads, D 128, unsplit ->
     this rule, us: 8 chunks of 256 up to 16317 keys beside 238k decode tokens
     407 -> 343 (bf16 484 -> 425); 6 of 187 up to 11009 beside 66k 309 -> 180;
     8 of 64 up to 14652 beside 114k, bf16, 413 -> 182; 2 of 38 up to 9519 beside
     184k 432 -> 228.  On the other side of
     the line: 8 of 256 up to 16351 beside 466k 557, split 606 at the least;
-    4 of 256 up to 5722 beside 113k 154, split 154 to 188.
+    4 of 256 up to 5722 beside 113k 154, split 154 to 188.  Few decode tokens
+    change nothing (device us beside one decode of 37 tokens; beside 1500 or six of
+    600, other heads and bf16 the same ratios): one chunk of 64 over 9000 keys 186
+    -> 88, of 32 over 3200 93 -> 82; two of 256 over 6000 and 5000 145 -> 101; four
+    of 256 over 9000 204 -> 188; 256 over 16000 and seven over 1000 324 -> 225.
     Memoised per length tuple (every layer of a step sees the same batch).
     """
     key = (tuple(int(x) for x in ctx_lens_host), tuple(int(x) for x in query_lens_host),
@@ -604,8 +607,7 @@ def choose_prefill_split(ctx_lens_host, query_lens_host, num_kv_heads: int,
     split = 0
     if beside_decode_tokens is not None:
         rest = 1.4 * share + 5.8e-5 * beside_decode_tokens * num_kv_heads
-        if beside_decode_tokens >= _SPLIT_BESIDE_TOKENS \
-                and longest > max(_SPLIT_BESIDE_TILES, 1.1 * rest):
+        if longest > max(_SPLIT_BESIDE_TILES, 1.1 * rest):
             quantum = _PREFILL_SPLIT_QUANTUM // _PREFILL_KEY_TILE
             most = max(slots, sum(q for q, _ in work) * heads_grid) + slots // 8
             piece = max(2, -(-int(rest / 2) // quantum)) * quantum
