@@ -59,11 +59,11 @@ enum { VAA_DTYPE_F16 = 0, VAA_DTYPE_BF16 = 1 };
  * vaa_attn_params.partition_size for decode:
  *   > 0  fixed split-K partitions of that many tokens (a multiple of 128);
  *   0    automatic, from max_seq_len alone;
- *   VAA_PARTITION_BALANCED  4-wave workgroups, up to four per CU's worth, each
+ *   VAA_PARTITION_BALANCED  4-wave workgroups, two per CU's worth, each
  *        taking an equal share of the 16-token tiles of all sequences (and of
  *        the sequences' start-ups), split on the device from seq_lens (for
  *        unequal lengths; at most 8192 sequences).
- *   VAA_PARTITION_BALANCED_SHARED  shares by tiles alone over always four
+ *   VAA_PARTITION_BALANCED_SHARED  shares by tiles alone over four
  *        workgroups per CU's worth, for a decode that runs concurrently with
  *        another kernel (a mixed step's prefill on a second stream): its
  *        smaller shares then fill the CUs the other kernel leaves.
@@ -218,13 +218,7 @@ int vaa_paged_attention_decode(const vaa_attn_params* p, const uint16_t* query,
  * device array of vaa_paged_attention_decode_noalloc_max_workspace() bytes
  * (32 MiB), one per GPU, held until the process ends; a split that needs
  * more (vaa_paged_attention_decode_workspace_size) is refused with
- * VAA_ERR_WORKSPACE before anything is enqueued.  VAA_PARTITION_BALANCED alone
- * has a smaller form to fall back to: a grid of two workgroups per CU's worth
- * and shares by tiles alone, taken where only its partials fit (32 query and 8
- * kv heads, head size 128, 256 CUs: from 1890 to 1952 sequences).  Its pieces
- * differ from the workspace entry point's, so its rows agree with that one's to
- * rounding and not bit for bit; it is refused in turn where it does not fit
- * either.  The stream must belong to
+ * VAA_ERR_WORKSPACE before anything is enqueued.  The stream must belong to
  * the current device.  All calls on one GPU share its array: calls that can
  * overlap on one GPU (different streams, no ordering) race and must not be
  * made.

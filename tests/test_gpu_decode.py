@@ -180,9 +180,8 @@ def test_decode_matches_pure_loop_oracle(gpu):
 def test_decode_balanced_ragged_batch(gpu, seed, mode):
     """Balanced split over many ragged sequences (empty ones included): every
     piece boundary (inside a sequence, between sequences, across workgroups)
-    against the oracle, with the fused write bit-exact.  mode -1 is one
-    8-wave workgroup per CU, -2 (shared) 4-wave workgroups, four per CU's
-    worth of the split."""
+    against the oracle, with the fused write bit-exact.  mode -1 is two
+    4-wave workgroups per CU's worth of the split, -2 (shared) four."""
     g = torch.Generator().manual_seed(seed)
     lens = torch.randint(0, 3000, (77,), generator=g)
     lens[::9] = 0
@@ -320,12 +319,12 @@ def test_merge_attn_states(gpu, dtype):
 @pytest.mark.parametrize("lens,KV", [
     ([16] * 90 + [1, 0, 17, 700], 8),          # ranges of many one-tile sequences
     ([0, 0, 5, 0], 2), ([512], 2), ([511, 1, 513, 2048], 4),
-    ([40] * 300, 32), ([1500, 30] * 16, 32),   # shares above and below the doubled grid's
-    ([1600] * 26, 32),
+    ([40] * 300, 32), ([1500, 30] * 16, 32), ([1600] * 26, 32),
+    ([9, 70], 32), ([200], 16),                # fewer ranges than workgroups
 ])
 def test_balanced_split_units(gpu, mode, lens, KV):
     """The balanced split's shares: ranges that end inside a sequence's start-up
-    units, sequences whole in a range and over several, coarse and fine grids,
+    units, sequences whole in a range and over several, workgroups without a range,
     empty sequences; every row in 64 bits."""
     from vllm_apple_amd import kernels
 

@@ -2,8 +2,7 @@
 through the C ABI, against vaa_paged_attention_decode with a caller
 workspace: bit-identical outputs and fused cache writes on two calls in a
 row, the second smaller, in every split mode that fits the fixed array; a
-split that does not fit is refused before anything runs.  The balanced split
-has a coarser grid to fall back to: same fused writes, rows to rounding."""
+split that does not fit is refused before anything runs."""
 import ctypes
 
 import numpy as np
@@ -80,46 +79,25 @@ def test_noalloc_matches_workspace_entry_point(gpu, part):
         assert not torch.any(o2 == 7.0), "rows left unwritten"
 
 
-def _balanced_bytes(S, per_cu, extra_row, H=32, KV=8, D=128):
-    """Header and partial rows of a balanced split of S sequences."""
-    from vllm_apple_amd import kernels
-
-    groups = -(-per_cu * kernels.device_cus() // KV)
-    rows = KV * (groups + S - 1 + extra_row) * (H // KV)
-    return -(-(S + 2) * 4 // 256) * 256 + rows * (D + 2) * 4
-
-
-def test_noalloc_balanced_falls_back_to_the_coarse_grid(gpu):
-    """The largest batch whose coarse partials fit the fixed array (and whose
-    fine ones do not): the attention of fp64 in every row, the workspace entry
-    point's fused writes.  One sequence more is refused."""
-    from helpers import assert_close, host
-    from vllm_apple_amd import _lib
+def test_noalloc_balanced_at_its_limit(gpu):
+    """The largest balanced batch whose partials fit the fixed array matches the
+    workspace entry point; one sequence more is refused."""
+    from vllm_apple_amd import _lib, kernels
 
     cap = _lib.load().vaa_paged_attention_decode_noalloc_max_workspace()
-    S = next(s for s in range(8, 8192) if _balanced_bytes(s + 1, 2, 1) > cap)
-    assert _balanced_bytes(S, 2, 1) <= cap < _balanced_bytes(S, 4, 0)
+
+    def need(S):  # header, and rows of 8 kv heads x 4 query heads, D 128
+        rows = 8 * (-(-2 * kernels.device_cus() // 8) + S) * 4
+        return -(-(S + 2) * 4 // 256) * 256 + rows * 130 * 4
+    S = next(s for s in range(8, 8192) if need(s + 1) > cap)
     lens = [(7 * i) % 23 + 1 for i in range(S)]
     lens[5], lens[700], lens[701], lens[S - 1] = 3000, 1500, 5000, 900
-    print(f"[case] noalloc coarse balanced, {S} sequences", flush=True)
+    print(f"[case] noalloc balanced, {S} sequences", flush=True)
     case = _case(S, 32, 8, 128, lens, seed=3)
-    kc, vc, bt, lens_d, q, nk, nv = case
-    p = _params(kc, vc, q, q, nk, lens_d, bt, -1)
-    need = _lib.load().vaa_paged_attention_decode_workspace_size(ctypes.byref(p), None)
-    assert need == _balanced_bytes(S, 4, 0)
+    p = _params(case[0], case[1], case[4], case[4], case[5], case[3], case[2], -1)
+    assert _lib.load().vaa_paged_attention_decode_workspace_size(ctypes.byref(p), None) == need(S)
     (o1, k1, v1), (o2, k2, v2) = _both(case, -1)
-    assert torch.equal(k1, k2) and torch.equal(v1, v2), "fused writes differ"
-    assert_close(host(o2), host(o1), what="coarse grid against the fine one")
-    ref = np.empty(o2.shape)
-    k, v = k2.cpu().double().numpy(), v2.cpu().double().numpy()
-    qn, table = q.cpu().double().numpy().reshape(S, 8, 4, 128), bt.cpu().numpy()
-    for s, L in enumerate(lens):
-        blocks = table[s, :-(-L // 16)]
-        ks, vs = (x[blocks].transpose(1, 0, 2, 3).reshape(8, -1, 128)[:, :L] for x in (k, v))
-        w = qn[s] @ ks.transpose(0, 2, 1) / np.sqrt(128)
-        w = np.exp(w - w.max(-1, keepdims=True))
-        ref[s] = ((w / w.sum(-1, keepdims=True)) @ vs).reshape(32, 128)
-    assert_close(host(o2), ref, what="coarse balanced split")
+    assert torch.equal(o1, o2) and torch.equal(k1, k2) and torch.equal(v1, v2)
     more = _case(S + 1, 32, 8, 128, [3] * (S + 1), seed=4)
     out = torch.full_like(more[4], 7.0)
     p = _params(more[0], more[1], more[4], out, more[5], more[3], more[2], -1)

@@ -17,10 +17,10 @@
 //              at the end.  Fixed partitions of at most 1024 tokens use
 //              4-wave workgroups, two per CU: one's start-up overlaps the
 //              other's streaming.  The balanced split uses 4-wave workgroups
-//              too, up to four per CU's worth; beside another kernel
-//              (VAA_PARTITION_BALANCED_SHARED) always four: the concurrent
-//              kernel's workgroups hold some CUs, and the shorter pieces let
-//              the dispatcher give the free CUs more of them.
+//              too, two per CU's worth; beside another kernel
+//              (VAA_PARTITION_BALANCED_SHARED) four: the concurrent kernel's
+//              workgroups hold some CUs, and the shorter pieces let the
+//              dispatcher give the free CUs more of them.
 //   split-K  = only when the (seq, kv_head) pairs cannot fill the GPU or the
 //              lengths are unequal; partials (max, sum, acc) go to a workspace
 //              and a second kernel merges them (log-sum-exp).  The merge is a
@@ -74,12 +74,15 @@ typedef short i16x4 __attribute__((ext_vector_type(4)));
 constexpr int kWaves = 8;   // waves per workgroup
 constexpr int kShortPartTiles = 64;  // fixed partitions up to 1024 tokens run 4-wave workgroups
 // Balanced split: 4-wave workgroups (C2u 0.115 -> 0.105 ms and C4 0.575 ->
-// 0.547 ms against one 8-wave workgroup per CU, one box), a grid of four per
-// CU's worth (kFinePerCu).  VAA_PARTITION_BALANCED_SHARED, beside a concurrent
-// kernel, always splits by that grid (C5 step beside the prefill: 3, 4, 6, 8
-// per CU's worth -> 0.577, 0.571, 0.579, 0.587 ms; two: 0.597); alone, short
-// shares are doubled (kFineMinUnits).  Three workgroups per CU's worth at three
-// waves per SIMD: C2u the same, C4 and the C5 step slower.
+// 0.547 ms against one 8-wave workgroup per CU, one box), two per CU's worth, as
+// many as are resident at D 128.  Four cost every batch of long shares the second
+// round (us, two / four: 84 contexts of 2498 to 4997, 28/4 heads, 111.2 / 118.4; 11
+// of 32000 127.3 / 138.2; 102 of 4533 to 9066, 16/2 heads, 123.8 / 129.4; 66 of
+// 12249 to 24499, 14/2 heads, D 64, 105 / 123; ahead only at D 32: 77 of 383 to 6115
+// 40.0 / 35.4, 80 of 16000 to 32000 88.7 / 84.4).  VAA_PARTITION_BALANCED_SHARED,
+// beside a concurrent kernel, takes four (C5 step beside the prefill: 3, 4, 6, 8
+// per CU's worth -> 0.577, 0.571, 0.579, 0.587 ms; two: 0.597).  Three workgroups per
+// CU's worth at three waves per SIMD: C2u the same, C4 and the C5 step slower.
 //
 // Loads run one tile ahead in the balanced and the 8-wave kernels (against
 // two ahead, one box: C2u 0.1031-0.1035 -> 0.1011-0.1014 ms, headline
@@ -88,7 +91,7 @@ constexpr int kShortPartTiles = 64;  // fixed partitions up to 1024 tokens run 4
 // against 0.638 ms).
 constexpr int kBalWaves = kWaves / 2;
 constexpr int kBalPerCu = 2;
-constexpr int kFinePerCu = 4;
+constexpr int kSharedPerCu = 4;
 constexpr int kTile = 16;   // tokens per MFMA tile
 
 // Tensors are raw 16-bit storage; the kernels' element type T (fp16 or bf16)
@@ -105,7 +108,7 @@ struct DecodeArgs {
   // Split-K partials, one row per (piece, query head): unnormalised acc [D]
   // and (max in the log2 domain, sum).  Fixed partitions use rows
   // (seq*H + qhead)*max_parts + part; the balanced split uses
-  // (y*bal_rows + c + seq)*Gc + h, with y = kv head x head
+  // (y*(max_parts + num_seqs) + c + seq)*Gc + h, with y = kv head x head
   // chunk, max_parts = workgroups per y, and keeps its geometry in ws_hdr
   // (per, starts[0..num_seqs]).
   float* ws_acc;
@@ -119,8 +122,6 @@ struct DecodeArgs {
   int bs16;
   int Gc, chunks;  // query heads per chunk (<= 16) and chunks per kv head
   int part_tiles, max_parts;
-  int shared;    // balanced split: VAA_PARTITION_BALANCED_SHARED
-  int bal_rows;  // balanced split: workspace rows per kv head and head chunk
   int seq_cost;  // balanced split: units of a sequence's start-up
   int lds_main;  // bytes of LDS before the balanced split's prefix sums
   int64_t num_blocks;
@@ -696,7 +697,7 @@ paged_decode_kernel(DecodeArgs a) {
 // workgroup derives the same prefix sums of units per sequence from seq_lens, so
 // the split follows the actual lengths without a host round trip.  A sequence
 // inside one workgroup's range is finished there; the pieces of a sequence that
-// crosses ranges go to workspace rows (y*bal_rows + c + seq)*Gc
+// crosses ranges go to workspace rows (y*(gridDim.x + num_seqs) + c + seq)*Gc
 // + h, y = blockIdx.y (kv head x head chunk) -- distinct for distinct (c, seq)
 // because the ranges and the sequences are both in increasing order -- and
 // the merge kernel combines them.
@@ -704,16 +705,10 @@ paged_decode_kernel(DecodeArgs a) {
 // A sequence's units are its tiles plus, in front of them, kSeqCost for its
 // start-up (table window, Q, first tiles, combine), so that a range of many short
 // sequences does not take longer than one of a long one (27 contexts of 115 to
-// 3866: 37.8 us without, 32.6 with 8 units; 12 and 16 level or slower).  per is
-// the total over the grid of four workgroups per CU's worth, or, where that is
-// less than kFineMinUnits, twice it: a second round of short workgroups costs more
-// than their balance gains (us, two per CU's worth -> this rule: 100 contexts of
-// 1000 to 2000 114.6 -> 110.1, 32 of 1024 to 8192 68.6 -> 65.2; 27 of 115 to 3866
-// stay at two: 32.4, four 41.7).  The shared split keeps the plain grid and no
-// start-up units: its ranges run beside the other kernel's, and the mixed step
-// lost 0.5 % with them.
+// 3866: 37.8 us without, 32.6 with 8 units; 12 and 16 level or slower).  The
+// shared split has no start-up units: its ranges run beside the other kernel's,
+// and the mixed step lost 0.5 % with them.
 constexpr int kBalMinUnits = 4 * kWaves;
-constexpr int kFineMinUnits = 72;
 constexpr int kSeqCost = 8;
 
 __device__ __forceinline__ int cost_of(const DecodeArgs& a, int seq) {
@@ -756,14 +751,12 @@ paged_decode_balanced_kernel(DecodeArgs a) {
   int* starts = reinterpret_cast<int*>(smem + a.lds_main);
   tile_prefix(a, starts, starts + B + 1);
   const int total = starts[B];
-  int per = (total + nc - 1) / nc;
-  if (!a.shared && per < kFineMinUnits) per = (2 * total + nc - 1) / nc;
-  per = max(per, kBalMinUnits);
-  // The ranges in use are numbered without gaps over all kv heads, so that the
-  // surplus workgroups are the last of the grid.  With each head's surplus behind
-  // its own ranges the dispatcher dealt ranges to some CUs and surplus, which
-  // exits at once, to the others (32 kv heads, half of the grid in use: 105
-  // contexts of 15 to 251 85 us, 13 of 2391 116).
+  const int per = max((total + nc - 1) / nc, kBalMinUnits);
+  // The ranges in use (a small total leaves some workgroups without) are numbered
+  // without gaps over all kv heads, so that the surplus workgroups are the last of
+  // the grid.  With each head's surplus behind its own ranges the dispatcher dealt
+  // ranges to some CUs and surplus, which exits at once, to the others (32 kv
+  // heads, half of a grid in use: 105 contexts of 15 to 251 85 us, 50 without gaps).
   const int used = max(1, (total + per - 1) / per);
   const int id = blockIdx.y * nc + blockIdx.x;
   const int y = id / used, c = id % used;
@@ -796,7 +789,7 @@ paged_decode_balanced_kernel(DecodeArgs a) {
     if (t1 <= t0) continue;  // only start-up units: the tiles are the next workgroup's
     RangeOut ro;
     ro.whole = (t0 == 0 && t1 == s1 - s0 - a.seq_cost);
-    ro.prow0 = (static_cast<int64_t>(y) * a.bal_rows + c + seq) * a.Gc;
+    ro.prow0 = (static_cast<int64_t>(y) * (nc + B) + c + seq) * a.Gc;
     ro.prow_step = 1;
     const int L = clamped_len(a, seq);
     decode_range<D, T, NW, false, kPad>(a, smem, seq, kvh, qh0, nh, L,
@@ -870,7 +863,7 @@ paged_decode_merge_balanced_kernel(DecodeArgs a) {
   const int c0 = (h0 + a.seq_cost) / per, c1 = (h1 - 1) / per;
   if (c0 == c1) return;
   const int hg = qh % a.G, y = (qh / a.G) * a.chunks + hg / a.Gc, h = hg % a.Gc;
-  const int64_t base = static_cast<int64_t>(y) * a.bal_rows + seq;
+  const int64_t base = static_cast<int64_t>(y) * (a.max_parts + a.num_seqs) + seq;
   MergeAcc4 m;
 #pragma unroll 4
   for (int c = c0; c <= c1; ++c) {
@@ -998,13 +991,10 @@ inline int heads_per_chunk(int G) {
 // How a call splits its sequences.
 struct Split {
   bool balanced;     // balanced split over the actual lengths
-  bool shared;       // balanced: shares by tiles alone over the grid as it is (the shared
-                     // mode, and the coarse grid of a limited workspace)
+  bool shared;       // balanced, kSharedPerCu (else kBalPerCu) workgroups per CU's worth
   int part;          // fixed: tokens per partition (balanced: -1)
   int max_parts;     // fixed: partitions per sequence; balanced: workgroups per kv head
                      // and head chunk
-  int bal_rows;      // balanced: partial rows (of a chunk's heads) per kv head and chunk:
-                     // workgroup + sequence is at most max_parts + num_seqs - 2
   size_t ws_bytes;   // workspace needed (0: none)
   size_t hdr_bytes;  // balanced: bytes before the partial rows
 };
@@ -1012,11 +1002,11 @@ struct Split {
 // Fixed partitions with partition_size > 0; with 0 the size comes from
 // max_seq_len alone (all sequences assumed at the maximum): split only as far
 // as needed for the workgroups to cover every CU once, in multiples of
-// 16 * kWaves tokens.  VAA_PARTITION_BALANCED(_SHARED): a grid of four 4-wave
-// workgroups per CU's worth, each taking an equal share of all sequences (split
-// on the device from seq_lens).  limit: the largest workspace the caller has;
-// the balanced split falls back to its coarse grid to fit it.
-int plan_split(const vaa_attn_params* p, Split* sp, size_t limit = SIZE_MAX) {
+// 16 * kWaves tokens.  VAA_PARTITION_BALANCED: 4-wave workgroups, two per
+// CU's worth, each taking an equal share of all sequences (split on the device
+// from seq_lens); VAA_PARTITION_BALANCED_SHARED: the same with four per CU's
+// worth.
+int plan_split(const vaa_attn_params* p, Split* sp) {
   const int64_t cap = static_cast<int64_t>(p->max_blocks_per_seq) * p->block_size;
   int64_t max_len = p->max_seq_len;
   if (max_len > cap) max_len = cap;
@@ -1034,18 +1024,11 @@ int plan_split(const vaa_attn_params* p, Split* sp, size_t limit = SIZE_MAX) {
     sp->shared = shared;
     sp->part = static_cast<int>(part);
     sp->hdr_bytes = ((static_cast<size_t>(p->num_seqs) + 2) * sizeof(int) + 255) / 256 * 256;
-    // The fine grid, or the coarse one (whose kernel splits as the shared mode
-    // does: by its own grid) where only that one's partials fit `limit`.
-    for (int per_cu : {kFinePerCu, kBalPerCu}) {
-      const int wgs = (per_cu * num_cus() + ys - 1) / ys;
-      sp->max_parts = wgs < 1 ? 1 : wgs;
-      sp->bal_rows = sp->max_parts + p->num_seqs - (sp->shared ? 0 : 1);
-      const size_t rows =
-          static_cast<size_t>(ys) * sp->bal_rows * heads_per_chunk(p->queries_per_kv);
-      sp->ws_bytes = sp->hdr_bytes + rows * row_bytes;
-      if (shared || sp->ws_bytes <= limit) break;
-      sp->shared = true;
-    }
+    const int wgs = ((shared ? kSharedPerCu : kBalPerCu) * num_cus() + ys - 1) / ys;
+    sp->max_parts = wgs < 1 ? 1 : wgs;
+    const size_t rows = static_cast<size_t>(ys) * (sp->max_parts + p->num_seqs) *
+                        heads_per_chunk(p->queries_per_kv);
+    sp->ws_bytes = sp->hdr_bytes + rows * row_bytes;
     return VAA_OK;
   }
   if (part > 0) {
@@ -1070,7 +1053,6 @@ int plan_split(const vaa_attn_params* p, Split* sp, size_t limit = SIZE_MAX) {
     return fail(VAA_ERR_UNSUPPORTED,
                 "partition_size=%lld splits max_seq_len=%lld into more than 65535 partitions",
                 (long long)part, (long long)max_len);
-  sp->bal_rows = 0;
   sp->balanced = false;
   sp->shared = false;
   sp->part = static_cast<int>(part);
@@ -1184,7 +1166,7 @@ int decode_impl(const char* what, const vaa_attn_params* p, const uint16_t* quer
                 uint16_t* key_cache, uint16_t* value_cache, const int32_t* block_table,
                 const int32_t* seq_lens, uint16_t* output, const uint16_t* new_keys,
                 const uint16_t* new_values, void* workspace, size_t workspace_bytes,
-                void* stream, size_t limit = SIZE_MAX) {
+                void* stream) {
   int st = check_params(p, what);
   if (st) return st;
   if (p->num_seqs == 0) return VAA_OK;
@@ -1201,7 +1183,7 @@ int decode_impl(const char* what, const vaa_attn_params* p, const uint16_t* quer
     return fail(VAA_ERR_INVALID_ARG,
                 "%s: query and caches must be 16-byte aligned", what);
   Split sp;
-  st = plan_split(p, &sp, limit);
+  st = plan_split(p, &sp);
   if (st) return st;
 
   DecodeArgs a;
@@ -1244,8 +1226,6 @@ int decode_impl(const char* what, const vaa_attn_params* p, const uint16_t* quer
   a.Gc = heads_per_chunk(a.G);
   a.part_tiles = sp.balanced ? 0 : sp.part / kTile;
   a.max_parts = sp.max_parts;
-  a.shared = sp.shared ? 1 : 0;
-  a.bal_rows = sp.bal_rows;
   a.seq_cost = sp.shared ? 0 : kSeqCost;
   a.lds_main = 0;
   a.num_blocks = p->num_blocks;
@@ -1348,7 +1328,7 @@ extern "C" int vaa_paged_attention_decode_noalloc(const vaa_attn_params* p,
   if (st) return st;
   if (p->num_seqs == 0) return VAA_OK;
   Split sp;
-  st = plan_split(p, &sp, kScratchBytes);
+  st = plan_split(p, &sp);
   if (st) return st;
   if (sp.ws_bytes > kScratchBytes)
     return fail(VAA_ERR_WORKSPACE,
@@ -1362,8 +1342,7 @@ extern "C" int vaa_paged_attention_decode_noalloc(const vaa_attn_params* p,
     if (!ws) return VAA_ERR_HIP;
   }
   return decode_impl(what, p, query, key_cache, value_cache, block_table, seq_lens, output,
-                     new_keys, new_values, ws, sp.ws_bytes > 0 ? kScratchBytes : 0, stream,
-                     kScratchBytes);
+                     new_keys, new_values, ws, sp.ws_bytes > 0 ? kScratchBytes : 0, stream);
 }
 
 extern "C" int vaa_merge_attn_states(const float* partial_out, const float* partial_lse,

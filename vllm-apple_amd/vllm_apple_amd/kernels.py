@@ -303,9 +303,9 @@ def decode_workspace_size(p: _lib.VaaAttnParams) -> tuple[int, int]:
 # Decode launch geometry (paged_decode.hip): partitions in multiples of 128
 # tokens; partitions up to 1024 tokens run 4-wave workgroups, two per CU (one's
 # start-up overlaps the other's streaming), longer ones one 8-wave workgroup
-# per CU.  The balanced split runs 4-wave workgroups, two to four per CU's worth,
-# gives each workgroup at least 32 tiles (512 tokens) and takes at most 8192
-# sequences.
+# per CU.  The balanced split runs 4-wave workgroups, two per CU's worth, gives
+# each workgroup at least 32 units (16-token tiles, and 8 for each sequence's
+# start-up) and takes at most 8192 sequences.
 _DECODE_QUANTUM = 128
 _SHORT_PART_TOKENS = 1024
 # How much faster than its share of HBM a decode workgroup streams when the
