@@ -669,15 +669,18 @@ size_t split_bytes(int tiles, int splits, int num_tokens) {
 }
 
 // 32-token blocks per wave (2, 3 or 4) for a batch over `cols` column tiles: the
-// fewest rounds of one workgroup per CU (256), a round costing NB + 1/2 (of a
-// k-step's time with one block; 80 k-steps, whole rounds: NB = 2, 3, 4 take 80,
-// 107 and 141 us).  300 tokens, 4096 x 14336: 106.3 us at NB = 4, 90.8 at 3;
-// 192 tokens: 85.0, 72.2 at 2; 2104 tokens, 5120 x 32768: 1170, 1151 at 3.
+// least rounds of one workgroup per CU (256) times a round's time, 17, 21 and 27 for
+// NB = 2, 3 and 4: a k-step takes 0.98, 1.22 and 1.57 us where there are several
+// rounds.  300 tokens, 4096 x 14336: 104.9 us at NB = 4, 84.8 at 3; 192 tokens 93.4,
+// 65.9 at 2; 2104 tokens, 5120 x 32768: 1170, 1151 at 3.  On the other side, which
+// rounds costing NB + 1/2 gave to NB = 2: 1024 tokens, 8192 x 28672 809 us at NB = 4,
+// 881 at 2; 3584 x 18944 267, 282.
 inline int wide_blocks(int num_tokens, int cols) {
+  constexpr int kRound[] = {0, 0, 17, 21, 27};
   int best = 4, cost = INT32_MAX;
   for (int nb = 4; nb >= 2; --nb) {
     const int64_t tiles = static_cast<int64_t>((num_tokens + 64 * nb - 1) / (64 * nb)) * cols;
-    const int c = static_cast<int>((tiles + 255) / 256) * (2 * nb + 1);
+    const int c = static_cast<int>((tiles + 255) / 256) * kRound[nb];
     if (c < cost) {
       cost = c;
       best = nb;
