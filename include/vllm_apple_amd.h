@@ -564,7 +564,9 @@ int vaa_qkv_epilogue(const vaa_attn_params* p, uint16_t* query, uint16_t* key,
  * chunks' survivors then go through `workspace`, whose size
  * vaa_topk_workspace_size returns (0: none needed, workspace may be null).  It
  * depends only on (num_tokens, vocab_size, k).  VAA_ERR_WORKSPACE when it is
- * missing, short or not 16-byte aligned.  Two launches at most, no allocation.
+ * missing, short or not 16-byte aligned.  Most rows of 8192 to 163833 columns are
+ * selected whole and leave the workspace unused; the size and the refusal are the
+ * same there.  Two launches at most, no allocation.
  */
 int vaa_topk_workspace_size(int num_tokens, int vocab_size, int k, size_t* workspace_bytes);
 int vaa_topk_logits(const uint16_t* logits, int num_tokens, int vocab_size,

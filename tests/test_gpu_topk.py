@@ -125,10 +125,9 @@ def test_engine_topk_encode_and_reconstruct(gpu, monkeypatch):
 @pytest.mark.parametrize("T,k", [(256, 50), (64, 50), (32, 64), (40, 1)])
 @pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
 def test_topk_bench_shape_one_wave_paths(gpu, T, k, dtype):
-    """The bench's vocabulary (128256) at k <= 64, where each chunk and each
-    row's merge runs on one wave: every row against the oracle, with some rows
-    flat or tied so that the chunk and merge lists overflow and take the
-    exact-key and ordered-compaction paths."""
+    """The bench's vocabulary (128256) at k <= 64, which the row kernel selects
+    whole: every row against the oracle, with some rows flat or tied so that the
+    list overflows and takes the exact-key and ordered-compaction paths."""
     from vllm_apple_amd import kernels
 
     print(f"[case] topk bench shape T={T} k={k} {dtype}", flush=True)
@@ -140,7 +139,7 @@ def test_topk_bench_shape_one_wave_paths(gpu, T, k, dtype):
     logits[3, ::97] = float("inf")                    # many equal maxima
     logits[4] = -float("inf")
     logits[4, 5000:5000 + 3] = 1.0
-    assert kernels.topk_workspace_size(T, V, k) > 0   # chunked: the merge runs
+    assert kernels.topk_workspace_size(T, V, k) > 0   # asked for, and left unused
     idx, vals = kernels.topk_logits(logits.cuda(), k)
     torch.cuda.synchronize()
     ref_idx, ref_vals = otk.topk(_bits(logits), k)
@@ -154,7 +153,7 @@ def test_topk_wave_path_ragged_tail_strided(gpu):
     k = 64, its largest k, with enough rows for the wave kernel."""
     from vllm_apple_amd import kernels
 
-    T, V, k = 1400, 10001, 64
+    T, V, k = 2100, 10001, 64  # above 2048 rows of less than 12288 columns
     print(f"[case] topk wave tail T={T} V={V} k={k}", flush=True)
     g = torch.Generator().manual_seed(17)
     big = (torch.randn(T, V + 7, generator=g) * 3).half()
@@ -164,6 +163,36 @@ def test_topk_wave_path_ragged_tail_strided(gpu):
     idx, vals = kernels.topk_logits(logits, k)
     torch.cuda.synchronize()
     ref_idx, ref_vals = otk.topk(_bits(big[:, :V].contiguous()), k)
+    assert np.array_equal(idx.cpu().numpy(), ref_idx)
+    assert np.array_equal(_bits(vals), ref_vals)
+
+
+@pytest.mark.parametrize("T,V,stride,k", [
+    (64, 200000, 200000, 50), (50, 163841, 163848, 64), (43, 200000, 200000, 1),
+    (1100, 8001, 8008, 64), (1050, 7000, 7000, 1),
+    (1100, 33000, 33000, 1), (1600, 12288, 12296, 2),
+])
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+def test_topk_one_wave_per_chunk(gpu, T, V, stride, k, dtype):
+    """Rows that the row kernel does not take, or takes more slowly (the last two),
+    in enough chunks (2048) and at a k (up to 64) for the one-wave chunk and merge
+    kernels: some rows flat or tied so that the chunk and merge lists overflow,
+    ragged tails."""
+    from vllm_apple_amd import kernels
+
+    print(f"[case] topk wave chunks T={T} V={V} k={k} {dtype}", flush=True)
+    g = torch.Generator().manual_seed(T + k)
+    x = (torch.randn(T, stride, generator=g) * 4).to(dtype)
+    x[1] = 0.5
+    x[2] = torch.randint(-2, 3, (stride,), generator=g).to(dtype)
+    x[3, ::97] = float("inf")
+    x[4] = -float("inf")
+    x[4, 5000:5003] = 1.0
+    x[5, V - 3:V] = 30.0
+    assert kernels.topk_workspace_size(T, V, k) >= 2048 * k * 8
+    idx, vals = kernels.topk_logits(x.cuda()[:, :V], k)
+    torch.cuda.synchronize()
+    ref_idx, ref_vals = otk.topk(_bits(x[:, :V].contiguous()), k)
     assert np.array_equal(idx.cpu().numpy(), ref_idx)
     assert np.array_equal(_bits(vals), ref_vals)
 

@@ -8,8 +8,8 @@
 //
 // Rows of 8192 to 163833 columns (the vocabularies served in practice) are
 // selected whole by one 16-wave workgroup each, in its registers
-// (topk_row_kernel).  Other rows, and large batches of the shortest of these,
-// are cut into S chunks of at most kChunkMax columns, one workgroup per chunk,
+// (topk_row_kernel).  Other rows, and large batches of these where that is faster
+// (row_kernel_ok, wave_chunks_ahead), are cut into S chunks of at most kChunkMax columns, one workgroup per chunk,
 // so a small batch still fills the chip.  A workgroup loads
 // its whole chunk into registers with every load in flight at once (one HBM
 // round trip) and selects on order-preserving 16-bit keys: a lower bound L
@@ -414,7 +414,7 @@ constexpr int kWaveCand = 512;                // list capacity per wave
 // chunk leaves the SIMDs too few waves to hide its serial phases (32 chunks a
 // row, k = 50, wave against workgroup kernel: 32 rows 21.1 against 17.7 us; 64
 // rows 22.5 / 24.6; 128 rows 26.9 / 35.5; 256 rows 38.3 / 59.4; 512 rows 57.3 /
-// 106.2).
+// 106.2; on rows of 128256 columns, before topk_row_kernel took that length).
 constexpr int kWaveMinWork = 2048;
 
 __device__ __forceinline__ int wave_sum_i(int v) {
@@ -985,6 +985,34 @@ bool row_kernel_ok(int T, int V) {
          (V >= 3 * kRowSlice / 2 || T <= kRowSmallMaxT);
 }
 
+// Whether the one-wave chunk kernels are ahead of the row kernel although that one
+// takes the row: many rows, a small k and a row that leaves much of the row
+// kernel's registers empty.  There the row kernel is bound by its slices (4, 8, 12,
+// 16 or 20 of 8192 columns, whether full or not) and the chunk path by the columns
+// and by k.  Both in ns a row (k 1 to 50, 1024 to 8192 rows; within 10 %); the
+// chunk path's two launches cost it 6 us more (us, chunk path / row kernel: 12288
+// columns, 8192 rows, k = 1 79 / 111, k = 50 125 / 132; 33000 columns, 4096 rows
+// 81 / 103, 134 / 123; 50000 columns, 4096 rows 110 / 121, 175 / 144; 32000
+// columns, 4096 rows 76 / 62, 126 / 74; 128256 columns, 2049 rows 119 / 118, 195 /
+// 133).
+constexpr int kWaveAheadMinT = 1000;
+constexpr int kWaveAheadMaxK = 50;
+bool wave_chunks_ahead(const TopkArgs& a) {
+  if (!a.vec || a.T < kWaveAheadMinT || a.k > kWaveAheadMaxK || a.C > kWaveChunk ||
+      static_cast<int64_t>(a.T) * a.S < kWaveMinWork)
+    return false;
+  struct Row {
+    double base, per_kcol, per_k;
+  };
+  constexpr Row kRow[] = {{11.3, 0.108, 0.050}, {15.9, 0.245, 0.107}, {15.9, 0.274, 0.128},
+                          {26.0, 0.243, 0.128}, {26.0, 0.260, 0.145}};
+  const double kcol = a.V * 1e-3, k = a.k;
+  const Row& r = kRow[(a.V + 7 + 4 * kRowSlice - 1) / (4 * kRowSlice) - 1];
+  const double row = r.base + r.per_kcol * kcol + r.per_k * k;
+  const double chunk = 3.4 + 0.395 * kcol + k * (0.083 + 0.0054 * kcol);
+  return a.T * (row - chunk) > 6000.0;
+}
+
 int launch_row(const TopkArgs& a, hipStream_t s) {
   const dim3 grid(a.T < (1 << 20) ? a.T : (1 << 20)), block(kRowThreads);
   const int nj = (a.V + 7 + kRowSlice - 1) / kRowSlice;
@@ -1065,9 +1093,11 @@ extern "C" int vaa_topk_logits(const uint16_t* logits, int num_tokens, int vocab
   const hipStream_t s = static_cast<hipStream_t>(stream);
   const int64_t n_work = static_cast<int64_t>(num_tokens) * a.S;
   const int grid1 = static_cast<int>(n_work < (1 << 20) ? n_work : (1 << 20));
-  // The row kernel leaves the workspace, which the call takes either way (its
-  // size depends only on the arguments), unused.
-  if (row_kernel_ok(num_tokens, vocab_size)) return launch_row(a, s);
+  // The row kernel leaves the workspace unused.  The call asks for it all the
+  // same: which calls are refused for want of one has never depended on the
+  // kernel that a row's length and the batch lead to, and a workspace sized for
+  // a vocabulary keeps serving shorter rows.
+  if (row_kernel_ok(num_tokens, vocab_size) && !wave_chunks_ahead(a)) return launch_row(a, s);
   if (a.vec && a.k <= kWaveK && a.C <= kWaveChunk && n_work >= kWaveMinWork) {
     const int64_t wgs = (n_work + kTkWaves - 1) / kTkWaves;
     hipLaunchKernelGGL(topk_chunk_wave_kernel, dim3(static_cast<int>(wgs < (1 << 20) ? wgs : (1 << 20))),

@@ -967,7 +967,9 @@ _topk_ws = _GrowOnlyScratch()
 
 
 def topk_workspace_size(num_tokens: int, vocab_size: int, k: int) -> int:
-    """Bytes of workspace vaa_topk_logits needs (0 when a row fits one workgroup)."""
+    """Bytes of workspace vaa_topk_logits asks for: the survivors of the chunks
+    that its plan cuts rows into, 0 for one chunk a row.  Rows that are selected
+    whole instead (most of 8192 to 163833 columns) leave it unused."""
     n = ctypes.c_size_t(0)
     _lib.call("vaa_topk_workspace_size", num_tokens, vocab_size, k, ctypes.byref(n))
     return int(n.value)
