@@ -39,7 +39,7 @@
 extern "C" {
 #endif
 
-#define VAA_ABI_VERSION 5
+#define VAA_ABI_VERSION 6
 
 enum {
   VAA_OK = 0,

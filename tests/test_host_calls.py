@@ -31,7 +31,8 @@ def test_declines_other_objects(name):
 _STUB = """
 #include <stddef.h>
 #include <unistd.h>
-int calls, delay_ms, inside;
+int calls, delay_ms, inside, version;
+int vaa_abi_version() { return version; }
 int vaa_topk_workspace_size(int t, int v, int k, size_t* n) { *n = 64; return 0; }
 """ + "".join(f"size_t {f}() {{ return 64; }}\n" for f in (
     "decode_workspace", "prefill_workspace", "step_workspace", "gate_workspace",
@@ -68,7 +69,9 @@ def stub_lib(tmp_path_factory):
     alias = [f"-Wl,--defsym={n}={f}" for f, ns in _STUB_NAMES.items() for n in ns]
     subprocess.run(["gcc", "-shared", "-fPIC", str(d / "stub.c"), "-o", str(so), *alias],
                    check=True)
-    return ctypes.CDLL(str(so))
+    lib = ctypes.CDLL(str(so))
+    ctypes.c_int.in_dll(lib, "version").value = _lib.ABI_VERSION
+    return lib
 
 
 @pytest.fixture
@@ -188,6 +191,29 @@ def test_product_is_left_to_torch_where_it_would_do_more(stub):
     with Sees():
         assert host.linear(*args) is False
     assert host.linear(*args) is True
+
+
+def test_a_library_of_another_version_is_refused(stub, stub_lib, monkeypatch):
+    """The host path calls entry points by the signatures it was built with: it
+    binds to no library of another version, and loading one says so."""
+    host, calls = stub
+    version = ctypes.c_int.in_dll(stub_lib, "version")
+    try:
+        for other in (_lib.ABI_VERSION - 1, _lib.ABI_VERSION + 1):
+            version.value = other
+            with pytest.raises(RuntimeError, match="version"):
+                host.bind(stub_lib._handle)
+    finally:
+        version.value = _lib.ABI_VERSION
+
+    def refuse(handle):
+        raise RuntimeError("ABI version mismatch")
+    monkeypatch.setattr(_lib, "_lib", None)
+    monkeypatch.setattr(_lib, "_host", None)
+    from vllm_apple_amd import _host
+    monkeypatch.setattr(_host, "bind", refuse)
+    with pytest.raises(_lib.NativeLibraryError, match="build_library"):
+        _lib.load()
 
 
 @pytest.mark.parametrize("name", NAMES)

@@ -628,6 +628,13 @@ PyObject* no_cache(const Args& a) {
 PyObject* bind(PyObject*, PyObject* arg) {
   void* h = PyLong_AsVoidPtr(arg);
   if (PyErr_Occurred()) return nullptr;
+  // The entry points are found by name and called by this build's signatures.
+  auto* version = reinterpret_cast<decltype(&::vaa_abi_version)>(dlsym(h, "vaa_abi_version"));
+  if (!version || version() != VAA_ABI_VERSION) {
+    PyErr_Format(PyExc_RuntimeError, "ABI version mismatch: the library has %d, _host needs %d",
+                 version ? version() : 0, VAA_ABI_VERSION);
+    return nullptr;
+  }
 #define VAA_BIND(f)                                                    \
   p_##f = reinterpret_cast<decltype(p_##f)>(dlsym(h, #f));             \
   if (!p_##f) {                                                        \

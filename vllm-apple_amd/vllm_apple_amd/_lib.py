@@ -35,7 +35,7 @@ VAA_PARTITION_BALANCED_SHARED = -2
 # Element types of caches, queries, new K/V and outputs (vaa_attn_params.dtype).
 VAA_DTYPE_F16 = 0
 VAA_DTYPE_BF16 = 1
-ABI_VERSION = 5
+ABI_VERSION = 6
 
 
 class NativeLibraryError(RuntimeError):
@@ -172,7 +172,11 @@ def load() -> ctypes.CDLL:
         except ImportError as e:
             raise NativeLibraryError(
                 f"the host extension is not built ({e}); run vllm_apple_amd.build_library()") from e
-        host_module.bind(lib._handle)
+        try:
+            host_module.bind(lib._handle)
+        except RuntimeError as e:
+            raise NativeLibraryError(f"the host extension does not fit {_LIB_PATH} ({e}); "
+                                     "run vllm_apple_amd.build_library()") from e
         _host = host_module
         _lib = lib
         return lib
