@@ -747,23 +747,15 @@ template <int D, typename T, int NW, bool kPad>
 __global__ void __launch_bounds__(NW* kWave) __attribute__((amdgpu_waves_per_eu(2)))
 paged_decode_balanced_kernel(DecodeArgs a) {
   extern __shared__ __align__(16) unsigned char smem[];
-  const int nc = gridDim.x, B = a.num_seqs;
+  const int c = blockIdx.x, y = blockIdx.y, nc = gridDim.x;
+  const int kvh = y / a.chunks, hc = y % a.chunks;
+  const int qh0 = kvh * a.G + hc * a.Gc, nh = min(a.Gc, a.G - hc * a.Gc);
+  const int B = a.num_seqs;
   int* starts = reinterpret_cast<int*>(smem + a.lds_main);
   tile_prefix(a, starts, starts + B + 1);
   const int total = starts[B];
   const int per = max((total + nc - 1) / nc, kBalMinUnits);
-  // The ranges in use (a small total leaves some workgroups without) are numbered
-  // without gaps over all kv heads, so that the surplus workgroups are the last of
-  // the grid.  With each head's surplus behind its own ranges the dispatcher dealt
-  // ranges to some CUs and surplus, which exits at once, to the others (32 kv
-  // heads, half of a grid in use: 105 contexts of 15 to 251 85 us, 50 without gaps).
-  const int used = max(1, (total + per - 1) / per);
-  const int id = blockIdx.y * nc + blockIdx.x;
-  const int y = id / used, c = id % used;
-  if (y >= static_cast<int>(gridDim.y)) return;
-  const int kvh = y / a.chunks, hc = y % a.chunks;
-  const int qh0 = kvh * a.G + hc * a.Gc, nh = min(a.Gc, a.G - hc * a.Gc);
-  if (id == 0) {
+  if (c == 0 && y == 0) {
     // Split geometry for the merge kernel.
     if (threadIdx.x == 0) a.ws_hdr[0] = per;
     for (int s = threadIdx.x; s <= B; s += blockDim.x) a.ws_hdr[1 + s] = starts[s];
