@@ -120,16 +120,17 @@ bool same_rows(const Tensor& a, const Tensor& b) {
   return a.sizes() == b.sizes() && a.strides() == b.strides();
 }
 
-// Calls an entry point without the interpreter lock, as ctypes does: a launch
+// Entry points are called without the interpreter lock, as by ctypes: a launch
 // into a full queue blocks until the GPU takes one, and other Python threads run
-// meanwhile.  The arguments are evaluated by the caller, with the lock; the
-// tensors live as long as the caller's argument list.
+// meanwhile.  The arguments are evaluated before, with the lock; the tensors live
+// as long as the caller's argument list.
+struct Unlocked {
+  PyThreadState* state = PyEval_SaveThread();
+  ~Unlocked() { PyEval_RestoreThread(state); }
+};
 template <typename... P, typename... A>
 int launch(int (*f)(P...), A... args) {
-  struct Unlocked {
-    PyThreadState* state = PyEval_SaveThread();
-    ~Unlocked() { PyEval_RestoreThread(state); }
-  } unlocked;
+  Unlocked unlocked;
   return f(args...);
 }
 
@@ -337,20 +338,19 @@ PyObject* linear(const Args& a) {
 
 // ------------------------------------------------------------ attention --
 
-// K/V rows key/value[:n] into the cache of p; 0 ok, else fall back.
-int write_rows(vaa_attn_params p, const Tensor& k, const Tensor& v, uint16_t* kc, uint16_t* vc,
-               const Tensor& slots, int64_t n, void* stream) {
-  const int it = slot_type(slots, n);
-  if (it < 0 || !rows3(k) || !same_rows(k, v) || k.size(0) < n || k.size(1) != p.num_kv_heads ||
-      k.size(2) != p.head_size)
-    return 1;
-  p.num_query_heads = p.num_kv_heads;
-  p.queries_per_kv = 1;
-  p.scale = 1.f;
-  p.new_kv_stride_token = k.stride(0);
-  p.new_kv_stride_head = k.stride(1);
-  return launch(p_vaa_kv_write_slots, &p, kc, vc, ptr(slots), it, p16(k), p16(v), n,
-                stream) != VAA_OK;
+// Fields and slot type of a write of K/V rows key/value[:n]; false: fall back.
+bool write_params(const Tensor& k, const Tensor& v, const Tensor& slots, int64_t n,
+                  vaa_attn_params* p, int* it) {
+  *it = slot_type(slots, n);
+  if (*it < 0 || !rows3(k) || !same_rows(k, v) || k.size(0) < n || k.size(1) != p->num_kv_heads ||
+      k.size(2) != p->head_size)
+    return false;
+  p->num_query_heads = p->num_kv_heads;
+  p->queries_per_kv = 1;
+  p->scale = 1.f;
+  p->new_kv_stride_token = k.stride(0);
+  p->new_kv_stride_head = k.stride(1);
+  return true;
 }
 
 // (key, value, key_cache, value_cache, slots, vllm, stream)
@@ -363,8 +363,10 @@ PyObject* kv_write(const Args& a) {
       !small(k->size(0)) || !cache4(*kc, *vc, a.b(5), &p))
     Py_RETURN_FALSE;
   p.dtype = dt;
-  if (write_rows(p, *k, *v, p16(*kc), p16(*vc), *sl, k->size(0), a.s(6))) Py_RETURN_FALSE;
-  Py_RETURN_TRUE;
+  int it;
+  if (!write_params(*k, *v, *sl, k->size(0), &p, &it)) Py_RETURN_FALSE;
+  return yes(launch(p_vaa_kv_write_slots, &p, p16(*kc), p16(*vc), ptr(*sl), it, p16(*k), p16(*v),
+                    k->size(0), a.s(6)));
 }
 
 // Fills the query, output, table and length fields of a decode over the first
@@ -462,10 +464,24 @@ PyObject* step_decode(const Args& a) {
   p.dtype = dt;
   const size_t need = p_vaa_paged_attention_decode_workspace_size(&p, nullptr);
   if (need && !room(ws, need, *q)) return PyLong_FromSize_t(need);
-  if (write && write_rows(p, *k, *v, kc, vc, *slots, n, a.s(15))) Py_RETURN_FALSE;
-  return yes(launch(p_vaa_paged_attention_decode, &p, p16(*q), kc, vc,
-                    static_cast<int32_t*>(ptr(*bt)), static_cast<int32_t*>(ptr(*sl)), p16(*o),
-                    nullptr, nullptr, need ? ptr(*ws) : nullptr, need ? ws->nbytes() : 0, a.s(15)));
+  vaa_attn_params wp = p;
+  int it = 0;
+  if (write && !write_params(*k, *v, *slots, n, &wp, &it)) Py_RETURN_FALSE;
+  const uint16_t *kp = write ? p16(*k) : nullptr, *vp = write ? p16(*v) : nullptr;
+  const void* slp = write ? ptr(*slots) : nullptr;
+  auto *btp = static_cast<int32_t*>(ptr(*bt)), *lp = static_cast<int32_t*>(ptr(*sl));
+  uint16_t *qp = p16(*q), *op = p16(*o);
+  void *wsp = need ? ptr(*ws) : nullptr, *stream = a.s(15);
+  const size_t ws_bytes = need ? ws->nbytes() : 0;
+  int st = VAA_OK;
+  {
+    Unlocked unlocked;
+    if (write) st = p_vaa_kv_write_slots(&wp, kc, vc, slp, it, kp, vp, n, stream);
+    if (st == VAA_OK)
+      st = p_vaa_paged_attention_decode(&p, qp, kc, vc, btp, lp, op, nullptr, nullptr, wsp,
+                                        ws_bytes, stream);
+  }
+  return yes(st);
 }
 
 // Fields of an unsplit prefill of tokens [0, n).
