@@ -8,7 +8,7 @@
 // elementwise.py:114-124); here the epilogue reads g and u from the
 // accumulators, so neither intermediate is written or read back.
 //
-// Tiling (one 4-wave workgroup per CU, all 160 KB of LDS):
+// Tiling (one 4-wave workgroup per CU, 128, 144 or 160 KB of LDS):
 //   workgroup = 64 NB tokens (NB = 2, 3 or 4, wide_blocks) x 128 output columns: a
 //               64 NB x 256 product of the token rows of x against 256 weight
 //               rows (128 gate, then the 128 up rows of the same columns);
@@ -30,6 +30,16 @@
 // M0).  The loads are inline asm, so the compiler does not track them (it
 // would otherwise wait for every one of them before any LDS read); the
 // kernel orders each LDS read behind its own counted vmcnt wait and barrier.
+// Weight tiles go through a ring of three 32 KB stages and activation tiles
+// through two of 8 NB KB: during step k the wave issues the activation
+// loads of step k + 1 and then the weight loads of step k + 2, spread over
+// the MFMAs of the step's first half, so the weight stream,
+// which comes from HBM, has two steps to land and the activations, which
+// come from L2 and the Infinity Cache, one.  The 16-byte chunks of each 128-byte LDS
+// row are XOR-swizzled by row & 7,
+// so the eight consecutive rows that an operand read spans per 128 bytes hit
+// distinct banks.  Token rows past num_tokens read the last token's row
+// (always in bounds) and their outputs are not stored.
 // What bounds a step is the LDS port beside the MFMAs: the operand reads and
 // the direct loads' writes take 1536 of its cycles against 2048 of MFMA at NB = 4
 // and 1344 against 1536 at NB = 3.
@@ -37,15 +47,6 @@
 // The same kernel runs 256 rows of a plain product (kPart: the down projection of
 // 129 to 1024 tokens) with the k-steps split so that one workgroup runs on every
 // CU; the fp32 partials are summed by wide_sum_kernel.
-// Weight tiles go through a ring of three 32 KB stages and activation tiles
-// through two, all of LDS: during step k the wave issues the activation
-// loads of step k + 1 and then the weight loads of step k + 2, one load
-// after every second MFMA of the step's first half, so the weight stream,
-// which comes from HBM, has two steps to land and the activations, which
-// come from L2 and the Infinity Cache, one.  The 16-byte chunks of each 128-byte LDS row are XOR-swizzled by row & 7,
-// so the eight consecutive rows that an operand read spans per 128 bytes hit
-// distinct banks.  Token rows past num_tokens read the last token's row
-// (always in bounds) and their outputs are not stored.
 //
 // Workgroup order: the 8 XCDs each take a contiguous range of (column tile,
 // token tile) pairs, token tile fastest, so all the token tiles that share a

@@ -6,15 +6,17 @@ up GEMMs into two [T, I] intermediates and a silu_mul pass over them; here
 the first half is one MFMA kernel with the SwiGLU epilogue
 (kernels.gate_up_silu), so only the activated [T, I] intermediate exists.  The
 down projection of up to 1024 tokens runs on kernels.linear where that pays
-(kernels.linear_pays); otherwise it is a plain library GEMM (torch.matmul on the
-step's stream).  Weights keep the reference's layouts: gate_proj / up_proj [I, H]
+(kernels.linear_pays) and nothing but the product is asked for; otherwise it is a
+plain library GEMM (torch.matmul on the step's stream).  Weights keep the reference's layouts: gate_proj / up_proj [I, H]
 or the fused gate_up_proj [2I, H] (gate rows first), down_proj [H, I].
 
 Above FUSED_MAX_TOKENS tokens encode takes the reference's order instead: a
-library GEMM into [T, 2I] and kernels.silu_mul over its halves.  On MI355X
-(hidden 5120, intermediate 32768) the fused kernel leads up to 1024 tokens
-(by 9 % at 16-64, 2-5 % at 256-1024) and hipBLASLt's GEMM leads at 2104 and
-4096 tokens (3 and 8 %).
+library GEMM into [T, 2I] and kernels.silu_mul over its halves.  On MI355X, bf16,
+weights beyond the caches, device us of that order / of the fused kernel: hidden
+5120, intermediate 32768, 64 tokens 122 / 108, 512 315 / 285, 1024 587 / 546, 2104
+1163 / 1188, 4096 2088 / 2173; 4096 x 14336, 64 tokens 56 / 41, 512 107 / 108, 1024
+199 / 212 (the one size on this side that loses), 2104 400 / 430; 2048 x 8192, 1024
+tokens 65 / 59, 2104 143 / 137, 4096 225 / 235.
 
 Only the gated SiLU form without biases is on this path; a standard MLP,
 GELU or biases raise NotImplementedError.

@@ -356,8 +356,15 @@ def choose_partition_size(seq_lens_host, num_kv_heads: int, num_cus: int,
     a CU's share and a cheaper start-up (for tiny batches a merge launch
     costs more than the split saves).  Balanced split: total/m plus one
     start-up per sequence piece a workgroup meets and the merge launch, which
-    it always has.  Equal lengths that already cover the CUs stay unsplit;
-    the balanced split must win by 3 % to be chosen.  Memoised per length
+    it always has.  (The kernel's shares count a start-up as 8 tiles instead, so
+    that no workgroup pays more of them than another; the estimate was fitted to
+    shares of tiles alone.)  Equal lengths that already cover the CUs stay unsplit;
+    the balanced split must win by 3 % to be chosen.  Over 70 batches of 4 to 64
+    sequences of 50 to 6000 tokens, six head shapes, the choice was 3.5 % behind the
+    best of its modes in the mean: level or within 3 % for 52 of them, behind the
+    balanced split by up to 22 % for equal lengths (15 of 2477, 32/8 heads, us: 43.0
+    in pieces of 2560, 35.3 balanced) and behind another fixed size by up to 39 %
+    (4 of 3061 to 4082: 23.2 at 384, 16.7 at 512).  Memoised per length
     tuple (the same step is decoded by every layer).
     """
     key = (_int_tuple(seq_lens_host), int(num_kv_heads), int(num_cus), merge_tokens, wg_tokens)
