@@ -98,6 +98,31 @@ def test_linear_strided_rows_and_refusals(gpu):
         kernels.linear(x, w[:200], out[:, :200])
 
 
+def test_split_products_on_a_stream_given_by_its_handle(gpu):
+    """stream may be any object with the raw handle, as for the other wrappers,
+    where the product needs scratch of that stream too."""
+    from types import SimpleNamespace
+
+    from vllm_apple_amd import kernels
+
+    side = torch.cuda.Stream()
+    by_handle = SimpleNamespace(cuda_stream=side.cuda_stream)
+    x = (torch.arange(7 * 2048, device="cuda") % 13).view(7, 2048).half()
+    w = (torch.arange(512 * 2048, device="cuda") % 7 / 2048).view(512, 2048).half()
+    outs = []
+    side.wait_stream(torch.cuda.current_stream())
+    for s in (side, by_handle):
+        act = torch.zeros(7, 256, dtype=x.dtype, device="cuda")
+        lin = torch.zeros(7, 512, dtype=x.dtype, device="cuda")
+        torch.cuda.synchronize()
+        kernels.gate_up_silu(x, w, out=act, stream=s)
+        kernels.linear(x, w, lin, stream=s)
+        torch.cuda.synchronize()
+        outs.append((act, lin))
+    assert torch.equal(outs[0][0], outs[1][0]) and torch.equal(outs[0][1], outs[1][1])
+    assert bool(outs[0][0].any()) and bool(outs[0][1].any())
+
+
 @pytest.mark.parametrize("which", ["down_proj", "out"])
 def test_mlp_refuses_gradients_as_the_library_product_does(gpu, which):
     """encode writes into a given buffer, which autograd cannot follow: a down

@@ -1146,6 +1146,8 @@ def _stream_scratch(nbytes: int, device: torch.device, stream) -> torch.Tensor |
         return None
     if stream is None:
         return torch.empty(nbytes, dtype=torch.uint8, device=device)
+    if not isinstance(stream, torch.cuda.Stream):  # anything with a raw handle
+        stream = torch.cuda.ExternalStream(int(stream.cuda_stream), device=device)
     with torch.cuda.stream(stream):
         return torch.empty(nbytes, dtype=torch.uint8, device=device)
 
