@@ -9,10 +9,10 @@
 // Rows of 8192 to 163833 columns (the vocabularies served in practice) are
 // selected whole by one 16-wave workgroup each, in its registers
 // (topk_row_kernel).  Other rows, and large batches of these where that is faster
-// (row_kernel_ok, wave_chunks_ahead), are cut into S chunks of at most kChunkMax columns, one workgroup per chunk,
-// so a small batch still fills the chip.  A workgroup loads
-// its whole chunk into registers with every load in flight at once (one HBM
-// round trip) and selects on order-preserving 16-bit keys: a lower bound L
+// (row_kernel_ok, wave_chunks_ahead), are cut into S chunks of at most kChunkMax
+// columns, one workgroup per chunk, so a small batch still fills the chip.  A
+// workgroup loads its whole chunk into registers with every load in flight at once
+// (one HBM round trip) and selects on order-preserving 16-bit keys: a lower bound L
 // from k thread-group maxima (the top k are all >= L; on logits only ~1-5% of
 // a chunk is), the items >= L listed in LDS, and each listed item's rank
 // among them as its output position.  Flat or heavily tied rows, where too
